@@ -20,16 +20,20 @@ PKG = os.path.dirname(HERE)
 ROOT = os.path.dirname(PKG)
 LIB = os.path.join(PKG, "libqmcmi355x.so")
 # (source, object tag, extra defines): kernel families are compiled once per radial type
-_FAMILIES = ["qmc_wf_f32.hip", "qmc_wf_f64.hip", "qmc_sweep_f32.hip", "qmc_sweep_f64.hip", "qmc_grad.hip",
+_FAMILIES = ["qmc_wf_f32.hip", "qmc_wf_f64.hip", "qmc_sweep_f32.hip", "qmc_sweep_f64.hip",
              "qmc_batch_sweep_f32.hip", "qmc_batch_sweep_f64.hip", "qmc_batch_wf_f32.hip", "qmc_batch_wf_f64.hip",
-             "qmc_exc.hip", "qmc_exc_hmc.hip",
+             "qmc_exc_hmc.hip",
 ]
+# families whose kernels are spread over several units (-DQMC_PART)
+_PARTS = [("qmc_exc.hip", p) for p in range(4)] + [("qmc_grad.hip", p) for p in range(4)]
 # HMC / drift kernels: single-configuration (MC=1) and multi-configuration (MC=8) instances
 _HMC = [("qmc_hmc_f32.hip", mc) for mc in (1, 8)] + [("qmc_hmc_f64.hip", mc) for mc in (1, 8)]
 UNITS = [("qmc_abi.hip", "qmc_abi", []), ("qmc_api.hip", "qmc_api", []), ("qmc_noalloc.hip", "qmc_noalloc", [])] + [
     (f, f.replace(".hip", "_r%d" % r), ["-DQMC_RAD=%d" % r]) for f in _FAMILIES for r in (0, 1)
 ] + [(f, f.replace(".hip", "_mc%d_r%d" % (mc, r)), ["-DQMC_RAD=%d" % r, "-DQMC_HMC_MC=%d" % mc])
-     for f, mc in _HMC for r in (0, 1)]
+     for f, mc in _HMC for r in (0, 1)] + [
+    (f, f.replace(".hip", "_p%d_r%d" % (p, r)), ["-DQMC_RAD=%d" % r, "-DQMC_PART=%d" % p])
+    for f, p in _PARTS for r in (0, 1)]
 SOURCES = [u[0] for u in UNITS]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -116,7 +120,8 @@ def build(verbose: bool = False, resource_usage: bool = False, jobs: int = 0, in
     if incremental:
         units = [u for u in units if _stale(u)]
     # the largest units first, so the parallel build ends sooner
-    units = sorted(units, key=lambda u: 0 if u[0].startswith(os.path.join(_obj_dir(), "spec")) else 1)
+    units = sorted(units, key=lambda u: 0 if u[0] in ("qmc_exc.hip", "qmc_grad.hip") else
+                   1 if u[0].startswith(os.path.join(_obj_dir(), "spec")) else 2)
     jobs = jobs or max(1, min(len(units), os.cpu_count() or 4, 16))
     with ThreadPoolExecutor(jobs) as ex:
         results = list(ex.map(lambda u: compile_one(u, extra), units))

@@ -220,7 +220,7 @@ int refuse_excitations(const QmcPlan* plan) {
 int launch_hmc(const HArgs& a, int precision, hipStream_t s) {
     const bool f64 = precision == QMC_PREC_FP64, sto = a.t.radial == QMC_RADIAL_STO;
     if (a.t.exc_mode) return QMC_BY_RAD(launch_hmc_exc, a.t.radial, a, precision, s);
-    if (a.t.nconf_max <= 1) {
+    if (a.t.identity_conf) {
         if (f64) return sto ? launch_hmc_f64<QMC_RADIAL_STO, 1>(a, s) : launch_hmc_f64<QMC_RADIAL_GTO_PURE, 1>(a, s);
         return sto ? launch_hmc_f32<QMC_RADIAL_STO, 1>(a, s) : launch_hmc_f32<QMC_RADIAL_GTO_PURE, 1>(a, s);
     }
@@ -356,7 +356,7 @@ int qmc_plan_create(const QmcSystemDesc* d, QmcPlan** out) {
             t.exc_dn = (decltype(t.exc_dn))p->upload(exc_dn.data(), exc_dn.size());
         }
         // generated kernels have no excitation path
-        p->spec = exc ? nullptr : find_spec(layout_signature(d), nm_bucket_fine(t), (64 / t.nelec) * t.nelec);
+        p->spec = exc ? nullptr : find_spec(layout_signature(d), nm_bucket_fine(t), (64 / t.nelec) * t.nelec, !ident);
     } catch (const std::exception& ex) {
         delete p;
         return fail(QMC_ERR_HIP, ex.what());
@@ -734,13 +734,14 @@ int take_slot(QmcBatch* b, int& slot) {
 struct Group {
     int rad, bucket;
     bool exc;  // excitation plans: their own kernels, one wavefront per block
+    bool multi;  // several configurations
     const SpecEntry* spec;
     std::vector<int> idx;
     size_t lds;  // exc: the largest exc_lds_bytes of the group's jobs
 };
 
-// Groups the jobs by (radial type, register bucket, excitation path, generated
-// layout), costliest systems first inside a group.  Returns an error for jobs
+// Groups the jobs by (radial type, register bucket, configuration kind, excitation
+// path, generated layout), costliest systems first inside a group.  Returns an error for jobs
 // without a bucket.
 template <typename JobT>
 int group_jobs(const JobT* jobs, int njobs, std::vector<Group>& groups) {
@@ -748,13 +749,13 @@ int group_jobs(const JobT* jobs, int njobs, std::vector<Group>& groups) {
         const Tables& t = jobs[j].plan->t;
         const int bk = nm_bucket_fine(t);
         if (bk < 0) return fail(QMC_ERR_UNSUPPORTED, kNoBucket);
-        const bool exc = t.exc_mode != 0;
+        const bool exc = t.exc_mode != 0, multi = !t.identity_conf;
         const SpecEntry* sp = (!exc && jobs[j].plan->use_spec) ? jobs[j].plan->spec : nullptr;
         Group* g = nullptr;
         for (auto& x : groups)
-            if (x.rad == t.radial && x.bucket == bk && x.exc == exc && x.spec == sp) g = &x;
+            if (x.rad == t.radial && x.bucket == bk && x.exc == exc && x.multi == multi && x.spec == sp) g = &x;
         if (!g) {
-            groups.push_back(Group{t.radial, bk, exc, sp, {}, 0});
+            groups.push_back(Group{t.radial, bk, exc, multi, sp, {}, 0});
             g = &groups.back();
         }
         g->idx.push_back(j);
@@ -823,7 +824,7 @@ int qmc_metropolis_sweep_batch(QmcBatch* b, int32_t precision, const QmcSweepJob
     SJob* dev = (SJob*)(b->dev + slot * b->slot_bytes);
     struct Launch {
         int rad, bucket, first, n, nwaves;
-        bool exc;
+        bool exc, multi;
         size_t lds;
         const SpecEntry* spec;
     };
@@ -845,7 +846,7 @@ int qmc_metropolis_sweep_batch(QmcBatch* b, int32_t precision, const QmcSweepJob
             waves += (x.nw + G - 1) / G;
         }
         if (waves > (int64_t)1 << 30) return fail(QMC_ERR_ARG, "batch too large");
-        launches.push_back(Launch{g.rad, g.bucket, first, k - first, (int)waves, g.exc, g.lds, g.spec});
+        launches.push_back(Launch{g.rad, g.bucket, first, k - first, (int)waves, g.exc, g.multi, g.lds, g.spec});
     }
     hipStream_t s = (hipStream_t)stream;
     QMC_HIP(hipMemcpyAsync(dev, host, (size_t)k * sizeof(SJob), hipMemcpyHostToDevice, s));
@@ -857,8 +858,8 @@ int qmc_metropolis_sweep_batch(QmcBatch* b, int32_t precision, const QmcSweepJob
         }
         if (L.spec && L.spec->sweep_batch(dev + L.first, L.n, L.nwaves, precision, s) == 0) continue;
         const int r = precision == QMC_PREC_FP64
-                          ? QMC_BY_RAD(launch_sweep_batch_f64, L.rad, dev + L.first, L.n, L.nwaves, L.bucket, s)
-                          : QMC_BY_RAD(launch_sweep_batch_f32, L.rad, dev + L.first, L.n, L.nwaves, L.bucket, s);
+                          ? QMC_BY_RAD(launch_sweep_batch_f64, L.rad, dev + L.first, L.n, L.nwaves, L.bucket, L.multi, s)
+                          : QMC_BY_RAD(launch_sweep_batch_f32, L.rad, dev + L.first, L.n, L.nwaves, L.bucket, L.multi, s);
         if (r) return fail(QMC_ERR_UNSUPPORTED, kNoBucket);
     }
     QMC_HIP(hipGetLastError());
@@ -892,7 +893,7 @@ int qmc_wf_eval_batch(QmcBatch* b, int32_t precision, int32_t mode, const QmcEva
     WJob* dev = (WJob*)(b->dev + slot * b->slot_bytes);
     struct Launch {
         int rad, bucket, first, n, nwaves;
-        bool exc;
+        bool exc, multi;
         size_t lds;
         const SpecEntry* spec;
     };
@@ -914,7 +915,7 @@ int qmc_wf_eval_batch(QmcBatch* b, int32_t precision, int32_t mode, const QmcEva
             waves += (x.nw + G - 1) / G;
         }
         if (waves > (int64_t)1 << 30) return fail(QMC_ERR_ARG, "batch too large");
-        launches.push_back(Launch{g.rad, g.bucket, first, k - first, (int)waves, g.exc, g.lds, g.spec});
+        launches.push_back(Launch{g.rad, g.bucket, first, k - first, (int)waves, g.exc, g.multi, g.lds, g.spec});
     }
     hipStream_t s = (hipStream_t)stream;
     QMC_HIP(hipMemcpyAsync(dev, host, (size_t)k * sizeof(WJob), hipMemcpyHostToDevice, s));
@@ -928,8 +929,8 @@ int qmc_wf_eval_batch(QmcBatch* b, int32_t precision, int32_t mode, const QmcEva
         if (L.spec && L.spec->wf_batch(dev + L.first, L.n, L.nwaves, precision, mode, s) == 0) continue;
         const int r =
             precision == QMC_PREC_FP64
-                ? QMC_BY_RAD(launch_wf_batch_f64, L.rad, dev + L.first, L.n, L.nwaves, L.bucket, mode, s)
-                : QMC_BY_RAD(launch_wf_batch_f32, L.rad, dev + L.first, L.n, L.nwaves, L.bucket, mode, s);
+                ? QMC_BY_RAD(launch_wf_batch_f64, L.rad, dev + L.first, L.n, L.nwaves, L.bucket, L.multi, mode, s)
+                : QMC_BY_RAD(launch_wf_batch_f32, L.rad, dev + L.first, L.n, L.nwaves, L.bucket, L.multi, mode, s);
         if (r) return fail(QMC_ERR_UNSUPPORTED, kNoBucket);
     }
     QMC_HIP(hipGetLastError());

@@ -187,8 +187,9 @@ struct GRedArgs {
 // Adds g * d log|psi| / d theta of the wavefront's walkers to its slot
 // (grad_kernel's quantities: Gamma rows, D_n / S, the Pade weight
 // derivatives and the exponent terms, contracted instead of written).
-// EXC: plans with exc_mode (Gamma from exc_gamma; xlds its LDS rows).
-template <int NM, int RAD, bool EXC = false>
+// MULTI: several configurations (else the ground-state determinant, in one
+// inversion); EXC: plans with exc_mode (Gamma from exc_gamma; xlds its LDS rows).
+template <int NM, int RAD, bool MULTI, bool EXC = false>
 __device__ __forceinline__ void logpsi_adjoint_reduce(const GRedArgs& a, const WalkerLane& L, double* slot,
                                                       double* stage, double* xlds = nullptr) {
     const Tables& t = a.t;
@@ -228,6 +229,11 @@ __device__ __forceinline__ void logpsi_adjoint_reduce(const GRedArgs& a, const W
             const int o = a.r.off_ci + n;
             if (red_owner(o) == L.lane) slot[o] += sum;
         }
+    } else if constexpr (!MULTI) {
+        const double sum = wave_sum((v && L.e == 0) ? gw / ldc(a.p.ci, 0) : 0.0);  // d log|psi| / d c = 1 / c
+        if (red_owner(a.r.off_ci) == L.lane) slot[a.r.off_ci] += sum;
+        double lg, sg;
+        conf_inverse<NM>(t, L, 0, mo, stage_conf_rows<NM>(t, L, mo), lg, sg, gam);
     } else {
         double ld[QMC_MAXCONF], sd[QMC_MAXCONF], td[QMC_MAXCONF], om[QMC_MAXCONF];
 #pragma unroll
@@ -239,7 +245,8 @@ __device__ __forceinline__ void logpsi_adjoint_reduce(const GRedArgs& a, const W
         }
 #pragma unroll
         for (int m = 0; m < NM; ++m) gam[m] = 0.0;
-        conf_dets<NM, false>(t, L, mo, ld, sd, om, gam);
+        const int own_ex = stage_conf_rows<NM>(t, L, mo);
+        conf_dets<NM, false>(t, L, mo, own_ex, ld, sd, om, gam);
         CiTerms ct;
         ci_terms(t, a.p, L, ld, sd, td, ct);
         for (int n = 0; n < t.nci; ++n) {
@@ -254,7 +261,7 @@ __device__ __forceinline__ void logpsi_adjoint_reduce(const GRedArgs& a, const W
             const int o = a.r.off_ci + n;
             if (red_owner(o) == L.lane) slot[o] += sum;
         }
-        conf_dets<NM, true>(t, L, mo, ld, sd, om, gam);
+        conf_dets<NM, true>(t, L, mo, own_ex, ld, sd, om, gam);
     }
     // W: stage the recomputed AO row, contract with g * Gamma
     double gG[NM], unused[NM];
@@ -343,7 +350,7 @@ __device__ __forceinline__ double* red_stage_rows() {
     return st + (threadIdx.x >> 6) * NS * 64 * (kRedCols + 1);
 }
 
-template <int NM, int RAD>
+template <int NM, int RAD, bool MULTI>
 __global__ __launch_bounds__(kBlock) void grad_reduce_kernel(GRedArgs a) {
     const int slot_id = global_wave();
     if (slot_id >= a.r.nslot) return;
@@ -353,7 +360,7 @@ __global__ __launch_bounds__(kBlock) void grad_reduce_kernel(GRedArgs a) {
     double* stage = red_stage_rows<1>();
     for (int64_t vw = slot_id; vw < a.r.nwaves; vw += a.r.nslot) {
         const WalkerLane L = lane_layout_w(a.t, a.nw, (int)vw);
-        logpsi_adjoint_reduce<NM, RAD>(a, L, slot, stage);
+        logpsi_adjoint_reduce<NM, RAD, MULTI>(a, L, slot, stage);
     }
 }
 
@@ -369,7 +376,7 @@ __global__ __launch_bounds__(64) void grad_reduce_kernel_exc(GRedArgs a) {
     __shared__ double stage[64 * (kRedCols + 1)];
     for (int64_t vw = slot_id; vw < a.r.nwaves; vw += a.r.nslot) {
         const WalkerLane L = lane_layout_w(a.t, a.nw, (int)vw);
-        logpsi_adjoint_reduce<NM, RAD, true>(a, L, slot, stage, (double*)qmc_dyn_lds);
+        logpsi_adjoint_reduce<NM, RAD, true, true>(a, L, slot, stage, (double*)qmc_dyn_lds);
     }
 }
 
@@ -383,10 +390,17 @@ struct ERedArgs {
     RedSlots r;
 };
 
+// Kinetic rows [64][NM] of this wavefront (larger buckets).
+template <int NM>
+__device__ __forceinline__ double* wave_brow() {
+    __shared__ double rows[kBlockWaves * 64 * NM];
+    return rows + (threadIdx.x >> 6) * 64 * NM;
+}
+
 // Adds g * d E_L / d theta of the wavefront's walkers to its slot
 // (eloc_grad_kernel's quantities, contracted instead of written).
-// EXC: plans with exc_mode (exc_eloc_gamma's rows in xlds).
-template <int NM, int RAD, bool EXC = false>
+// MULTI, EXC as in logpsi_adjoint_reduce (exc_eloc_gamma's rows in xlds).
+template <int NM, int RAD, bool MULTI, bool EXC = false>
 __device__ __forceinline__ void eloc_adjoint_reduce(const ERedArgs& a, const WalkerLane& L, double* slot,
                                                     double* stage, double* xlds = nullptr) {
     const Tables& t = a.t;
@@ -428,6 +442,19 @@ __device__ __forceinline__ void eloc_adjoint_reduce(const ERedArgs& a, const Wal
     double GA[NM], GB[NM];
     double s[3] = {0.0, 0.0, 0.0};
     double T;
+    // the kinetic rows (and, for small matrices, the lanes' inverse columns) in
+    // LDS: in the stage rows, free until the W sums, or the larger buckets' own
+    double *brow = stage, *ycol = stage + 64 * NM;
+    int own_ex = 0;
+    if constexpr (!EXC) {
+        if constexpr (!use_minors<NM>()) brow = wave_brow<NM>();
+        static_assert(!use_minors<NM>() || NM <= kRedCols + 1, "both fit the stage rows");
+        wave_lds_sync();  // the previous walkers' loads come first
+#pragma unroll
+        for (int k = 0; k < NM; ++k) brow[L.lane * NM + k] = bk[k];
+        own_ex = stage_conf_rows<NM>(t, L, mo);
+        wave_lds_sync();
+    }
     if constexpr (EXC) {
         T = exc_eloc_gamma<NM>(t, a.p, L, mo, bk, xlds, GA, GB, [&](int nn, double val) {
             const double sum = wave_sum((v && L.e == 0) ? gw * val : 0.0);
@@ -442,6 +469,23 @@ __device__ __forceinline__ void eloc_adjoint_reduce(const ERedArgs& a, const Wal
                 s[2] += GB[m] * gz[m];
             }
         }
+    } else if constexpr (!MULTI) {
+        double lg, sg, inv[NM], zz[NM];
+        conf_inverse<NM>(t, L, 0, mo, own_ex, lg, sg, inv);
+        inverse_b_inverse<NM>(t, L, inv, brow, ycol, [](int k) { return k; }, zz);
+        double tp = 0.0;
+#pragma unroll
+        for (int k = 0; k < NM; ++k) {
+            const bool in = k < L.n_sig;
+            tp += in ? bk[k] * inv[k] : 0.0;
+            GA[k] = in ? -zz[k] : 0.0;
+            GB[k] = in ? inv[k] : 0.0;
+            s[0] += in ? inv[k] * gx[k] : 0.0;
+            s[1] += in ? inv[k] * gy[k] : 0.0;
+            s[2] += in ? inv[k] * gz[k] : 0.0;
+        }
+        T = seg_sum(tp, L.wbase, t.nelec, t.nelec);
+        // d E_L / d c of a single term is zero: its slot stays as it is
     } else {
         double ld[QMC_MAXCONF], sd[QMC_MAXCONF], td[QMC_MAXCONF];
 #pragma unroll
@@ -452,12 +496,12 @@ __device__ __forceinline__ void eloc_adjoint_reduce(const ERedArgs& a, const Wal
         }
 #pragma unroll 1
         for (int c = 0; c < t.nconf_max; ++c) {
-            double aa[NM], bb[NM];
-            gather_conf<NM>(t, L, c, mo, aa);
+            double inv[NM], bb[NM];
+            double lg, sg, tp = 0.0;
             gather_conf<NM>(t, L, c, bk, bb);
-            double lg, sg, tp;
-            int col;
-            lane_gj<NM>(L, t.nsig_max, aa, bb, lg, sg, tp, col);
+            conf_inverse<NM>(t, L, c, mo, own_ex, lg, sg, inv);
+#pragma unroll
+            for (int k = 0; k < NM; ++k) tp += k < L.n_sig ? bb[k] * inv[k] : 0.0;
             const double tr = seg_sum(tp, L.gbase, L.n_sig, t.nsig_max);
 #pragma unroll
             for (int c2 = 0; c2 < QMC_MAXCONF; ++c2)
@@ -499,18 +543,11 @@ __device__ __forceinline__ void eloc_adjoint_reduce(const ERedArgs& a, const Wal
         for (int m = 0; m < NM; ++m) GA[m] = GB[m] = 0.0;
 #pragma unroll 1
         for (int c = 0; c < t.nconf_max; ++c) {
-            double aa[NM], xb[NM], ib[NM];
-            gather_conf<NM>(t, L, c, mo, aa);
-            gather_conf<NM>(t, L, c, bk, xb);
-            double lg, sg, tp;
-            int col, col2;
-            lane_gj<NM>(L, t.nsig_max, aa, xb, lg, sg, tp, col);
-            gather_conf<NM>(t, L, c, mo, aa);
-#pragma unroll
-            for (int j = 0; j < NM; ++j) ib[j] = (j == L.myrow) ? 1.0 : 0.0;
-            lane_gj<NM>(L, t.nsig_max, aa, ib, lg, sg, tp, col2);
-            double inv[NM], zz[NM];
-            inverse_columns<NM>(L, t.nsig_max, col, xb, ib, inv, zz);
+            double lg, sg, inv[NM], zz[NM];
+            conf_inverse<NM>(t, L, c, mo, own_ex, lg, sg, inv);
+            const int nc = L.spin == 0 ? t.nconf_up : t.nconf_dn, cc = c < nc ? c : nc - 1;
+            const QMC_CONST int* cf = L.spin == 0 ? t.conf_up + cc * t.nup : t.conf_dn + cc * t.ndown;
+            inverse_b_inverse<NM>(t, L, inv, brow, ycol, [&](int k) { return t.identity_conf ? k : (int)cf[k]; }, zz);
             double rc = 0.0, oc = 0.0;
 #pragma unroll
             for (int c2 = 0; c2 < QMC_MAXCONF; ++c2)
@@ -581,7 +618,7 @@ __device__ __forceinline__ void eloc_adjoint_reduce(const ERedArgs& a, const Wal
     }
 }
 
-template <int NM, int RAD>
+template <int NM, int RAD, bool MULTI>
 __global__ __launch_bounds__(kBlock) void eloc_grad_reduce_kernel(ERedArgs a) {
     const int slot_id = global_wave();
     if (slot_id >= a.r.nslot) return;
@@ -591,7 +628,7 @@ __global__ __launch_bounds__(kBlock) void eloc_grad_reduce_kernel(ERedArgs a) {
     double* stage = red_stage_rows<2>();
     for (int64_t vw = slot_id; vw < a.r.nwaves; vw += a.r.nslot) {
         const WalkerLane L = lane_layout_w(a.t, a.nw, (int)vw);
-        eloc_adjoint_reduce<NM, RAD>(a, L, slot, stage);
+        eloc_adjoint_reduce<NM, RAD, MULTI>(a, L, slot, stage);
     }
 }
 
@@ -607,7 +644,7 @@ __global__ __launch_bounds__(64) void eloc_grad_reduce_kernel_exc(ERedArgs a) {
     __shared__ double stage[2 * 64 * (kRedCols + 1)];
     for (int64_t vw = slot_id; vw < a.r.nwaves; vw += a.r.nslot) {
         const WalkerLane L = lane_layout_w(a.t, a.nw, (int)vw);
-        eloc_adjoint_reduce<NM, RAD, true>(a, L, slot, stage, (double*)qmc_dyn_lds);
+        eloc_adjoint_reduce<NM, RAD, true, true>(a, L, slot, stage, (double*)qmc_dyn_lds);
     }
 }
 

@@ -7,9 +7,15 @@
 #ifndef QMC_RAD
 #error "compile with -DQMC_RAD=0 (gto_pure) or -DQMC_RAD=1 (sto)"
 #endif
+// One unit per kernel family, so that they compile in parallel: -DQMC_PART=0
+// (psi / local energy), 1 (sweeps), 2 (log|psi| adjoint), 3 (E_L adjoint)
+#ifndef QMC_PART
+#error "compile with -DQMC_PART=0..3"
+#endif
 
 namespace qmc {
 
+#if QMC_PART == 0
 template <int NM, int RAD>
 static void go_wf(const KArgs& a, int prec, int mode, hipStream_t s) {
     const size_t lds = exc_lds_bytes(a.t, NM);
@@ -19,22 +25,9 @@ static void go_wf(const KArgs& a, int prec, int mode, hipStream_t s) {
             hipLaunchKernelGGL((wf_kernel_exc<double, NM, RAD, true>), g, dim3(64), lds, s, a);
         else
             hipLaunchKernelGGL((wf_kernel_exc<double, NM, RAD, false>), g, dim3(64), lds, s, a);
-    } else {
-        if (mode == QMC_EVAL_ELOC)
-            hipLaunchKernelGGL((wf_kernel_exc<float, NM, RAD, true>), g, dim3(64), lds, s, a);
-        else
-            hipLaunchKernelGGL((wf_kernel_exc<float, NM, RAD, false>), g, dim3(64), lds, s, a);
+    } else {  // psi only: local energies are FP64
+        hipLaunchKernelGGL((wf_kernel_exc<float, NM, RAD, false>), g, dim3(64), lds, s, a);
     }
-}
-
-template <int NM, int RAD>
-static void go_sweep(const SArgs& a, int prec, hipStream_t s) {
-    const size_t lds = exc_lds_bytes(a.t, NM);
-    const dim3 g = exc_grid(a.t, a.nw);
-    if (prec == QMC_PREC_FP64)
-        hipLaunchKernelGGL((sweep_kernel_exc<double, NM, RAD>), g, dim3(64), lds, s, a);
-    else
-        hipLaunchKernelGGL((sweep_kernel_exc<float, NM, RAD>), g, dim3(64), lds, s, a);
 }
 
 template <>
@@ -48,6 +41,45 @@ int launch_wf_exc<QMC_RAD>(const KArgs& a, int prec, int mode, hipStream_t s) {
 #undef QMC_CASE
         default: return -1;
     }
+}
+
+template <int NM, int RAD>
+static void go_wf_batch(const WJob* jobs, int njobs, int nwaves, size_t lds, int prec, int mode, hipStream_t s) {
+    const dim3 g((unsigned)nwaves);
+    if (prec == QMC_PREC_FP64) {
+        if (mode == QMC_EVAL_ELOC)
+            hipLaunchKernelGGL((wf_batch_kernel_exc<double, NM, RAD, true>), g, dim3(64), lds, s, jobs, njobs, nwaves);
+        else
+            hipLaunchKernelGGL((wf_batch_kernel_exc<double, NM, RAD, false>), g, dim3(64), lds, s, jobs, njobs,
+                               nwaves);
+    } else {
+        hipLaunchKernelGGL((wf_batch_kernel_exc<float, NM, RAD, false>), g, dim3(64), lds, s, jobs, njobs, nwaves);
+    }
+}
+
+template <>
+int launch_wf_batch_exc<QMC_RAD>(const WJob* jobs, int njobs, int nwaves, int bucket, size_t lds, int prec, int mode,
+                                 hipStream_t s) {
+    switch (bucket) {
+#define QMC_CASE(K)                                                       \
+    case K:                                                               \
+        go_wf_batch<K, QMC_RAD>(jobs, njobs, nwaves, lds, prec, mode, s); \
+        return 0;
+        QMC_EXC_BUCKETS(QMC_CASE)
+#undef QMC_CASE
+        default: return -1;
+    }
+}
+
+#elif QMC_PART == 1
+template <int NM, int RAD>
+static void go_sweep(const SArgs& a, int prec, hipStream_t s) {
+    const size_t lds = exc_lds_bytes(a.t, NM);
+    const dim3 g = exc_grid(a.t, a.nw);
+    if (prec == QMC_PREC_FP64)
+        hipLaunchKernelGGL((sweep_kernel_exc<double, NM, RAD>), g, dim3(64), lds, s, a);
+    else
+        hipLaunchKernelGGL((sweep_kernel_exc<float, NM, RAD>), g, dim3(64), lds, s, a);
 }
 
 template <>
@@ -86,37 +118,7 @@ int launch_sweep_batch_exc<QMC_RAD>(const SJob* jobs, int njobs, int nwaves, int
     }
 }
 
-template <int NM, int RAD>
-static void go_wf_batch(const WJob* jobs, int njobs, int nwaves, size_t lds, int prec, int mode, hipStream_t s) {
-    const dim3 g((unsigned)nwaves);
-    if (prec == QMC_PREC_FP64) {
-        if (mode == QMC_EVAL_ELOC)
-            hipLaunchKernelGGL((wf_batch_kernel_exc<double, NM, RAD, true>), g, dim3(64), lds, s, jobs, njobs, nwaves);
-        else
-            hipLaunchKernelGGL((wf_batch_kernel_exc<double, NM, RAD, false>), g, dim3(64), lds, s, jobs, njobs,
-                               nwaves);
-    } else {
-        if (mode == QMC_EVAL_ELOC)
-            hipLaunchKernelGGL((wf_batch_kernel_exc<float, NM, RAD, true>), g, dim3(64), lds, s, jobs, njobs, nwaves);
-        else
-            hipLaunchKernelGGL((wf_batch_kernel_exc<float, NM, RAD, false>), g, dim3(64), lds, s, jobs, njobs, nwaves);
-    }
-}
-
-template <>
-int launch_wf_batch_exc<QMC_RAD>(const WJob* jobs, int njobs, int nwaves, int bucket, size_t lds, int prec, int mode,
-                                 hipStream_t s) {
-    switch (bucket) {
-#define QMC_CASE(K)                                                       \
-    case K:                                                               \
-        go_wf_batch<K, QMC_RAD>(jobs, njobs, nwaves, lds, prec, mode, s); \
-        return 0;
-        QMC_EXC_BUCKETS(QMC_CASE)
-#undef QMC_CASE
-        default: return -1;
-    }
-}
-
+#elif QMC_PART == 2
 template <int NM, int RAD>
 static void go_grad_reduce(const GRedArgs& a, hipStream_t s) {
     const size_t lds = exc_lds_bytes(a.t, NM);
@@ -138,6 +140,7 @@ int launch_grad_reduce_exc<QMC_RAD>(const GRedArgs& a, const RedOut& o, hipStrea
     return 0;
 }
 
+#else
 // static LDS of a kernel plus dynamic bytes within the device's per-block limit
 template <typename K>
 static bool lds_fits(K kernel, size_t dynamic) {
@@ -173,5 +176,7 @@ int launch_eloc_reduce_exc<QMC_RAD>(const ERedArgs& a, const RedOut& o, hipStrea
     red_slot_sum(a.t, a.r, o, s);
     return 0;
 }
+
+#endif
 
 }  // namespace qmc

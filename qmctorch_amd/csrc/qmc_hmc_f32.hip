@@ -5,7 +5,7 @@
 #error "compile with -DQMC_RAD=0 (gto_pure) or -DQMC_RAD=1 (sto)"
 #endif
 #ifndef QMC_HMC_MC
-#error "compile with -DQMC_HMC_MC=1 (single configuration) or -DQMC_HMC_MC=QMC_MAXCONF"
+#error "compile with -DQMC_HMC_MC=1 (ground-state determinant) or -DQMC_HMC_MC=QMC_MAXCONF"
 #endif
 
 namespace qmc {

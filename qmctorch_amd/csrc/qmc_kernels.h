@@ -13,6 +13,7 @@
 #include <type_traits>
 
 #include "qmc_device.h"
+#include "qmc_minors.h"
 
 namespace qmc {
 
@@ -596,6 +597,193 @@ __device__ __forceinline__ void lane_gj(const WalkerLane& L, int nmax, double (&
                         tp, col);
 }
 
+// ---------------------------------------------- small matrices (minors)
+// Up to kMaxMinors columns no lane eliminates: every lane stores its MO row in
+// the wavefront's LDS block, reads the other rows of its group and expands the
+// determinant along its own row (first_row_cofactors).  One exchange instead
+// of two per column, and the same cofactors give the lane's column of A^-1
+// that the kinetic trace, the drift and the adjoints need.  H2O (5 x 5), against
+// the lane eliminations: 8192 walkers x 100 steps 0.699 -> 0.491 ms, HMC of
+// 4096 walkers (L = 10, 10 steps) 0.843 -> 0.557 ms, E_L of 65536 walkers
+// 107 -> 90 us; LiH (STO, 2 x 2, 4 CI terms) 1000 walkers x 100 steps 1.371 ->
+// 1.226 ms.
+// Row stride in doubles: 16-byte aligned rows whose 16-byte loads by 16
+// consecutive lanes fall into distinct LDS banks (12 and 20 words apart), with
+// room for the row's exponent at [NM].
+template <int NM>
+constexpr bool use_minors() {
+    return NM <= kMaxMinors;
+}
+template <int NM>
+constexpr int minor_stride() {
+    return NM <= 5 ? 6 : 10;
+}
+template <int NM>
+__device__ __forceinline__ double* wave_minor_rows() {
+    // 64 lanes' rows and the NM unit rows of groups with fewer
+    __shared__ __attribute__((aligned(16))) double rows[kBlockWaves * (64 + NM) * minor_stride<NM>()];
+    return rows + (threadIdx.x >> 6) * (64 + NM) * minor_stride<NM>();
+}
+
+// Every group of the plan has the expanded matrices' rows (no unit rows needed).
+template <int NM>
+__device__ __forceinline__ bool minors_full(const Tables& t) {
+    return (t.ndown == t.nup || t.ndown == 0) && (t.nup == NM || !t.identity_conf);
+}
+
+// Stores this lane's row.  SCALE (FP64 rows): divided by a power of two that
+// brings its largest entry into [1/2, 1), so that products of N entries far
+// from every nucleus neither underflow nor overflow; returns that exponent.
+// FP32 rows need none (seven factors above 2^-149 stay above 2^-1074).
+// With groups of fewer than NM rows (full = false) the unit rows follow.
+template <int NM, bool SCALE, typename S>
+__device__ __forceinline__ int stage_minor_row(const WalkerLane& L, const S (&mo)[NM], bool full, double* rows) {
+    double* q = rows + L.lane * minor_stride<NM>();
+    int ex = 0;
+    if constexpr (SCALE) {
+        double big = 0.0;
+#pragma unroll
+        for (int k = 0; k < NM; ++k) big = fmax(big, fabs((double)mo[k]));
+        if (big > 0.0 && big < INFINITY) ex = __builtin_amdgcn_frexp_exp(big);
+        q[NM] = (double)ex;
+    }
+#pragma unroll
+    for (int k = 0; k < NM; ++k) q[k] = SCALE ? ldexp((double)mo[k], -ex) : (double)mo[k];
+    if (!full && L.lane < NM) {
+        double* u = rows + (64 + L.lane) * minor_stride<NM>();
+#pragma unroll
+        for (int k = 0; k < NM; ++k) u[k] = k == L.lane ? 1.0 : 0.0;
+        u[NM] = 0.0;
+    }
+    return ex;
+}
+
+// Cofactors c of this lane's row a in its group's matrix (n <= N rows; columns
+// col(k) of the staged rows), in the rows' cyclic order from this lane's: the
+// determinant is sum_k a[k] c[k], negated where `flip` is set, and c / sum a c
+// the lane's column of the inverse.  A group of fewer than N rows is completed
+// by rows of the unit matrix, which leave both unchanged (their columns n..
+// come out as zero cofactors).  ex: the sum of the other rows' exponents.
+template <int N, int NM, bool SCALE, typename Col>
+__device__ __forceinline__ void group_cofactors(const WalkerLane& L, const double* rows, Col col, double (&a)[N],
+                                                double (&c)[N], bool& flip, int& ex) {
+    constexpr int S = minor_stride<NM>();
+    double R[N > 1 ? N - 1 : 1][N];
+    const double* own = rows + L.lane * S;
+    double e = 0.0;
+#pragma unroll
+    for (int k = 0; k < N; ++k) a[k] = own[col(k)];
+#pragma unroll
+    for (int j = 1; j < N; ++j) {
+        const int r0 = L.myrow + j, r = r0 >= N ? r0 - N : r0;
+        const bool unit = r >= L.n_sig;
+        const double* q = rows + (unit ? 64 + r : L.gbase + r) * S;
+#pragma unroll
+        for (int k = 0; k < N; ++k) R[j - 1][k] = q[unit ? k : col(k)];
+        if constexpr (SCALE) e += q[NM];
+    }
+    ex = SCALE ? (int)e : 0;
+    first_row_cofactors<N, SCALE>(R, c);
+    flip = (N & 1) == 0 && (L.myrow & 1);
+}
+
+// log|d1 d2 2^ex| (-inf at zero)
+__device__ __forceinline__ double log_abs_product(double d1, double d2, int ex) {
+    const double m = __builtin_amdgcn_frexp_mant(fabs(d1)) * __builtin_amdgcn_frexp_mant(fabs(d2));
+    ex += __builtin_amdgcn_frexp_exp(d1) + __builtin_amdgcn_frexp_exp(d2) + __builtin_amdgcn_frexp_exp(m);
+    const double l = log_mantissa(__builtin_amdgcn_frexp_mant(m)) + 0.6931471805599453 * (double)ex;
+    return (d1 == 0.0 || d2 == 0.0) ? -INFINITY : l;
+}
+
+// Configuration c of this lane's spin from the staged rows: log|det|, its sign
+// and (INV) y[k] = (A_c^-1)[k][this row], the coefficient of configuration
+// column k, zero past the group's n.  own_ex: this lane's row exponent.
+template <int N, int NM, bool SCALE, bool INV, typename Col>
+__device__ __forceinline__ void minor_det_n(const WalkerLane& L, const double* rows, int own_ex, Col col, double& lg,
+                                            double& sg, double (&y)[NM]) {
+    double a[N], c[N];
+    bool flip;
+    int ex;
+    group_cofactors<N, NM, SCALE>(L, rows, col, a, c, flip, ex);
+    double d = 0.0;
+#pragma unroll
+    for (int k = 0; k < N; ++k) d = fma(a[k], c[k], d);
+    // one determinant for the group (qmc_minors.h): its first lane's
+    const double D = __shfl(flip ? -d : d, L.gbase);
+    lg = log_abs_product(D, 1.0, ex + own_ex);
+    sg = D < 0.0 ? -1.0 : 1.0;
+    if constexpr (INV) {
+        const double id = ldexp(1.0 / (flip ? -D : D), -own_ex);
+#pragma unroll
+        for (int k = 0; k < NM; ++k) y[k] = k < N ? c[k < N ? k : 0] * id : 0.0;
+    }
+}
+
+template <int NM, bool SCALE, bool INV>
+__device__ __forceinline__ void minor_det(const Tables& t, const WalkerLane& L, const double* rows, int own_ex, int c,
+                                          double& lg, double& sg, double (&y)[NM]) {
+    if (t.identity_conf) {
+        minor_det_n<NM, NM, SCALE, INV>(L, rows, own_ex, [](int k) { return k; }, lg, sg, y);
+        return;
+    }
+    const int nconf = L.spin == 0 ? t.nconf_up : t.nconf_dn;
+    const int cc = c < nconf ? c : nconf - 1;  // a spin with fewer configurations repeats its last one, unused
+    const QMC_CONST int* conf = L.spin == 0 ? t.conf_up + cc * t.nup : t.conf_dn + cc * t.ndown;
+    // column k of a group with fewer rows than the other spin's: any (the
+    // cofactors of its columns past n are zero)
+    auto col = [&](int k) { return (int)conf[k < L.n_sig ? k : 0]; };
+    static_for<1, NM + 1>([&](auto nc) {
+        constexpr int N = decltype(nc)::value;
+        if (t.nsig_max == N) minor_det_n<N, NM, SCALE, INV>(L, rows, own_ex, col, lg, sg, y);
+    });
+}
+
+// Single configuration, single CI term: log|D_up D_dn| and its sign in every
+// lane, and (INV) this lane's inverse column y; ksum: the sum of kj over the
+// walker's lanes, in lane order, exchanged together with the rows.
+template <int NM, bool INV, typename T, typename KT>
+__device__ __forceinline__ void slater_single_minors(const Tables& t, const QmcParams& prm, const WalkerLane& L,
+                                                     const T (&mo)[NM], double logc0, KT kj, double& logabs,
+                                                     double& sgn, KT& ksum, double (&y)[NM]) {
+    constexpr bool SCALE = std::is_same<T, double>::value;
+    double* rows = wave_minor_rows<NM>();
+    KT* K = wave_sumbuf<KT>();
+    wave_lds_sync();  // the previous evaluation's loads come first
+    K[L.lane] = kj;
+    const int own_ex = stage_minor_row<NM, SCALE>(L, mo, minors_full<NM>(t), rows);
+    wave_lds_sync();
+    double a[NM], c[NM];
+    bool flip;
+    int ex;
+    group_cofactors<NM, NM, SCALE>(L, rows, [](int k) { return k; }, a, c, flip, ex);
+    ksum = KT(0);
+    for (int u = 0; u < t.nelec; ++u) ksum += K[L.wbase + u];
+    double d = 0.0;
+#pragma unroll
+    for (int k = 0; k < NM; ++k) d = fma(a[k], c[k], d);
+    d = flip ? -d : d;
+    // every lane of the walker takes the determinants of its first up and down
+    // lanes (the lanes' own expansions differ in rounding)
+    const int dn_lane = L.wbase + (t.ndown > 0 ? t.nup : 0);
+    const double du = __shfl(d, L.wbase), dd_ = __shfl(d, dn_lane);
+    const double dd = t.ndown > 0 ? dd_ : 1.0;
+    if constexpr (INV) {
+        const double D = L.spin == 0 ? du : dd;
+        const double id = ldexp(1.0 / (flip ? -D : D), -own_ex);
+#pragma unroll
+        for (int k = 0; k < NM; ++k) y[k] = c[k] * id;
+    }
+    int et = 0;
+    if constexpr (SCALE) {
+        ex += own_ex;
+        const int eu = __shfl(ex, L.wbase), ed = __shfl(ex, dn_lane);
+        et = eu + (t.ndown > 0 ? ed : 0);
+    }
+    const double c0 = ldc(prm.ci, 0);
+    logabs = log_abs_product(du, dd, et) + logc0;
+    sgn = (((du < 0.0) != (dd < 0.0)) != (c0 < 0.0)) ? -1.0 : 1.0;
+}
+
 // Single configuration, single CI term: log|D_up D_dn| and its sign (ground state).
 template <int NM, typename T>
 __device__ __forceinline__ void slater_single(const Tables& t, const QmcParams& prm, const WalkerLane& L,
@@ -610,6 +798,29 @@ __device__ __forceinline__ void slater_single(const Tables& t, const QmcParams& 
     const double ldn = __shfl(lg, dn_lane), sdn = __shfl(sg, dn_lane);
     const double c0 = ldc(prm.ci, 0);
     logabs = lu + (t.ndown > 0 ? ldn : 0.0) + logc0;
+    sgn = su * (t.ndown > 0 ? sdn : 1.0) * (c0 < 0.0 ? -1.0 : 1.0);
+}
+
+// slater_single with the kinetic ratio tr(A^-1 B) (eliminations of [A | B]).
+template <int NM>
+__device__ __forceinline__ void slater_single_kin(const Tables& t, const QmcParams& prm, const WalkerLane& L,
+                                                  const double (&mo)[NM], const double (&bk)[NM], double& logabs,
+                                                  double& sgn, double& kin) {
+    double a[NM], b[NM];
+#pragma unroll
+    for (int j = 0; j < NM; ++j) {
+        a[j] = mo[j];
+        b[j] = bk[j];
+    }
+    double lg, sg, tp;
+    int col;
+    lane_gj<NM>(L, t.nsig_max, a, b, lg, sg, tp, col);
+    kin = seg_sum(tp, L.wbase, t.nelec, t.nelec);
+    const int dn_lane = L.wbase + (t.ndown > 0 ? t.nup : 0);
+    const double lu = __shfl(lg, L.wbase), su = __shfl(sg, L.wbase);
+    const double ldn = __shfl(lg, dn_lane), sdn = __shfl(sg, dn_lane);
+    const double c0 = ldc(prm.ci, 0);
+    logabs = lu + (t.ndown > 0 ? ldn : 0.0) + log(fabs(c0));
     sgn = su * (t.ndown > 0 ? sdn : 1.0) * (c0 < 0.0 ? -1.0 : 1.0);
 }
 
@@ -654,17 +865,34 @@ __device__ __forceinline__ void slater_combine(const Tables& t, const QmcParams&
         sd[c] = 1.0;
         td[c] = 0.0;
     }
+    constexpr bool SCALE = std::is_same<T, double>::value;
+    double* rows = nullptr;
+    int own_ex = 0;
+    if constexpr (use_minors<NM>()) {
+        rows = wave_minor_rows<NM>();
+        wave_lds_sync();  // the previous evaluation's loads come first
+        own_ex = stage_minor_row<NM, SCALE>(L, mo, minors_full<NM>(t), rows);
+        wave_lds_sync();
+    }
 #pragma unroll 1
     for (int c = 0; c < t.nconf_max; ++c) {
         double a[NM], b[NM];
-        gather_conf<NM>(t, L, c, mo, a);
-        if (KIN) gather_conf<NM>(t, L, c, bk, b);
         double lg, sg, tp = 0.0;
-        if constexpr (!KIN) {
+        if constexpr (use_minors<NM>()) {
+            minor_det<NM, SCALE, KIN>(t, L, rows, own_ex, c, lg, sg, a);
+            if constexpr (KIN) {
+                gather_conf<NM>(t, L, c, bk, b);
+#pragma unroll
+                for (int k = 0; k < NM; ++k) tp += k < L.n_sig ? b[k] * a[k] : 0.0;
+            }
+        } else if constexpr (!KIN) {
+            gather_conf<NM>(t, L, c, mo, a);
             lane_det_lds<NM>(a, L.n_sig, t.nsig_max, L.myrow, L.gbase, L.spin, L.gmask, L.lane_real,
                              det_rowbuf<NM>(L), lg, sg);
         } else {
             int col;
+            gather_conf<NM>(t, L, c, mo, a);
+            gather_conf<NM>(t, L, c, bk, b);
             lane_gj<NM>(L, t.nsig_max, a, b, lg, sg, tp, col);
         }
         const double tr = KIN ? seg_sum(tp, L.gbase, L.n_sig, t.nsig_max) : 0.0;
@@ -1233,8 +1461,11 @@ struct KArgs {
     QmcWfOut out;
 };
 
-// psi / kinetic / local energy of the walkers of one wavefront.
-template <typename T, int NM, int RAD, bool ELOC, typename AO = AoGeneric, bool EXC = false>
+// psi / kinetic / local energy of the walkers of one wavefront.  MULTI: plans
+// of several configurations (up to QMC_MAXCONF unique ones per spin); without
+// it the plan is the ground-state determinant (identity_conf) and the kernel
+// holds none of their registers and code.
+template <typename T, int NM, int RAD, bool ELOC, bool MULTI, typename AO = AoGeneric, bool EXC = false>
 __device__ __forceinline__ void wf_walkers(const KArgs& a, const WalkerLane& L) {
     const Tables& t = a.t;
     const double* p = a.pos + (size_t)L.wclamp * 3 * t.nelec + 3 * L.e;
@@ -1256,22 +1487,52 @@ __device__ __forceinline__ void wf_walkers(const KArgs& a, const WalkerLane& L) 
     if (ELOC) {
         const double l2 = jlap + jgx * jgx + jgy * jgy + jgz * jgz;  // (lap J)/J
 #pragma unroll
-        for (int m = 0; m < NM; ++m)
+        for (int m = 0; m < NM; ++m) {
             bk[m] = -0.5 * ((double)lp[m] + 2.0 * (jgx * (double)gx[m] + jgy * (double)gy[m] + jgz * (double)gz[m]) +
                             l2 * (double)mo[m]);
+            // formed here: the compiler otherwise sinks the row and its whole AO
+            // evaluation past the determinants, spilling what it holds meanwhile
+            asm volatile("" : "+v"(bk[m]));
+        }
     }
-    double logabs, sgn, kin;
-    if constexpr (EXC)
-        slater_exc<NM, ELOC>(t, a.p, L, mo, bk, (double*)qmc_dyn_lds, logabs, sgn, kin);
-    else
-        slater_combine<NM, ELOC>(t, a.p, L, mo, bk, logabs, sgn, kin);
-    const double logj = seg_sum(0.5 * kee + ken, L.wbase, t.nelec, t.nelec);
-    double epot = 0.0, svee = 0.0, sven = 0.0;
-    if (ELOC) {
-        svee = seg_sum(vee, L.wbase, t.nelec, t.nelec);
-        sven = seg_sum(ven, L.wbase, t.nelec, t.nelec);
-        epot = svee + sven + t.vnn;
+    double logabs, sgn, kin = 0.0, logj, svee = 0.0, sven = 0.0;
+    if constexpr (!EXC && !MULTI && use_minors<NM>()) {
+        double yc[NM];
+        slater_single_minors<NM, ELOC>(t, a.p, L, mo, log(fabs(ldc(a.p.ci, 0))), 0.5 * kee + ken, logabs, sgn, logj, yc);
+        if constexpr (ELOC) {
+            // this lane's share of tr(A^-1 B), V_ee and V_en: one exchange for the three sums
+            double tp = 0.0;
+#pragma unroll
+            for (int k = 0; k < NM; ++k) tp += k < L.n_sig ? bk[k] * yc[k] : 0.0;
+            double* V = wave_posbuf<double>();
+            wave_lds_sync();
+            V[L.lane * 4 + 0] = tp;
+            V[L.lane * 4 + 1] = vee;
+            V[L.lane * 4 + 2] = ven;
+            wave_lds_sync();
+            for (int u = 0; u < t.nelec; ++u) {
+                const double* q = V + (L.wbase + u) * 4;
+                kin += q[0];
+                svee += q[1];
+                sven += q[2];
+            }
+        }
+    } else {
+        if constexpr (EXC)
+            slater_exc<NM, ELOC>(t, a.p, L, mo, bk, (double*)qmc_dyn_lds, logabs, sgn, kin);
+        else if constexpr (MULTI)
+            slater_combine<NM, ELOC>(t, a.p, L, mo, bk, logabs, sgn, kin);
+        else if constexpr (ELOC)
+            slater_single_kin<NM>(t, a.p, L, mo, bk, logabs, sgn, kin);
+        else
+            slater_single<NM>(t, a.p, L, mo, log(fabs(ldc(a.p.ci, 0))), logabs, sgn);
+        logj = seg_sum(0.5 * kee + ken, L.wbase, t.nelec, t.nelec);
+        if (ELOC) {
+            svee = seg_sum(vee, L.wbase, t.nelec, t.nelec);
+            sven = seg_sum(ven, L.wbase, t.nelec, t.nelec);
+        }
     }
+    const double epot = svee + sven + t.vnn;
     if (L.valid && L.e == 0) {
         const double la = logabs + logj;
         if (a.out.logabs) a.out.logabs[L.w] = la;
@@ -1287,11 +1548,18 @@ __device__ __forceinline__ void wf_walkers(const KArgs& a, const WalkerLane& L) 
     }
 }
 
-template <typename T, int NM, int RAD, bool ELOC, typename AO = AoGeneric>
-__global__ __launch_bounds__(kBlock) void wf_kernel(KArgs a) {
+// Waves per SIMD the evaluation kernels are held to: what their registers allow
+// without spilling (168 VGPRs up to 5 columns, 256 up to 7).
+template <int NM>
+constexpr int wf_waves() {
+    return NM <= 5 ? 3 : (NM <= 7 ? 2 : 1);
+}
+
+template <typename T, int NM, int RAD, bool ELOC, bool MULTI, typename AO = AoGeneric>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(wf_waves<NM>()))) void wf_kernel(KArgs a) {
     const WalkerLane L = lane_layout(a.t, a.nw);
     if ((int64_t)L.wave * L.G >= a.nw) return;  // whole wavefront beyond the batch
-    wf_walkers<T, NM, RAD, ELOC, AO>(a, L);
+    wf_walkers<T, NM, RAD, ELOC, MULTI, AO>(a, L);
 }
 
 // Kernels of exc_mode plans: one wavefront per block, dynamic LDS of
@@ -1300,7 +1568,7 @@ template <typename T, int NM, int RAD, bool ELOC>
 __global__ __launch_bounds__(64) void wf_kernel_exc(KArgs a) {
     const WalkerLane L = lane_layout(a.t, a.nw);
     if ((int64_t)L.wave * L.G >= a.nw) return;
-    wf_walkers<T, NM, RAD, ELOC, AoGeneric, true>(a, L);
+    wf_walkers<T, NM, RAD, ELOC, true, AoGeneric, true>(a, L);
 }
 
 // Many systems in one launch: job j owns global waves [wave0[j], wave0[j+1]).
@@ -1309,15 +1577,15 @@ struct WJob {
     int64_t wave0;
 };
 
-template <typename T, int NM, int RAD, bool ELOC, typename AO = AoGeneric>
-__global__ __launch_bounds__(kBlock) void wf_batch_kernel(const WJob* __restrict__ jobs, int njobs, int nwaves) {
+template <typename T, int NM, int RAD, bool ELOC, bool MULTI, typename AO = AoGeneric>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(wf_waves<NM>()))) void wf_batch_kernel(const WJob* __restrict__ jobs, int njobs, int nwaves) {
     const int wave = global_wave();
     if (wave >= nwaves) return;
     const int j = find_job(jobs, njobs, wave);
     const KArgs a = jobs[j].a;
     const WalkerLane L = lane_layout_w(a.t, a.nw, wave - (int)jobs[j].wave0);
     if ((int64_t)L.wave * L.G >= a.nw) return;
-    wf_walkers<T, NM, RAD, ELOC, AO>(a, L);
+    wf_walkers<T, NM, RAD, ELOC, MULTI, AO>(a, L);
 }
 
 // wf_batch_kernel for excitation plans: one wavefront per block (as
@@ -1330,7 +1598,7 @@ __global__ __launch_bounds__(64) void wf_batch_kernel_exc(const WJob* __restrict
     const KArgs a = jobs[j].a;
     const WalkerLane L = lane_layout_w(a.t, a.nw, wave - (int)jobs[j].wave0);
     if ((int64_t)L.wave * L.G >= a.nw) return;
-    wf_walkers<T, NM, RAD, ELOC, AoGeneric, true>(a, L);
+    wf_walkers<T, NM, RAD, ELOC, true, AoGeneric, true>(a, L);
 }
 
 struct SArgs {
@@ -1342,7 +1610,7 @@ struct SArgs {
 };
 
 // wlds: with WLDS, this wavefront's LDS copy of the entry-ordered W rows
-template <typename T, int NM, int RAD, typename AO = AoGeneric, bool WLDS = false, bool EXC = false>
+template <typename T, int NM, int RAD, bool MULTI, typename AO = AoGeneric, bool WLDS = false, bool EXC = false>
 __device__ __forceinline__ double eval_logpsi(const Tables& t, const QmcParams& prm, const WalkerLane& L, double x,
                                               double y, double z, double logc0, double& sgn,
                                               const T* wlds = nullptr) {
@@ -1368,11 +1636,16 @@ __device__ __forceinline__ double eval_logpsi(const Tables& t, const QmcParams& 
     if constexpr (EXC) {
         double bk[NM], kin;
         slater_exc<NM, false>(t, prm, L, mo, bk, (double*)qmc_dyn_lds, logabs, sgn, kin);
-    } else if (t.identity_conf) {
-        slater_single<NM>(t, prm, L, mo, logc0, logabs, sgn);
-    } else {
+    } else if constexpr (MULTI) {
         double bk[NM], kin;
         slater_combine<NM, false>(t, prm, L, mo, bk, logabs, sgn, kin);
+    } else if constexpr (use_minors<NM>()) {
+        T ksum;
+        double y_[NM];
+        slater_single_minors<NM, false>(t, prm, L, mo, logc0, kj, logabs, sgn, ksum, y_);
+        return logabs + (double)ksum;
+    } else {
+        slater_single<NM>(t, prm, L, mo, logc0, logabs, sgn);
     }
     // ln J of the walker, summed in the bulk precision
     return logabs + (double)seg_sum<T>(kj, L.wbase, t.nelec, t.nelec);
@@ -1380,7 +1653,7 @@ __device__ __forceinline__ double eval_logpsi(const Tables& t, const QmcParams& 
 
 // Persistent Metropolis sweep: nstep all-electron moves per launch, walker
 // state in registers (sampler/metropolis.py:134-165, 256-298).
-template <typename T, int NM, int RAD, typename AO = AoGeneric, bool WLDS = false, bool EXC = false>
+template <typename T, int NM, int RAD, bool MULTI, typename AO = AoGeneric, bool WLDS = false, bool EXC = false>
 __device__ __forceinline__ void sweep_walkers(const SArgs& a, const WalkerLane& L, const T* wlds = nullptr) {
     const Tables& t = a.t;
     const int Ne = t.nelec;
@@ -1390,7 +1663,7 @@ __device__ __forceinline__ void sweep_walkers(const SArgs& a, const WalkerLane& 
     double lp;
     const double logc0 = log(fabs(ldc(a.p.ci, 0)));  // single-configuration CI weight, once per launch
     if (a.sw.init_logpsi) {
-        lp = eval_logpsi<T, NM, RAD, AO, WLDS, EXC>(t, a.p, L, x, y, z, logc0, sgn, wlds);
+        lp = eval_logpsi<T, NM, RAD, MULTI, AO, WLDS, EXC>(t, a.p, L, x, y, z, logc0, sgn, wlds);
     } else {
         lp = a.wk.logabs[L.wclamp];
         sgn = a.wk.sign[L.wclamp];
@@ -1456,7 +1729,7 @@ __device__ __forceinline__ void sweep_walkers(const SArgs& a, const WalkerLane& 
         }
         const double xn = x + nx, yn = y + ny, zn = z + nz;
         double sgn_n;
-        double lpn = eval_logpsi<T, NM, RAD, AO, WLDS, EXC>(t, a.p, Ls, xn, yn, zn, logc0, sgn_n, wlds);
+        double lpn = eval_logpsi<T, NM, RAD, MULTI, AO, WLDS, EXC>(t, a.p, Ls, xn, yn, zn, logc0, sgn_n, wlds);
         if (lpn < lp_zero) lpn = lp_eps;
         // accept iff min(1, psi'^2/psi^2) >= U  <=>  2 (lpn - lp) >= log U; the
         // logarithm in the bulk precision (the hardware log2 in the mixed sweep,
@@ -1507,12 +1780,12 @@ __device__ __forceinline__ void sweep_walkers(const SArgs& a, const WalkerLane& 
 // The 16- and 24-orbital buckets (one or two walkers per wavefront) are held to
 // two waves per SIMD, so a second wavefront covers the latency of the FP64
 // elimination; left alone the compiler keeps VGPRs and AGPRs for one.
-template <typename T, int NM, int RAD, typename AO = AoGeneric>
+template <typename T, int NM, int RAD, bool MULTI, typename AO = AoGeneric>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NM >= 16 ? 2 : 1))) void sweep_kernel(
     SArgs a) {
     const WalkerLane L = lane_layout(a.t, a.nw);
     if ((int64_t)L.wave * L.G >= a.nw) return;
-    sweep_walkers<T, NM, RAD, AO>(a, L);
+    sweep_walkers<T, NM, RAD, MULTI, AO>(a, L);
 }
 
 // sweep_kernel with the entry-ordered W rows staged in LDS once per block
@@ -1522,7 +1795,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NM >= 16
 // which a 50-step loop otherwise hoists and spills to VGPR lanes.  Two waves
 // per SIMD are requested explicitly: the extra VGPRs of the LDS operands would
 // otherwise leave one.
-template <typename T, int NM, int RAD, typename AO>
+template <typename T, int NM, int RAD, bool MULTI, typename AO>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void sweep_kernel_wlds(SArgs a) {
     {
         T* w = (T*)qmc_dyn_lds;
@@ -1533,14 +1806,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     }
     const WalkerLane L = lane_layout(a.t, a.nw);
     if ((int64_t)L.wave * L.G >= a.nw) return;
-    sweep_walkers<T, NM, RAD, AO, true>(a, L, (const T*)qmc_dyn_lds);
+    sweep_walkers<T, NM, RAD, MULTI, AO, true>(a, L, (const T*)qmc_dyn_lds);
 }
 
 template <typename T, int NM, int RAD>
 __global__ __launch_bounds__(64) void sweep_kernel_exc(SArgs a) {
     const WalkerLane L = lane_layout(a.t, a.nw);
     if ((int64_t)L.wave * L.G >= a.nw) return;
-    sweep_walkers<T, NM, RAD, AoGeneric, false, true>(a, L);
+    sweep_walkers<T, NM, RAD, true, AoGeneric, false, true>(a, L);
 }
 
 // Sweeps of many systems (each with its own walkers, step count and seed) in
@@ -1561,10 +1834,10 @@ __global__ __launch_bounds__(64) void sweep_batch_kernel_exc(const SJob* __restr
     const SArgs a = jobs[j].a;
     const WalkerLane L = lane_layout_w(a.t, a.nw, wave - (int)jobs[j].wave0);
     if ((int64_t)L.wave * L.G >= a.nw) return;
-    sweep_walkers<T, NM, RAD, AoGeneric, false, true>(a, L);
+    sweep_walkers<T, NM, RAD, true, AoGeneric, false, true>(a, L);
 }
 
-template <typename T, int NM, int RAD, typename AO = AoGeneric>
+template <typename T, int NM, int RAD, bool MULTI, typename AO = AoGeneric>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NM >= 16 ? 2 : 1))) void sweep_batch_kernel(
     const SJob* __restrict__ jobs, int njobs, int nwaves) {
     const int wave = global_wave();
@@ -1573,13 +1846,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NM >= 16
     const SArgs a = jobs[j].a;
     const WalkerLane L = lane_layout_w(a.t, a.nw, wave - (int)jobs[j].wave0);
     if ((int64_t)L.wave * L.G >= a.nw) return;
-    sweep_walkers<T, NM, RAD, AO>(a, L);
+    sweep_walkers<T, NM, RAD, MULTI, AO>(a, L);
 }
 
 // sweep_batch_kernel with W in LDS: every wavefront stages the W rows of its
 // own job into its slice of wstride elements (dynamic LDS of 4 slices), so
 // each walker runs the arithmetic of sweep_kernel_wlds exactly.
-template <typename T, int NM, int RAD, typename AO>
+template <typename T, int NM, int RAD, bool MULTI, typename AO>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void sweep_batch_kernel_wlds(
     const SJob* __restrict__ jobs, int njobs, int nwaves, int wstride) {
     const int wave = global_wave();
@@ -1593,7 +1866,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     const int n = a.t.nentry * NM;  // <= wstride (one layout per launch)
     for (int i = L.lane; i < n; i += 64) w[i] = src[i];
     wave_lds_sync();
-    sweep_walkers<T, NM, RAD, AO, true>(a, L, w);
+    sweep_walkers<T, NM, RAD, MULTI, AO, true>(a, L, w);
 }
 
 // ------------------------------------------------------------------ drift
@@ -1657,8 +1930,8 @@ __device__ __forceinline__ T jastrow_value_grad(const Tables& t, const QmcParams
 // lane that pivoted column k holds row k); the rows are transposed through
 // the wavefront's LDS block lds[64][NM] so that lane i reads column i.  AO and
 // MO rows in T, elimination and combination in FP64.  MC bounds the unique
-// configurations per spin (1, or QMC_MAXCONF for multi-configuration plans):
-// the per-configuration values live in registers.
+// configurations per spin (1 for the ground-state determinant, QMC_MAXCONF for
+// every other plan): the per-configuration values live in registers.
 template <typename T, int NM, int RAD, int MC, typename AO = AoGeneric>
 __device__ __forceinline__ double eval_drift(const Tables& t, const QmcParams& prm, const WalkerLane& L, double x,
                                              double y, double z, double logc0, double* lds, double& sgn,
@@ -1669,10 +1942,42 @@ __device__ __forceinline__ double eval_drift(const Tables& t, const QmcParams& p
     // values and gradients only: the row's Laplacian terms are dead code here
     MoSink<T, NM, true, T, false> sink{(const T*)prm.entry_w, t.nmo, mo, gx, gy, gz, nullptr};
     AO::template row<T, RAD, true, false>(t, prm, x, y, z, sink);
+    if constexpr (use_minors<NM>()) {
+        // formed here, not sunk past the determinants (as the kinetic row of wf_walkers)
+#pragma unroll
+        for (int m = 0; m < NM; ++m) asm volatile("" : "+v"(gx[m]), "+v"(gy[m]), "+v"(gz[m]));
+    }
     T jg[3];
     const T kj = jastrow_value_grad<T>(t, prm, L, x, y, z, jg);
+    if constexpr (MC == 1 && use_minors<NM>()) {
+        double logabs, yc[NM];
+        T ksum;
+        slater_single_minors<NM, true>(t, prm, L, mo, logc0, kj, logabs, sgn, ksum, yc);
+        double v0 = 0.0, v1 = 0.0, v2 = 0.0;
+#pragma unroll
+        for (int k = 0; k < NM; ++k) {
+            if (k < L.n_sig) {
+                v0 += yc[k] * (double)gx[k];
+                v1 += yc[k] * (double)gy[k];
+                v2 += yc[k] * (double)gz[k];
+            }
+        }
+        dr[0] = v0 + (double)jg[0];
+        dr[1] = v1 + (double)jg[1];
+        dr[2] = v2 + (double)jg[2];
+        return logabs + (double)ksum;
+    } else {
     const double logj = (double)seg_sum<T>(kj, L.wbase, t.nelec, t.nelec);
 
+    constexpr bool SCALE = std::is_same<T, double>::value;
+    double* rows = nullptr;
+    int own_ex = 0;
+    if constexpr (use_minors<NM>()) {
+        rows = wave_minor_rows<NM>();
+        wave_lds_sync();  // the previous evaluation's loads come first
+        own_ex = stage_minor_row<NM, SCALE>(L, mo, minors_full<NM>(t), rows);
+        wave_lds_sync();
+    }
     double ld[MC], sd[MC], s0[MC], s1[MC], s2[MC];
 #pragma unroll
     for (int c = 0; c < MC; ++c) {
@@ -1682,18 +1987,23 @@ __device__ __forceinline__ double eval_drift(const Tables& t, const QmcParams& p
 #pragma unroll 1
     for (int c = 0; c < t.nconf_max; ++c) {
         double aa[NM], ib[NM];
-        gather_conf<NM>(t, L, c, mo, aa);
+        double lg, sg;
+        if constexpr (use_minors<NM>()) {
+            minor_det<NM, SCALE, true>(t, L, rows, own_ex, c, lg, sg, ib);
+        } else {
+            gather_conf<NM>(t, L, c, mo, aa);
 #pragma unroll
-        for (int j = 0; j < NM; ++j) ib[j] = (j == L.myrow) ? 1.0 : 0.0;
-        double lg, sg, tp;
-        int col;
-        lane_gj<NM>(L, t.nsig_max, aa, ib, lg, sg, tp, col);
-        wave_lds_sync();  // earlier reads of the row buffer are done
-        if (L.lane_real && col >= 0) {
+            for (int j = 0; j < NM; ++j) ib[j] = (j == L.myrow) ? 1.0 : 0.0;
+            double tp;
+            int col;
+            lane_gj<NM>(L, t.nsig_max, aa, ib, lg, sg, tp, col);
+            wave_lds_sync();  // earlier reads of the row buffer are done
+            if (L.lane_real && col >= 0) {
 #pragma unroll
-            for (int j = 0; j < NM; ++j) lds[(L.gbase + col) * NM + j] = ib[j];
+                for (int j = 0; j < NM; ++j) lds[(L.gbase + col) * NM + j] = ib[j];
+            }
+            wave_lds_sync();
         }
-        wave_lds_sync();
         double ga[NM], gb[NM], gc[NM];
         gather_conf<NM>(t, L, c, gx, ga);
         gather_conf<NM>(t, L, c, gy, gb);
@@ -1702,7 +2012,7 @@ __device__ __forceinline__ double eval_drift(const Tables& t, const QmcParams& p
 #pragma unroll
         for (int k = 0; k < NM; ++k) {
             if (k < L.n_sig) {
-                const double inv = lds[(L.gbase + k) * NM + L.myrow];
+                const double inv = use_minors<NM>() ? ib[k] : lds[(L.gbase + k) * NM + L.myrow];
                 v0 += inv * ga[k];
                 v1 += inv * gb[k];
                 v2 += inv * gc[k];
@@ -1721,7 +2031,7 @@ __device__ __forceinline__ double eval_drift(const Tables& t, const QmcParams& p
     }
     const int up_lane = L.wbase, dn_lane = L.wbase + (t.ndown > 0 ? t.nup : 0);
     double logabs;
-    if (t.identity_conf) {
+    if (MC == 1) {  // the ground-state determinant
         const double lu = __shfl(ld[0], up_lane), su = __shfl(sd[0], up_lane);
         const double lo = __shfl(ld[0], dn_lane), so = __shfl(sd[0], dn_lane);
         const double c0 = ldc(prm.ci, 0);
@@ -1790,6 +2100,7 @@ __device__ __forceinline__ double eval_drift(const Tables& t, const QmcParams& p
     dr[1] += (double)jg[1];
     dr[2] += (double)jg[2];
     return logabs + logj;
+    }
 }
 
 // log|psi| (every lane) and the drift of this lane's electron for plans with
@@ -1850,6 +2161,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NM <= 8 
     double* lds;  // row transposes (above 8 rows also the pivot rows), or the exc_gamma rows
     if constexpr (EXC)
         lds = (double*)qmc_dyn_lds;
+    else if constexpr (use_minors<NM>())
+        lds = nullptr;
     else
         lds = wave_rowbuf<NM>();
     const Tables& t = a.t;
@@ -2004,26 +2317,99 @@ struct GArgs {
     double* dexp_rows;   // [nw*nelec][nprim_ref] or null
 };
 
+// Small matrices: this lane's row stored for minor_det; returns its exponent.
+template <int NM>
+__device__ __forceinline__ int stage_conf_rows(const Tables& t, const WalkerLane& L, const double (&mo)[NM]) {
+    int own_ex = 0;
+    if constexpr (use_minors<NM>()) {
+        wave_lds_sync();  // the previous walkers' loads come first
+        own_ex = stage_minor_row<NM, true>(L, mo, minors_full<NM>(t), wave_minor_rows<NM>());
+        wave_lds_sync();
+    }
+    return own_ex;
+}
+
+// log|det| and sign of configuration c of this lane's spin and its inverse
+// column inv[k] = (A_c^-1)[k][this row], zero past the group's n (rows staged
+// by stage_conf_rows).  Above the minors' sizes the lane that pivoted column k
+// of [A | I] holds row k of A^-1, and the transpose goes through the
+// wavefront's row buffer, which then holds A_c^-1 of every group: (k, l) at
+// [(gbase + k) NM + l].
+template <int NM>
+__device__ __forceinline__ void conf_inverse(const Tables& t, const WalkerLane& L, int c, const double (&mo)[NM],
+                                             int own_ex, double& lg, double& sg, double (&inv)[NM]) {
+    if constexpr (use_minors<NM>()) {
+        minor_det<NM, true, true>(t, L, wave_minor_rows<NM>(), own_ex, c, lg, sg, inv);
+    } else {
+        double aa[NM], bb[NM], tp;
+        int col;
+        gather_conf<NM>(t, L, c, mo, aa);
+#pragma unroll
+        for (int j = 0; j < NM; ++j) bb[j] = (j == L.myrow) ? 1.0 : 0.0;
+        lane_gj<NM>(L, t.nsig_max, aa, bb, lg, sg, tp, col);
+        double* rb = wave_rowbuf<NM>();
+        wave_lds_sync();  // the elimination's loads come first
+        if (L.lane_real && col >= 0) {
+#pragma unroll
+            for (int j = 0; j < NM; ++j) rb[(L.gbase + col) * NM + j] = bb[j];
+        }
+        wave_lds_sync();
+#pragma unroll
+        for (int k = 0; k < NM; ++k) inv[k] = k < L.n_sig ? rb[(L.gbase + (k < L.n_sig ? k : 0)) * NM + L.myrow] : 0.0;
+    }
+}
+
+// zz = column of A^-1 B A^-1 for this lane's row, inv its column of A^-1: with
+// Y_l the inverse column of row l and B_l its kinetic row,
+// zz = sum_l Y_l (B_l . inv).  B_l: row [lane][NM] of brow, column k of the
+// configuration at col(k); Y_l: ycol [lane][NM] (small matrices, written here)
+// or the row buffer left by conf_inverse.
+template <int NM, typename Col>
+__device__ __forceinline__ void inverse_b_inverse(const Tables& t, const WalkerLane& L, const double (&inv)[NM],
+                                                  const double* brow, double* ycol, Col col, double (&zz)[NM]) {
+    const double* rb = nullptr;
+    if constexpr (use_minors<NM>()) {
+        wave_lds_sync();  // the previous configuration's loads come first
+#pragma unroll
+        for (int k = 0; k < NM; ++k) ycol[L.lane * NM + k] = inv[k];
+        wave_lds_sync();
+    } else {
+        rb = wave_rowbuf<NM>() + L.gbase * NM;
+    }
+#pragma unroll
+    for (int k = 0; k < NM; ++k) zz[k] = 0.0;
+    for (int l = 0; l < t.nsig_max; ++l) {
+        const int ll = l < L.n_sig ? l : 0, lane_l = L.gbase + ll;
+        double tl = 0.0;
+#pragma unroll
+        for (int k = 0; k < NM; ++k)
+            if (k < L.n_sig) tl += brow[lane_l * NM + col(k)] * inv[k];
+        if (l >= L.n_sig) tl = 0.0;
+#pragma unroll
+        for (int k = 0; k < NM; ++k)
+            if (k < L.n_sig) zz[k] += tl * (use_minors<NM>() ? ycol[lane_l * NM + k] : rb[k * NM + ll]);
+    }
+}
+
 // log|det| and sign of every unique configuration of the lane's spin; with
 // INV the inverse column of this lane's row, weighted by om[c] and scattered
 // to MO columns, is accumulated into gam (second pass of the adjoint).
 template <int NM, bool INV>
-__device__ __forceinline__ void conf_dets(const Tables& t, const WalkerLane& L, const double (&mo)[NM],
+__device__ __forceinline__ void conf_dets(const Tables& t, const WalkerLane& L, const double (&mo)[NM], int own_ex,
                                           double (&ld)[QMC_MAXCONF], double (&sd)[QMC_MAXCONF],
                                           const double (&om)[QMC_MAXCONF], double (&gam)[NM]) {
 #pragma unroll 1
     for (int c = 0; c < t.nconf_max; ++c) {
-        double aa[NM], bb[NM];
-        gather_conf<NM>(t, L, c, mo, aa);
-#pragma unroll
-        for (int j = 0; j < NM; ++j) bb[j] = (j == L.myrow) ? 1.0 : 0.0;
-        double lg, sg, tp;
-        int col;
-        if constexpr (INV)
-            lane_gj<NM>(L, t.nsig_max, aa, bb, lg, sg, tp, col);
-        else
+        double aa[NM], lg, sg;
+        if constexpr (INV) {
+            conf_inverse<NM>(t, L, c, mo, own_ex, lg, sg, aa);
+        } else if constexpr (use_minors<NM>()) {
+            minor_det<NM, true, false>(t, L, wave_minor_rows<NM>(), own_ex, c, lg, sg, aa);
+        } else {
+            gather_conf<NM>(t, L, c, mo, aa);
             lane_det_lds<NM>(aa, L.n_sig, t.nsig_max, L.myrow, L.gbase, L.spin, L.gmask, L.lane_real,
                              det_rowbuf<NM>(L), lg, sg);
+        }
 #pragma unroll
         for (int c2 = 0; c2 < QMC_MAXCONF; ++c2)
             if (c2 == c) {
@@ -2037,25 +2423,13 @@ __device__ __forceinline__ void conf_dets(const Tables& t, const WalkerLane& L, 
                 if (c2 == c) w = om[c2];
             const QMC_CONST int* conf = L.spin == 0 ? t.conf_up + c * t.nup : t.conf_dn + c * t.ndown;
             const int nconf = L.spin == 0 ? t.nconf_up : t.nconf_dn;
-            // the lane that pivoted column k holds row k of A^-1 in bb; this
-            // lane needs (A^-1)[k][myrow] for every k
-            for (int k = 0; k < t.nsig_max; ++k) {
-                int src = 0;
-                for (int s = 0; s < t.nsig_max; ++s) {
-                    const int cs = __shfl(col, L.gbase + (s < L.n_sig ? s : 0));
-                    if (s < L.n_sig && cs == k) src = s;
-                }
-                double inv_ki = 0.0;
 #pragma unroll
-                for (int j = 0; j < NM; ++j) {
-                    const double vj = __shfl(bb[j], L.gbase + src);
-                    if (j == L.myrow) inv_ki = vj;
-                }
+            for (int k = 0; k < NM; ++k) {
                 if (k < L.n_sig && c < nconf) {
                     const int mcol = t.identity_conf ? k : conf[k];
 #pragma unroll
                     for (int m = 0; m < NM; ++m)
-                        if (m == mcol) gam[m] += w * inv_ki;
+                        if (m == mcol) gam[m] += w * aa[k];
                 }
             }
         }
@@ -2138,7 +2512,8 @@ __global__ __launch_bounds__(kBlock) void grad_kernel(GArgs a) {
     }
 #pragma unroll
     for (int m = 0; m < NM; ++m) gam[m] = 0.0;
-    conf_dets<NM, false>(t, L, mo, ld, sd, om, gam);
+    const int own_ex = stage_conf_rows<NM>(t, L, mo);
+    conf_dets<NM, false>(t, L, mo, own_ex, ld, sd, om, gam);
     // CI weights omega_n = c_n D_n / S with D_n = D_up D_dn (slater_pooling.py:96-111)
     const int up_lane = L.wbase, dn_lane = L.wbase + (t.ndown > 0 ? t.nup : 0);
     double lu[QMC_MAXCONF], su[QMC_MAXCONF], lo[QMC_MAXCONF], so[QMC_MAXCONF];
@@ -2188,7 +2563,7 @@ __global__ __launch_bounds__(kBlock) void grad_kernel(GArgs a) {
             if (c == mine) om[c] += ldc(a.p.ci, n) * dn_s;
         if (v && L.e == 0) a.dci[(size_t)L.w * t.nci + n] = dn_s;
     }
-    conf_dets<NM, true>(t, L, mo, ld, sd, om, gam);
+    conf_dets<NM, true>(t, L, mo, own_ex, ld, sd, om, gam);
     if (v) {
         double* gr = a.gamma_rows + row * t.nmo;
 #pragma unroll
@@ -2298,56 +2673,6 @@ __device__ __forceinline__ void jastrow_w_derivs(const Tables& t, const QmcParam
     }
 }
 
-// For this lane: column myrow of A^-1 (inv[k]) and of A^-1 B A^-1 (zz[k]), k < n,
-// from the two eliminations [A|B] (rows of X = A^-1 B in xb) and [A|I] (rows of
-// A^-1 in ib); col is this lane's pivot column (identical in both runs).
-template <int NM>
-__device__ __forceinline__ void inverse_columns(const WalkerLane& L, int nmax, int col, const double (&xb)[NM],
-                                                const double (&ib)[NM], double (&inv)[NM], double (&zz)[NM]) {
-#pragma unroll
-    for (int k = 0; k < NM; ++k) inv[k] = zz[k] = 0.0;
-    int srcs[NM];
-#pragma unroll
-    for (int k = 0; k < NM; ++k) {
-        int src = 0;
-        if (k < nmax) {
-            for (int s = 0; s < nmax; ++s) {
-                const int cs = __shfl(col, L.gbase + (s < L.n_sig ? s : 0));
-                if (s < L.n_sig && cs == k) src = s;
-            }
-        }
-        srcs[k] = src;
-    }
-#pragma unroll
-    for (int k = 0; k < NM; ++k) {
-        if (k < nmax) {
-            double v = 0.0;
-#pragma unroll
-            for (int j = 0; j < NM; ++j) {
-                if (j < nmax) {
-                    const double vj = __shfl(ib[j], L.gbase + srcs[k]);
-                    if (j == L.myrow) v = vj;
-                }
-            }
-            inv[k] = (k < L.n_sig) ? v : 0.0;
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < NM; ++k) {
-        if (k < nmax) {
-            double s = 0.0;
-#pragma unroll
-            for (int j = 0; j < NM; ++j) {
-                if (j < nmax) {
-                    const double xkj = __shfl(xb[j], L.gbase + srcs[k]);
-                    s += xkj * inv[j];
-                }
-            }
-            zz[k] = (k < L.n_sig) ? s : 0.0;
-        }
-    }
-}
-
 template <int NM, int RAD>
 __global__ __launch_bounds__(kBlock) void eloc_grad_kernel(EArgs a) {
     const Tables& t = a.t;
@@ -2393,6 +2718,12 @@ __global__ __launch_bounds__(kBlock) void eloc_grad_kernel(EArgs a) {
         bk[m] = -0.5 * (lp[m] + 2.0 * (g[0] * gx[m] + g[1] * gy[m] + g[2] * gz[m]) + l2 * mo[m]);
 
     // pass 1: log|det|, sign and trace of every unique configuration
+    __shared__ double bsh[kBlockWaves * 64 * NM], ysh[use_minors<NM>() ? kBlockWaves * 64 * NM : 1];
+    double* brow = bsh + (threadIdx.x >> 6) * 64 * NM;
+    double* ycol = use_minors<NM>() ? ysh + (threadIdx.x >> 6) * 64 * NM : nullptr;
+#pragma unroll
+    for (int k = 0; k < NM; ++k) brow[L.lane * NM + k] = bk[k];
+    const int own_ex = stage_conf_rows<NM>(t, L, mo);
     double ld[QMC_MAXCONF], sd[QMC_MAXCONF], td[QMC_MAXCONF];
 #pragma unroll
     for (int c = 0; c < QMC_MAXCONF; ++c) {
@@ -2402,12 +2733,12 @@ __global__ __launch_bounds__(kBlock) void eloc_grad_kernel(EArgs a) {
     }
 #pragma unroll 1
     for (int c = 0; c < t.nconf_max; ++c) {
-        double aa[NM], bb[NM];
-        gather_conf<NM>(t, L, c, mo, aa);
+        double inv[NM], bb[NM];
         gather_conf<NM>(t, L, c, bk, bb);
-        double lg, sg, tp;
-        int col;
-        lane_gj<NM>(L, t.nsig_max, aa, bb, lg, sg, tp, col);
+        double lg, sg, tp = 0.0;
+        conf_inverse<NM>(t, L, c, mo, own_ex, lg, sg, inv);
+#pragma unroll
+        for (int k = 0; k < NM; ++k) tp += k < L.n_sig ? bb[k] * inv[k] : 0.0;
         const double tr = seg_sum(tp, L.gbase, L.n_sig, t.nsig_max);
 #pragma unroll
         for (int c2 = 0; c2 < QMC_MAXCONF; ++c2)
@@ -2488,18 +2819,11 @@ __global__ __launch_bounds__(kBlock) void eloc_grad_kernel(EArgs a) {
     double s[3] = {0.0, 0.0, 0.0};
 #pragma unroll 1
     for (int c = 0; c < t.nconf_max; ++c) {
-        double aa[NM], xb[NM], ib[NM];
-        gather_conf<NM>(t, L, c, mo, aa);
-        gather_conf<NM>(t, L, c, bk, xb);
-        double lg, sg, tp;
-        int col, col2;
-        lane_gj<NM>(L, t.nsig_max, aa, xb, lg, sg, tp, col);
-        gather_conf<NM>(t, L, c, mo, aa);
-#pragma unroll
-        for (int j = 0; j < NM; ++j) ib[j] = (j == L.myrow) ? 1.0 : 0.0;
-        lane_gj<NM>(L, t.nsig_max, aa, ib, lg, sg, tp, col2);
-        double inv[NM], zz[NM];
-        inverse_columns<NM>(L, t.nsig_max, col, xb, ib, inv, zz);
+        double lg, sg, inv[NM], zz[NM];
+        conf_inverse<NM>(t, L, c, mo, own_ex, lg, sg, inv);
+        const int nc = L.spin == 0 ? t.nconf_up : t.nconf_dn, cc = c < nc ? c : nc - 1;
+        const QMC_CONST int* cf = L.spin == 0 ? t.conf_up + cc * t.nup : t.conf_dn + cc * t.ndown;
+        inverse_b_inverse<NM>(t, L, inv, brow, ycol, [&](int k) { return t.identity_conf ? k : (int)cf[k]; }, zz);
         double rc = 0.0, oc = 0.0;
 #pragma unroll
         for (int c2 = 0; c2 < QMC_MAXCONF; ++c2)

@@ -6,17 +6,6 @@
 
 namespace qmc {
 
-// register-array bucket for max(nmo, nup)
-inline int nm_bucket(const Tables& t) {
-    const int need = t.nmo > t.nup ? t.nmo : t.nup;
-    if (need <= 2) return 2;
-    if (need <= 4) return 4;
-    if (need <= 8) return 8;
-    if (need <= 16) return 16;
-    if (need <= 24) return 24;
-    return -1;
-}
-
 // register-array bound of the psi / local-energy / sweep kernels: exact up to
 // 8 occupied orbitals per spin, so the lane elimination and the MO rows carry
 // no idle columns, then 12, 16, 24
@@ -72,16 +61,18 @@ int launch_sweep_batch_exc(const SJob* jobs, int njobs, int nwaves, int bucket, 
 template <int RAD>
 int launch_wf_batch_exc(const WJob* jobs, int njobs, int nwaves, int bucket, size_t lds, int precision, int mode,
                         hipStream_t s);
-// HMC / drift: MC = 1 for single-configuration plans, QMC_MAXCONF otherwise
+// HMC / drift: MC = 1 for ground-state determinants, QMC_MAXCONF otherwise
 template <int RAD, int MC> int launch_hmc_f32(const HArgs& a, hipStream_t s);
 template <int RAD, int MC> int launch_hmc_f64(const HArgs& a, hipStream_t s);
-// batched launches: jobs (device) sorted into one register bucket, nwaves in total
-template <int RAD> int launch_sweep_batch_f32(const SJob* jobs, int njobs, int nwaves, int bucket, hipStream_t s);
-template <int RAD> int launch_sweep_batch_f64(const SJob* jobs, int njobs, int nwaves, int bucket, hipStream_t s);
+// batched launches: jobs (device) of one register bucket and configuration kind, nwaves in total
 template <int RAD>
-int launch_wf_batch_f32(const WJob* jobs, int njobs, int nwaves, int bucket, int mode, hipStream_t s);
+int launch_sweep_batch_f32(const SJob* jobs, int njobs, int nwaves, int bucket, bool multi, hipStream_t s);
 template <int RAD>
-int launch_wf_batch_f64(const WJob* jobs, int njobs, int nwaves, int bucket, int mode, hipStream_t s);
+int launch_sweep_batch_f64(const SJob* jobs, int njobs, int nwaves, int bucket, bool multi, hipStream_t s);
+template <int RAD>
+int launch_wf_batch_f32(const WJob* jobs, int njobs, int nwaves, int bucket, bool multi, int mode, hipStream_t s);
+template <int RAD>
+int launch_wf_batch_f64(const WJob* jobs, int njobs, int nwaves, int bucket, bool multi, int mode, hipStream_t s);
 
 inline dim3 grid_for_waves(int nwaves) { return dim3((unsigned)((nwaves + (kBlock / 64) - 1) / (kBlock / 64))); }
 
@@ -104,6 +95,7 @@ struct SpecEntry {
     uint64_t signature;  // layout_signature of the layout
     int nm;              // register bucket the kernels were built for
     int max_rows;        // lanes of real walkers per wavefront (G Ne) the sweeps' matrix tiles cover
+    bool multi;          // built for several configurations (else for the ground-state determinant)
     const char* name;
     int (*sweep)(const SArgs& a, int precision, hipStream_t s);
     int (*sweep_batch)(const SJob* jobs, int njobs, int nwaves, int precision, hipStream_t s);
@@ -112,9 +104,9 @@ struct SpecEntry {
     int (*hmc)(const HArgs& a, int precision, hipStream_t s);  // mixed HMC / drift
 };
 
-// the generated layout with this signature and bucket whose kernels cover
-// `rows` lanes of real walkers per wavefront, or nullptr
-const SpecEntry* find_spec(uint64_t signature, int nm, int rows);
+// the generated layout with this signature, bucket and configuration kind
+// whose kernels cover `rows` lanes of real walkers per wavefront, or nullptr
+const SpecEntry* find_spec(uint64_t signature, int nm, int rows, bool multi);
 
 #define QMC_BY_RAD(fn, rad, ...) ((rad) == QMC_RADIAL_STO ? fn<QMC_RADIAL_STO>(__VA_ARGS__) : fn<QMC_RADIAL_GTO_PURE>(__VA_ARGS__))
 

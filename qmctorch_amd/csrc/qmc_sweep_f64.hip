@@ -9,7 +9,10 @@ namespace qmc {
 
 template <int NM, int RAD>
 static void go(const SArgs& a, hipStream_t s) {
-    hipLaunchKernelGGL((sweep_kernel<double, NM, RAD>), grid_for(a.t, a.nw), dim3(kBlock), 0, s, a);
+    if (a.t.identity_conf)
+        hipLaunchKernelGGL((sweep_kernel<double, NM, RAD, false>), grid_for(a.t, a.nw), dim3(kBlock), 0, s, a);
+    else
+        hipLaunchKernelGGL((sweep_kernel<double, NM, RAD, true>), grid_for(a.t, a.nw), dim3(kBlock), 0, s, a);
 }
 
 template <int RAD>

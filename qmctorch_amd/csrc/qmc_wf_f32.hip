@@ -11,7 +11,10 @@ template <int NM, int RAD>
 static void go(const KArgs& a, int mode, hipStream_t s) {
     // psi only: local energies are evaluated by the FP64 kernels in every precision
     (void)mode;
-    hipLaunchKernelGGL((wf_kernel<float, NM, RAD, false>), grid_for(a.t, a.nw), dim3(kBlock), 0, s, a);
+    if (a.t.identity_conf)
+        hipLaunchKernelGGL((wf_kernel<float, NM, RAD, false, false>), grid_for(a.t, a.nw), dim3(kBlock), 0, s, a);
+    else
+        hipLaunchKernelGGL((wf_kernel<float, NM, RAD, false, true>), grid_for(a.t, a.nw), dim3(kBlock), 0, s, a);
 }
 
 template <int RAD>

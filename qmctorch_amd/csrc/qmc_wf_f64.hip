@@ -10,10 +10,15 @@ namespace qmc {
 template <int NM, int RAD>
 static void go(const KArgs& a, int mode, hipStream_t s) {
     const dim3 g = grid_for(a.t, a.nw);
-    if (mode == QMC_EVAL_ELOC)
-        hipLaunchKernelGGL((wf_kernel<double, NM, RAD, true>), g, dim3(kBlock), 0, s, a);
+    const bool multi = !a.t.identity_conf;
+    if (mode == QMC_EVAL_ELOC && multi)
+        hipLaunchKernelGGL((wf_kernel<double, NM, RAD, true, true>), g, dim3(kBlock), 0, s, a);
+    else if (mode == QMC_EVAL_ELOC)
+        hipLaunchKernelGGL((wf_kernel<double, NM, RAD, true, false>), g, dim3(kBlock), 0, s, a);
+    else if (multi)
+        hipLaunchKernelGGL((wf_kernel<double, NM, RAD, false, true>), g, dim3(kBlock), 0, s, a);
     else
-        hipLaunchKernelGGL((wf_kernel<double, NM, RAD, false>), g, dim3(kBlock), 0, s, a);
+        hipLaunchKernelGGL((wf_kernel<double, NM, RAD, false, false>), g, dim3(kBlock), 0, s, a);
 }
 
 template <int RAD>

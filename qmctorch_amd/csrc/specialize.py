@@ -144,6 +144,7 @@ struct AoSpec {
 
 constexpr int kNM = %(nm)d;
 constexpr int kRAD = %(rad)d;
+constexpr bool kMulti = %(multi)s;  // several configurations, or the ground-state determinant only
 
 }  // namespace
 '''
@@ -168,7 +169,7 @@ HMC = '''
 constexpr int kMC = %(mc)d;
 
 int spec_%(name)s_hmc(const HArgs& a, int prec, hipStream_t s) {
-    if (prec != QMC_PREC_MIXED || a.t.nconf_max > kMC) return -1;
+    if (prec != QMC_PREC_MIXED) return -1;
     hipLaunchKernelGGL((hmc_kernel<float, kNM, kRAD, kMC, AoSpec>), grid_for(a.t, a.nw), dim3(kBlock), 0, s, a);
     return 0;
 }
@@ -179,13 +180,13 @@ int spec_%(name)s_hmc(const HArgs& a, int prec, hipStream_t s) {
 ELOC = '''
 int spec_%(name)s_wf(const KArgs& a, int prec, int mode, hipStream_t s) {
     if (prec != QMC_PREC_FP64 || mode != QMC_EVAL_ELOC) return -1;
-    hipLaunchKernelGGL((wf_kernel<double, kNM, kRAD, true, AoSpec>), grid_for(a.t, a.nw), dim3(kBlock), 0, s, a);
+    hipLaunchKernelGGL((wf_kernel<double, kNM, kRAD, true, kMulti, AoSpec>), grid_for(a.t, a.nw), dim3(kBlock), 0, s, a);
     return 0;
 }
 
 int spec_%(name)s_wf_batch(const WJob* jobs, int njobs, int nwaves, int prec, int mode, hipStream_t s) {
     if (prec != QMC_PREC_FP64 || mode != QMC_EVAL_ELOC) return -1;
-    hipLaunchKernelGGL((wf_batch_kernel<double, kNM, kRAD, true, AoSpec>), grid_for_waves(nwaves), dim3(kBlock), 0,
+    hipLaunchKernelGGL((wf_batch_kernel<double, kNM, kRAD, true, kMulti, AoSpec>), grid_for_waves(nwaves), dim3(kBlock), 0,
                        s, jobs, njobs, nwaves);
     return 0;
 }
@@ -201,11 +202,11 @@ namespace qmc {
 %(decls)s
 // host-side table (the device pass of this unit needs none of it)
 #if !defined(__HIP_DEVICE_COMPILE__)
-const SpecEntry* find_spec(uint64_t signature, int nm, int rows) {
+const SpecEntry* find_spec(uint64_t signature, int nm, int rows, bool multi) {
     static const SpecEntry table[] = {
-%(rows)s        {0, 0, 0, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr}};
+%(rows)s        {0, 0, 0, false, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr}};
     for (const SpecEntry* e = table; e->name; ++e)
-        if (e->signature == signature && e->nm == nm && rows <= e->max_rows) return e;
+        if (e->signature == signature && e->nm == nm && rows <= e->max_rows && multi == e->multi) return e;
     return nullptr;
 }
 #endif
@@ -223,15 +224,15 @@ def sweep_launch(nentry: int, nm: int) -> Tuple[str, str]:
     staged in LDS when they fit (the two must run the same arithmetic, so that
     a walker's chain is the same alone and in a batch), else both without."""
     if nentry * nm * 4 <= WLDS_MAX_BYTES:
-        single = ("    hipLaunchKernelGGL((sweep_kernel_wlds<float, kNM, kRAD, AoSpec>), grid_for(a.t, a.nw), dim3(kBlock),\n"
+        single = ("    hipLaunchKernelGGL((sweep_kernel_wlds<float, kNM, kRAD, kMulti, AoSpec>), grid_for(a.t, a.nw), dim3(kBlock),\n"
                   "                       (size_t)a.t.nentry * kNM * sizeof(float), s, a);")
-        batch = ("    hipLaunchKernelGGL((sweep_batch_kernel_wlds<float, kNM, kRAD, AoSpec>), grid_for_waves(nwaves),\n"
+        batch = ("    hipLaunchKernelGGL((sweep_batch_kernel_wlds<float, kNM, kRAD, kMulti, AoSpec>), grid_for_waves(nwaves),\n"
                  "                       dim3(kBlock), (kBlock / 64) * %d * sizeof(float), s, jobs, njobs, nwaves, %d);"
                  % (nentry * nm, nentry * nm))
         return single, batch
-    single = ("    hipLaunchKernelGGL((sweep_kernel<float, kNM, kRAD, AoSpec>), grid_for(a.t, a.nw), dim3(kBlock), 0, s, "
+    single = ("    hipLaunchKernelGGL((sweep_kernel<float, kNM, kRAD, kMulti, AoSpec>), grid_for(a.t, a.nw), dim3(kBlock), 0, s, "
               "a);")
-    batch = ("    hipLaunchKernelGGL((sweep_batch_kernel<float, kNM, kRAD, AoSpec>), grid_for_waves(nwaves), dim3(kBlock), "
+    batch = ("    hipLaunchKernelGGL((sweep_batch_kernel<float, kNM, kRAD, kMulti, AoSpec>), grid_for_waves(nwaves), dim3(kBlock), "
              "0, s,\n                       jobs, njobs, nwaves);")
     return single, batch
 
@@ -241,7 +242,7 @@ def unit_sources(name: str, tab, nm: int, mc: int = 1) -> Dict[str, str]:
     in parallel.  mc bounds the unique configurations per spin of the HMC
     instance (1, or QMC_MAXCONF)."""
     head = ROW % dict(name=name, ngroup=len(tab.grp_atom), nentry=len(tab.gao_mu), nm=nm, rad=int(tab.radial),
-                      rowblocks=row_blocks(tab), body=row_source(tab))
+                      rowblocks=row_blocks(tab), body=row_source(tab), multi="true" if mc > 1 else "false")
     single, batch = sweep_launch(len(tab.gao_mu), nm)
     sweep = SWEEP % dict(name=name, launch=single, launch_batch=batch)
     return {"qmc_spec_%s_sweep.hip" % name: head + sweep,
@@ -251,15 +252,16 @@ def unit_sources(name: str, tab, nm: int, mc: int = 1) -> Dict[str, str]:
 
 def registry_source(layouts) -> str:
     decls, rows = "", ""
-    for name, tab, nm, _ in layouts:
+    for name, tab, nm, mc in layouts:
         decls += ("int spec_%(n)s_sweep(const SArgs&, int, hipStream_t);\n"
                   "int spec_%(n)s_sweep_batch(const SJob*, int, int, int, hipStream_t);\n"
                   "int spec_%(n)s_wf(const KArgs&, int, int, hipStream_t);\n"
                   "int spec_%(n)s_wf_batch(const WJob*, int, int, int, int, hipStream_t);\n"
                   "int spec_%(n)s_hmc(const HArgs&, int, hipStream_t);\n" % dict(n=name))
-        rows += ("        {0x%016xull, %d, %d, \"%s\", &spec_%s_sweep, &spec_%s_sweep_batch, &spec_%s_wf, "
-                 "&spec_%s_wf_batch, &spec_%s_hmc},\n" % (layout_signature(tab), nm, 16 * row_blocks(tab), name,
-                                                           name, name, name, name, name))
+        rows += ("        {0x%016xull, %d, %d, %s, \"%s\", &spec_%s_sweep, &spec_%s_sweep_batch, &spec_%s_wf, "
+                 "&spec_%s_wf_batch, &spec_%s_hmc},\n" % (layout_signature(tab), nm, 16 * row_blocks(tab),
+                                                           "true" if mc > 1 else "false", name, name, name, name, name,
+                                                           name))
     return REGISTRY % dict(decls=decls, rows=rows)
 
 

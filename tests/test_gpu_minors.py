@@ -1,0 +1,65 @@
+"""Small-matrix (minors) kernels on the device at every size and spin split.
+
+Chains of n hydrogen atoms with one unpaired electron: the up block is
+(n + 1) / 2 columns and the down block one fewer, so each size from 2 to 7
+runs with a group completed by unit rows, and 8 is the first size of the
+eliminations.  psi, the local energy and the gradient against the float64
+oracle; log|psi| far from every nucleus, where products of orbital values
+leave the double range, against the sum of the single-electron decays.
+"""
+import numpy as np
+import pytest
+import torch
+
+from qmctorch_amd.scf import Molecule
+from tests import helpers
+
+pytestmark = pytest.mark.gpu
+
+
+def _chain(n):
+    atoms = "; ".join("H %.3f %.3f %.3f" % (0.3 * (k % 2), 0.2 * (k % 3), 1.6 * k) for k in range(n))
+    return Molecule(atoms, basis="cc-pvdz", unit="bohr", spin=n % 2, mo_coeffs="random", name="h%d" % n)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 7, 9, 11, 13, 14, 15])
+def test_every_block_size(n):
+    print("case minors H%d" % n, flush=True)
+    mol = _chain(n)
+    wf, orc = helpers.make_pair(mol, w_ee=None if n == 1 else 1.0, w_en=1.0)
+    pos = helpers.positions(mol, 67, seed=n, sigma=1.0)
+    x = pos.cuda()
+    psi, psi_o = wf(x).detach().cpu().view(-1), orc(pos).detach().view(-1)
+    # rounding of the orbitals (1e-15) times the condition of the blocks
+    assert float(((psi - psi_o).abs() / psi_o.abs()).max()) < 1e-9
+    e, e_o = wf.local_energy(x).cpu().view(-1), orc.local_energy(pos).detach().view(-1)
+    assert float(((e - e_o).abs() / e_o.abs().clamp(min=1.0)).max()) < 1e-8
+    p = pos.clone().requires_grad_()
+    g_o = torch.autograd.grad(orc(p).sum(), p)[0]
+    g = wf.gradients_jacobi(x).cpu()
+    assert float((g - g_o).abs().max() / g_o.abs().max()) < 1e-9
+
+
+@pytest.mark.parametrize("n", [5, 9, 13])
+def test_rows_far_from_the_nuclei(n):
+    """Every electron is moved out so far that its orbitals are below 1e-80: the
+    block's products underflow, its logarithm does not."""
+    print("case minors far H%d" % n, flush=True)
+    mol = _chain(n)
+    wf, orc = helpers.make_pair(mol, w_ee=1.0, w_en=1.0)
+    rng = np.random.default_rng(n)
+    d = rng.standard_normal((33, n, 3))
+    d *= 40.0 / np.linalg.norm(d, axis=2, keepdims=True)
+    pos = torch.as_tensor((d + np.asarray(mol.atom_coords)[None]).reshape(33, 3 * n))
+    la, sg = wf.log_psi(pos.cuda())
+    mo = orc.mo(orc.ao(pos)).detach()
+    scale = mo.abs().amax(-1, keepdim=True)
+    rows = (mo / scale)[..., :wf.highest_occ_mo]
+    su, lu = torch.linalg.slogdet(rows[:, :mol.nup, :mol.nup])
+    sd, ld = torch.linalg.slogdet(rows[:, mol.nup:, :mol.ndown])
+    ref = lu + ld + scale.log().sum((1, 2)) + orc.jastrow(pos).detach().view(-1).log()
+    print("  log|psi| from %.0f to %.0f, largest difference %.1e" % (ref.min(), ref.max(),
+                                                                   (la.cpu() - ref).abs().max()), flush=True)
+    assert float(ref.max()) < -745.0  # below the smallest double
+    # exponents of 200 per electron rounded to 1e-16, times the blocks' condition
+    assert float((la.cpu() - ref).abs().max()) < 1e-9 and torch.equal(sg.cpu(), su * sd)
