@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <stdexcept>
 #include <string>
@@ -207,6 +208,86 @@ bool excitation_table(const int32_t* conf, int nconf, int n, std::vector<int32_t
     return true;
 }
 
+// Shell records and coefficients of the table-driven AO row (ao_shells): the
+// entries of a group in order, consecutive ones merged into p shells (x, y, z
+// with equal coefficients) and d shells (xx, xy, xz, yy, yz, zz, the mixed ones
+// at one ratio to the others) with one STO r power, else one by one; a group
+// entry whose primitives have several r powers gives one record per primitive.
+struct ShellRecords {
+    std::vector<int32_t> rec;
+    std::vector<double> K;
+    int end = -1;  // the entry after the last record's shells
+    void add(int atom, int np, int p0, int entry, int word, const double* k, double ratio) {
+        const size_t n = rec.size() / kRecWords;
+        int32_t* last = n ? &rec[(n - 1) * kRecWords] : nullptr;
+        if (last && last[0] == atom && (last[7] & 0xFF) == np && (last[7] >> 8) < kRecShells && last[1] == p0 &&
+            end == entry) {
+            last[4 + (last[7] >> 8)] = word;
+            last[7] += 1 << 8;
+        } else {
+            rec.insert(rec.end(), {atom, p0, (int32_t)K.size(), entry, word, 0, 0, np | 1 << 8});
+        }
+        end = entry + ((word & 15) == kShellP ? 3 : ((word & 15) == kShellD ? 6 : 1));
+        K.insert(K.end(), k, k + np);
+        K.push_back(ratio);
+    }
+};
+
+ShellRecords shell_records(const QmcSystemDesc* d) {
+    ShellRecords out;
+    const bool sto = d->radial_type == QMC_RADIAL_STO;  // Gaussians have no r power
+    const int kP[3] = {0x001, 0x010, 0x100}, kD[6] = {0x002, 0x011, 0x101, 0x020, 0x110, 0x200};
+    for (int g = 0; g < d->ngroup; ++g) {
+        const int np = d->grp_nprim[g], p0 = d->grp_prim0[g], i1 = d->grp_ao0[g] + d->grp_nao[g];
+        auto K = [&](int i) { return d->gao_K + (size_t)i * QMC_MAXP; };
+        auto N = [&](int i) { return d->gao_n + (size_t)i * QMC_MAXP; };
+        auto one_power = [&](int i) {
+            for (int q = 1; sto && q < np; ++q)
+                if (N(i)[q] != N(i)[0]) return false;
+            return true;
+        };
+        auto matches = [&](int i, const int* k, int n) {  // powers k and one r power over n entries from i
+            if (i + n > i1) return false;
+            for (int j = 0; j < n; ++j)
+                if (d->gao_k[i + j] != k[j] || !one_power(i + j) || (sto && N(i + j)[0] != N(i)[0]))
+                    return false;
+            return true;
+        };
+        auto scaled = [&](int i, int j, double f) {  // K(j) = f K(i) to rounding
+            for (int q = 0; q < np; ++q)
+                if (!(std::fabs(K(j)[q] - f * K(i)[q]) <= 8e-16 * std::fabs(K(j)[q]))) return false;
+            return true;
+        };
+        for (int i = d->grp_ao0[g]; i < i1;) {
+            const int power = sto ? (int)N(i)[0] << 16 : 0, k = d->gao_k[i];
+            if (matches(i, kP, 3) && scaled(i, i + 1, 1.0) && scaled(i, i + 2, 1.0)) {
+                out.add(d->grp_atom[g], np, p0, i, kShellP | power, K(i), 0.0);
+                i += 3;
+                continue;
+            }
+            if (matches(i, kD, 6) && K(i)[0] != 0.0) {
+                const double f = K(i + 1)[0] / K(i)[0];
+                if (scaled(i, i + 3, 1.0) && scaled(i, i + 5, 1.0) && scaled(i, i + 1, f) && scaled(i, i + 2, f) &&
+                    scaled(i, i + 4, f)) {
+                    out.add(d->grp_atom[g], np, p0, i, kShellD | power, K(i), f);
+                    i += 6;
+                    continue;
+                }
+            }
+            const int type = k == 0 ? kShellS : kShellOne;
+            const int word = type | (k & 15) << 4 | ((k >> 4) & 15) << 8 | ((k >> 8) & 15) << 12;
+            if (one_power(i)) {
+                out.add(d->grp_atom[g], np, p0, i, word | power, K(i), 0.0);
+            } else {
+                for (int q = 0; q < np; ++q)
+                    out.add(d->grp_atom[g], 1, p0 + q, i, word | (int)N(i)[q] << 16, K(i) + q, 0.0);
+            }
+            ++i;
+        }
+    }
+    return out;
+}
+
 // Entry points without the trace-trick path refuse plans that need it.
 int refuse_excitations(const QmcPlan* plan) {
     if (plan && plan->t.exc_mode)
@@ -306,13 +387,16 @@ int qmc_plan_create(const QmcSystemDesc* d, QmcPlan** out) {
         t.gao_mu = (decltype(t.gao_mu))p->upload(d->gao_mu, d->nentry);
         t.gao_k = (decltype(t.gao_k))p->upload(d->gao_k, d->nentry);
         t.gao_K = (decltype(t.gao_K))p->upload(d->gao_K, (size_t)d->nentry * QMC_MAXP);
-        {
-            std::vector<float> kf((size_t)d->nentry * QMC_MAXP);
-            for (size_t i = 0; i < kf.size(); ++i) kf[i] = (float)d->gao_K[i];
-            t.gao_Kf = (decltype(t.gao_Kf))p->upload(kf.data(), kf.size());
-        }
         t.gao_n = (decltype(t.gao_n))p->upload(d->gao_n, (size_t)d->nentry * QMC_MAXP);
         t.gao_src = (decltype(t.gao_src))p->upload(d->gao_src, (size_t)d->nentry * QMC_MAXP);
+        {
+            const ShellRecords r = shell_records(d);
+            std::vector<float> kf(r.K.begin(), r.K.end());
+            t.nrec = (int)(r.rec.size() / kRecWords);
+            t.rec = (decltype(t.rec))p->upload(r.rec.data(), r.rec.size());
+            t.rec_K = (decltype(t.rec_K))p->upload(r.K.data(), r.K.size());
+            t.rec_Kf = (decltype(t.rec_Kf))p->upload(kf.data(), kf.size());
+        }
         t.atom_z = (decltype(t.atom_z))p->upload(d->atom_z, d->natom);
         t.jas_atoms = (decltype(t.jas_atoms))p->upload(d->jastrow_atoms, (size_t)d->natom * 3);
         t.conf_up = (decltype(t.conf_up))p->upload(d->conf_up, (size_t)d->nconf_up * d->nup);

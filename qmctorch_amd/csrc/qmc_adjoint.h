@@ -205,13 +205,13 @@ __device__ __forceinline__ void logpsi_adjoint_reduce(const GRedArgs& a, const W
 #pragma unroll
     for (int m = 0; m < NM; ++m) mo[m] = 0.0;
     {
-        auto sink = [&](int, int mu, double val, double, double, double, double) {
-            const QMC_CONST double* wr = (const QMC_CONST double*)W + (size_t)mu * t.nmo;
+        auto sink = [&](int i, int, double val, double, double, double, double) {
+            const QMC_CONST double* wr = (const QMC_CONST double*)W + (size_t)t.gao_mu[i] * t.nmo;
 #pragma unroll
             for (int m = 0; m < NM; ++m)
                 if (m < t.nmo) mo[m] += val * wr[m];
         };
-        ao_row<double, RAD, false>(t, a.p, x, y, z, sink);
+        ao_shells<double, RAD, false>(t, a.p, x, y, z, sink);
     }
     double gam[NM];
     if constexpr (EXC) {
@@ -275,7 +275,7 @@ __device__ __forceinline__ void logpsi_adjoint_reduce(const GRedArgs& a, const W
         st.clear();
         wave_lds_sync();
         auto sink = [&](int i, int, double val, double, double, double, double) { st.put(i, v ? val : 0.0, 0.0); };
-        ao_row<double, RAD, false>(t, a.p, x, y, z, sink);
+        ao_shells<double, RAD, false>(t, a.p, x, y, z, sink);
         st.flush();
     }
     // exponents: per term slot (entry i, primitive q) the walker sum of
@@ -418,8 +418,8 @@ __device__ __forceinline__ void eloc_adjoint_reduce(const ERedArgs& a, const Wal
 #pragma unroll
     for (int m = 0; m < NM; ++m) mo[m] = gx[m] = gy[m] = gz[m] = lp[m] = 0.0;
     {
-        auto sink = [&](int, int mu, double ao, double ax, double ay, double az, double al) {
-            const QMC_CONST double* wr = (const QMC_CONST double*)W + (size_t)mu * t.nmo;
+        auto sink = [&](int i, int, double ao, double ax, double ay, double az, double al) {
+            const QMC_CONST double* wr = (const QMC_CONST double*)W + (size_t)t.gao_mu[i] * t.nmo;
 #pragma unroll
             for (int m = 0; m < NM; ++m) {
                 if (m < t.nmo) {
@@ -432,7 +432,7 @@ __device__ __forceinline__ void eloc_adjoint_reduce(const ERedArgs& a, const Wal
                 }
             }
         };
-        ao_row<double, RAD, true>(t, a.p, x, y, z, sink);
+        ao_shells<double, RAD, true>(t, a.p, x, y, z, sink);
     }
     double bk[NM];
 #pragma unroll
@@ -591,7 +591,7 @@ __device__ __forceinline__ void eloc_adjoint_reduce(const ERedArgs& a, const Wal
         auto sink = [&](int i, int, double ao, double ax, double ay, double az, double al) {
             st.put(i, v ? ao : 0.0, v ? -0.5 * (al + 2.0 * (g[0] * ax + g[1] * ay + g[2] * az) + l2 * ao) : 0.0);
         };
-        ao_row<double, RAD, true>(t, a.p, x, y, z, sink);
+        ao_shells<double, RAD, true>(t, a.p, x, y, z, sink);
         st.flush();
     }
     // Pade weights

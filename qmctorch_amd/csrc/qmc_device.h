@@ -45,7 +45,6 @@ struct Tables {
     const QMC_CONST int* gao_mu;
     const QMC_CONST int* gao_k;
     const QMC_CONST double* gao_K;
-    const QMC_CONST float* gao_Kf;
     const QMC_CONST double* gao_n;
     const QMC_CONST int* gao_src;
     const QMC_CONST double* atom_z;
@@ -60,6 +59,12 @@ struct Tables {
     // ao_ent[ao_ptr[mu] .. ao_ptr[mu + 1]), the exponent-term columns
     // (entry i, primitive q) -> i * QMC_MAXP + q of bas_exp index k are
     // exp_col[exp_ptr[k] .. exp_ptr[k + 1]), both ascending
+    // shell records of the table-driven AO row (ao_shells), kRecWords words each,
+    // and their contraction coefficients
+    int nrec;
+    const QMC_CONST int* rec;
+    const QMC_CONST double* rec_K;
+    const QMC_CONST float* rec_Kf;
     const QMC_CONST int* ao_ptr;
     const QMC_CONST int* ao_ent;
     const QMC_CONST int* exp_ptr;
@@ -154,17 +159,6 @@ __device__ __forceinline__ void cart_poly(T x, T y, T z, int kx, int ky, int kz,
 // AO that were split across groups are delivered separately (all consumers
 // are linear in the AO).  The primitive count of a group selects a fully
 // unrolled instance (no predicated slots).
-template <typename T>
-__device__ __forceinline__ const QMC_CONST T* coeff_table(const Tables& t);
-template <>
-__device__ __forceinline__ const QMC_CONST float* coeff_table<float>(const Tables& t) {
-    return t.gao_Kf;
-}
-template <>
-__device__ __forceinline__ const QMC_CONST double* coeff_table<double>(const Tables& t) {
-    return t.gao_K;
-}
-
 // exponents gathered in group-primitive order, in the evaluation precision
 template <typename T>
 __device__ __forceinline__ const T* group_exponents(const QmcParams& prm);
@@ -187,11 +181,6 @@ __device__ __forceinline__ void group_prims_from(const T* gexp, int p0, T r2, T 
         A[p] = a;
         E[p] = (RAD == QMC_RADIAL_GTO_PURE) ? fexp(-a * r2) : fexp(-a * r);
     }
-}
-
-template <typename T, int RAD, int NP>
-__device__ __forceinline__ void group_prims(const QmcParams& prm, int p0, T r2, T r, T (&E)[NP], T (&A)[NP]) {
-    group_prims_from<T, RAD, NP>(group_exponents<T>(prm), p0, r2, r, E, A);
 }
 
 // AO entry i (AO mu, Cartesian powers kx, ky, kz) of a group from its
@@ -251,90 +240,177 @@ __device__ __forceinline__ void ao_entry_with(KF kcoef, NF rpow, int i, int mu, 
     }
 }
 
-template <typename T, int RAD, bool DERIV, int NP, typename Sink>
-__device__ __forceinline__ void ao_entry(const Tables& t, int i, int mu, int kx, int ky, int kz, const T (&E)[NP],
-                                         const T (&A)[NP], T dx, T dy, T dz, T r2, T r, T ir, Sink& sink) {
-    const QMC_CONST T* Kp = coeff_table<T>(t) + (size_t)i * QMC_MAXP;
-    const QMC_CONST double* Np = t.gao_n + (size_t)i * QMC_MAXP;
-    ao_entry_with<T, RAD, DERIV, NP>([&](int p) { return Kp[p]; }, [&](int p) { return Np[p]; }, i, mu, kx, ky, kz,
-                                     E, A, dx, dy, dz, r2, r, ir, sink);
+// ----------------------------------------------- table-driven AO row by shells
+// The row of the kernels for any basis layout.  The plan describes it as
+// records of up to three shells that share their primitives:
+//   {atom, first exponent, first coefficient, first AO entry, shell word x 3,
+//    np | nk << 8},
+//   shell word: type | kx << 4 | ky << 8 | kz << 12 | r power << 16,
+// each shell with np + 1 coefficients (its contraction, then the d_xy / d_xx
+// normalisation ratio).  One scalar load fetches a record, one record ahead of
+// its use, and the loads it leads to (exponents, coefficients, W rows) are
+// issued together: walking the group and entry tables instead cost four
+// dependent scalar loads per group and three per entry, and every entry
+// selected its Cartesian powers at run time.  With the primitives' moments
+// m_j = sum_p K_p a_p^j e_p, e_p = exp(-a_p r^2) or exp(-a_p r), a shell's
+// radial part is
+//   value v, gradient  v grad Y + c Y r,  Laplacian  Y (A + L B) + v lap Y:
+//   GTO  v = m0, c = -2 m1, A = 4 r^2 m2 - 6 m1, B = -4 m1;
+//   STO  R = r^n:  v = R m0, c = R (n m0 / r^2 - m1 / r),
+//        A = R (n (n+1) m0 / r^2 - 2 (n+1) m1 / r + m2), B = 2 c
+// (L the total Cartesian power), shared by its 1, 3 or 6 entries.  Two waters
+// (20 electrons, 50 AOs, FP64), 2047 walkers x 50 steps: 1.411 -> 1.181 ms.
+constexpr int kRecWords = 8;
+constexpr int kRecShells = 3;  // shells per record at most
+enum ShellType { kShellS = 0, kShellP = 1, kShellD = 2, kShellOne = 3 };  // D: xx xy xz yy yz zz; One: one entry
+
+template <typename T>
+__device__ __forceinline__ const QMC_CONST T* record_coeffs(const Tables& t);
+template <>
+__device__ __forceinline__ const QMC_CONST float* record_coeffs<float>(const Tables& t) {
+    return t.rec_Kf;
+}
+template <>
+__device__ __forceinline__ const QMC_CONST double* record_coeffs<double>(const Tables& t) {
+    return t.rec_K;
 }
 
-template <typename T, int RAD, bool DERIV, int NP, typename Sink>
-__device__ __forceinline__ void ao_group(const Tables& t, int g, const QmcParams& prm, T dx, T dy, T dz, T r2, T r,
-                                         T ir, Sink& sink) {
+// moments m[shell][j] (j = 0, with DERIV also 1 and 2) of a record's NP primitives
+template <typename T, int RAD, bool DERIV, int NP>
+__device__ __forceinline__ void record_moments(const T* gexp, const QMC_CONST T* K, int nk, T r2, T r,
+                                               T (&m)[kRecShells][3]) {
     T E[NP], A[NP];
-    group_prims<T, RAD, NP>(prm, t.grp_prim0[g], r2, r, E, A);
-    const int i0 = t.grp_ao0[g], i1 = i0 + t.grp_nao[g];
-    for (int i = i0; i < i1; ++i) {
-        const int kk = t.gao_k[i];
-        ao_entry<T, RAD, DERIV, NP>(t, i, t.gao_mu[i], kk & 15, (kk >> 4) & 15, (kk >> 8) & 15, E, A, dx, dy, dz, r2,
-                                    r, ir, sink);
+    group_prims_from<T, RAD, NP>(gexp, 0, r2, r, E, A);
+#pragma unroll
+    for (int q = 0; q < kRecShells; ++q) {
+        if (q < nk) {
+            T m0 = 0, m1 = 0, m2 = 0;
+#pragma unroll
+            for (int p = 0; p < NP; ++p) {
+                const T ke = K[q * (NP + 1) + p] * E[p];
+                m0 += ke;
+                if (DERIV) {
+                    m1 += ke * A[p];
+                    m2 += ke * A[p] * A[p];
+                }
+            }
+            m[q][0] = m0;
+            m[q][1] = m1;
+            m[q][2] = m2;
+        }
     }
 }
 
-// TIGHT: groups flagged in grp_tight are evaluated in FP64 whatever T is (the
-// mixed-precision local energy: tight core primitives cancel in lap AO near the
-// nucleus, which FP32 cannot resolve).
-template <typename T, int RAD, bool DERIV, bool TIGHT = false, typename Sink>
-__device__ __forceinline__ void ao_row(const Tables& t, const QmcParams& prm, double ex, double ey, double ez,
-                                       Sink&& sink) {
-    const double* atom_xyz = prm.atom_coords;
+template <typename T, int RAD, bool DERIV, typename Sink>
+__device__ __forceinline__ void ao_shells(const Tables& t, const QmcParams& prm, double ex, double ey, double ez,
+                                          Sink&& sink) {
+    typedef int int8v __attribute__((ext_vector_type(8)));
+    const QMC_CONST int8v* rec = (const QMC_CONST int8v*)t.rec;
     int cur_atom = -1;
-    double dxd = 0, dyd = 0, dzd = 0, r2d = 0, rd = 0, ird = 0;
-    T dx = 0, dy = 0, dz = 0, r2 = 0, r = 0, ir = 0;
-    for (int g = 0; g < t.ngroup; ++g) {
-        const int at = t.grp_atom[g];
+    T x = 0, y = 0, z = 0, r2 = 0, r = 0, ir = 0;
+    int8v next = rec[0];
+    for (int k = 0; k < t.nrec; ++k) {
+        const int8v w = next;
+        next = rec[k + 1 < t.nrec ? k + 1 : k];
+        const int at = w[0], np = w[7] & 0xFF, nk = w[7] >> 8;
         if (at != cur_atom) {
             cur_atom = at;
-            dxd = ex - ldc(atom_xyz, 3 * at + 0);
-            dyd = ey - ldc(atom_xyz, 3 * at + 1);
-            dzd = ez - ldc(atom_xyz, 3 * at + 2);
-            dx = (T)dxd;
-            dy = (T)dyd;
-            dz = (T)dzd;
-            r2 = dx * dx + dy * dy + dz * dz;
+            x = (T)(ex - ldc(prm.atom_coords, 3 * at + 0));
+            y = (T)(ey - ldc(prm.atom_coords, 3 * at + 1));
+            z = (T)(ez - ldc(prm.atom_coords, 3 * at + 2));
+            r2 = x * x + y * y + z * z;
             if (RAD == QMC_RADIAL_STO) {
                 r = fsqrt(r2);
                 ir = T(1) / r;
             }
-            if (TIGHT) {
-                r2d = dxd * dxd + dyd * dyd + dzd * dzd;
-                if (RAD == QMC_RADIAL_STO) {
-                    rd = sqrt(r2d);
-                    ird = 1.0 / rd;
+        }
+        const T* gexp = group_exponents<T>(prm) + w[1];
+        const QMC_CONST T* K = record_coeffs<T>(t) + w[2];
+        T m[kRecShells][3];
+        switch (np) {
+#define QMC_REC_CASE(N)                                              \
+    case N:                                                          \
+        record_moments<T, RAD, DERIV, N>(gexp, K, nk, r2, r, m);     \
+        break;
+            QMC_REC_CASE(1) QMC_REC_CASE(2) QMC_REC_CASE(3) QMC_REC_CASE(4) QMC_REC_CASE(5) QMC_REC_CASE(6)
+            QMC_REC_CASE(7) QMC_REC_CASE(8) QMC_REC_CASE(9) QMC_REC_CASE(10) QMC_REC_CASE(11) QMC_REC_CASE(12)
+#undef QMC_REC_CASE
+            default: break;
+        }
+        int i = w[3];
+#pragma unroll 1
+        for (int q = 0; q < nk; ++q) {
+            const int word = q == 0 ? w[4] : (q == 1 ? w[5] : w[6]);
+            const int type = word & 15;
+            const T m0 = q == 0 ? m[0][0] : (q == 1 ? m[1][0] : m[2][0]);
+            T v = m0, c = 0, A = 0, B = 0;
+            if (RAD == QMC_RADIAL_GTO_PURE) {
+                if (DERIV) {
+                    const T m1 = q == 0 ? m[0][1] : (q == 1 ? m[1][1] : m[2][1]);
+                    const T m2 = q == 0 ? m[0][2] : (q == 1 ? m[1][2] : m[2][2]);
+                    c = T(-2) * m1;
+                    A = T(4) * r2 * m2 - T(6) * m1;
+                    B = T(-4) * m1;
+                }
+            } else {
+                const int n = word >> 16;
+                const T R = ipow(r, n);
+                v = R * m0;
+                if (DERIV) {
+                    const T m1 = q == 0 ? m[0][1] : (q == 1 ? m[1][1] : m[2][1]);
+                    const T m2 = q == 0 ? m[0][2] : (q == 1 ? m[1][2] : m[2][2]);
+                    const T fn = T(n);
+                    c = R * (fn * m0 * ir * ir - m1 * ir);
+                    A = R * (fn * (fn + T(1)) * m0 * ir * ir - T(2) * (fn + T(1)) * m1 * ir + m2);
+                    B = T(2) * c;
                 }
             }
-        }
-        const bool tight = TIGHT && t.grp_tight != nullptr && t.grp_tight[g] != 0;
-        switch (t.grp_nprim[g]) {
-#define QMC_AO_CASE(K)                                                                               \
-    case K:                                                                                          \
-        if (tight)                                                                                   \
-            ao_group<double, RAD, DERIV, K>(t, g, prm, dxd, dyd, dzd, r2d, rd, ird, sink);           \
-        else                                                                                         \
-            ao_group<T, RAD, DERIV, K>(t, g, prm, dx, dy, dz, r2, r, ir, sink);                      \
-        break;
-            QMC_AO_CASE(1) QMC_AO_CASE(2) QMC_AO_CASE(3) QMC_AO_CASE(4) QMC_AO_CASE(5) QMC_AO_CASE(6)
-            QMC_AO_CASE(7) QMC_AO_CASE(8) QMC_AO_CASE(9) QMC_AO_CASE(10) QMC_AO_CASE(11) QMC_AO_CASE(12)
-#undef QMC_AO_CASE
-            default: break;
+            if (type == kShellS) {
+                sink(i, 0, v, c * x, c * y, c * z, A);
+                i += 1;
+            } else if (type == kShellP) {
+                const T l = A + B, cx = c * x, cy = c * y, cz = c * z;
+                sink(i + 0, 0, v * x, v + cx * x, cx * y, cx * z, l * x);
+                sink(i + 1, 0, v * y, cy * x, v + cy * y, cy * z, l * y);
+                sink(i + 2, 0, v * z, cz * x, cz * y, v + cz * z, l * z);
+                i += 3;
+            } else if (type == kShellD) {
+                const T f = K[q * (np + 1) + np];  // normalisation of xy relative to xx
+                const T l = A + T(2) * B, vf = v * f, cf = c * f, lf = l * f;
+                const T xx = x * x, xy = x * y, xz = x * z, yy = y * y, yz = y * z, zz = z * z;
+                const T v2 = v + v;
+                sink(i + 0, 0, v * xx, x * (v2 + c * xx), c * xx * y, c * xx * z, l * xx + v2);
+                sink(i + 1, 0, vf * xy, y * (vf + cf * xx), x * (vf + cf * yy), cf * xy * z, lf * xy);
+                sink(i + 2, 0, vf * xz, z * (vf + cf * xx), cf * xz * y, x * (vf + cf * zz), lf * xz);
+                sink(i + 3, 0, v * yy, c * yy * x, y * (v2 + c * yy), c * yy * z, l * yy + v2);
+                sink(i + 4, 0, vf * yz, cf * yz * x, z * (vf + cf * yy), y * (vf + cf * zz), lf * yz);
+                sink(i + 5, 0, v * zz, c * zz * x, c * zz * y, z * (v2 + c * zz), l * zz + v2);
+                i += 6;
+            } else {
+                const int kx = (word >> 4) & 15, ky = (word >> 8) & 15, kz = (word >> 12) & 15;
+                T Y, Yx = 0, Yy = 0, Yz = 0, Yl = 0;
+                cart_poly<T, DERIV>(x, y, z, kx, ky, kz, Y, Yx, Yy, Yz, Yl);
+                const T cY = c * Y;
+                sink(i, 0, v * Y, v * Yx + cY * x, v * Yy + cY * y, v * Yz + cY * z,
+                     Y * (A + T(kx + ky + kz) * B) + v * Yl);
+                i += 1;
+            }
         }
     }
 }
 
-// AO evaluation policies of the kernels: AoGeneric walks the group tables
+// AO evaluation policies of the kernels: AoGeneric walks the shell records
 // above; a generated policy (qmc_spec_*.hip) walks one basis layout with every
 // group, entry, primitive offset and Cartesian power a compile-time constant,
-// built from the same atom_geo / group_prims / ao_entry pieces in the same
-// order, so both give the same values.
+// built from the atom_geo / group_prims / ao_entry pieces above in the same
+// order of entries, so both give the same values up to rounding.
 struct AoGeneric {
     static constexpr int kEntries = 0;    // AO entries of the row: known at run time only
     static constexpr int kRowBlocks = 4;  // 16-lane row blocks of the MFMA contraction: all
     template <typename T, int RAD, bool DERIV, bool TIGHT, typename Sink>
     static __device__ __forceinline__ void row(const Tables& t, const QmcParams& prm, double ex, double ey, double ez,
                                                Sink&& sink) {
-        ao_row<T, RAD, DERIV, TIGHT>(t, prm, ex, ey, ez, sink);
+        ao_shells<T, RAD, DERIV>(t, prm, ex, ey, ez, sink);
     }
 };
 

@@ -2289,8 +2289,9 @@ __global__ __launch_bounds__(kBlock) void ao_kernel(AArgs a) {
     double* ao = a.ao;
     double* dao = a.dao;
     double* d2ao = a.d2ao;
-    auto sink = [&](int, int mu, double val, double ax, double ay, double az, double al) {
+    auto sink = [&](int i, int, double val, double ax, double ay, double az, double al) {
         if (!v) return;
+        const int mu = t.gao_mu[i];
         ao[row + mu] += val;
         if (DERIV) {
             if (dao) {
@@ -2301,7 +2302,7 @@ __global__ __launch_bounds__(kBlock) void ao_kernel(AArgs a) {
             if (d2ao) d2ao[row + mu] += al;
         }
     };
-    ao_row<double, RAD, DERIV>(t, a.p, p[0], p[1], p[2], sink);
+    ao_shells<double, RAD, DERIV>(t, a.p, p[0], p[1], p[2], sink);
 }
 
 // Adjoint rows of log|psi| (see qmc_logpsi_grad_rows in the header).
@@ -2494,14 +2495,15 @@ __global__ __launch_bounds__(kBlock) void grad_kernel(GArgs a) {
     {
         double* aor = a.ao_rows + row * t.nao;
         const double* W = (const double*)a.p.mo_w;
-        auto sink = [&](int, int mu, double val, double, double, double, double) {
+        auto sink = [&](int i, int, double val, double, double, double, double) {
+            const int mu = t.gao_mu[i];
             if (v) aor[mu] += val;
             const QMC_CONST double* wr = (const QMC_CONST double*)W + (size_t)mu * t.nmo;
 #pragma unroll
             for (int m = 0; m < NM; ++m)
                 if (m < t.nmo) mo[m] += val * wr[m];
         };
-        ao_row<double, RAD, false>(t, a.p, x, y, z, sink);
+        ao_shells<double, RAD, false>(t, a.p, x, y, z, sink);
     }
     double ld[QMC_MAXCONF], sd[QMC_MAXCONF], om[QMC_MAXCONF], gam[NM];
 #pragma unroll
@@ -2694,7 +2696,8 @@ __global__ __launch_bounds__(kBlock) void eloc_grad_kernel(EArgs a) {
         const double* W = (const double*)a.p.mo_w;
         double* aor = a.ao_rows ? a.ao_rows + row * t.nao : nullptr;
         double* bor = a.b_rows ? a.b_rows + row * t.nao : nullptr;
-        auto sink = [&](int, int mu, double ao, double ax, double ay, double az, double al) {
+        auto sink = [&](int i, int, double ao, double ax, double ay, double az, double al) {
+            const int mu = t.gao_mu[i];
             if (v && aor) aor[mu] += ao;
             if (v && bor) bor[mu] += -0.5 * (al + 2.0 * (g[0] * ax + g[1] * ay + g[2] * az) + l2 * ao);
             const QMC_CONST double* wr = (const QMC_CONST double*)W + (size_t)mu * t.nmo;
@@ -2710,7 +2713,7 @@ __global__ __launch_bounds__(kBlock) void eloc_grad_kernel(EArgs a) {
                 }
             }
         };
-        ao_row<double, RAD, true>(t, a.p, x, y, z, sink);
+        ao_shells<double, RAD, true>(t, a.p, x, y, z, sink);
     }
     double bk[NM];
 #pragma unroll
