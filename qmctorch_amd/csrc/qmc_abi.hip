@@ -439,6 +439,7 @@ int qmc_plan_create(const QmcSystemDesc* d, QmcPlan** out) {
             t.exc_up = (decltype(t.exc_up))p->upload(exc_up.data(), exc_up.size());
             t.exc_dn = (decltype(t.exc_dn))p->upload(exc_dn.data(), exc_dn.size());
         }
+        p->upload_done();
         // generated kernels have no excitation path
         p->spec = exc ? nullptr : find_spec(layout_signature(d), nm_bucket_fine(t), (64 / t.nelec) * t.nelec, !ident);
     } catch (const std::exception& ex) {

@@ -471,8 +471,8 @@ __device__ __forceinline__ void eloc_adjoint_reduce(const ERedArgs& a, const Wal
         }
     } else if constexpr (!MULTI) {
         double lg, sg, inv[NM], zz[NM];
-        conf_inverse<NM>(t, L, 0, mo, own_ex, lg, sg, inv);
-        inverse_b_inverse<NM>(t, L, inv, brow, ycol, [](int k) { return k; }, zz);
+        const int oc_ = conf_inverse<NM>(t, L, 0, mo, own_ex, lg, sg, inv);
+        inverse_b_inverse<NM>(t, L, inv, oc_, brow, ycol, [](int k) { return k; }, zz);
         double tp = 0.0;
 #pragma unroll
         for (int k = 0; k < NM; ++k) {
@@ -544,10 +544,10 @@ __device__ __forceinline__ void eloc_adjoint_reduce(const ERedArgs& a, const Wal
 #pragma unroll 1
         for (int c = 0; c < t.nconf_max; ++c) {
             double lg, sg, inv[NM], zz[NM];
-            conf_inverse<NM>(t, L, c, mo, own_ex, lg, sg, inv);
+            const int oc_ = conf_inverse<NM>(t, L, c, mo, own_ex, lg, sg, inv);
             const int nc = L.spin == 0 ? t.nconf_up : t.nconf_dn, cc = c < nc ? c : nc - 1;
             const QMC_CONST int* cf = L.spin == 0 ? t.conf_up + cc * t.nup : t.conf_dn + cc * t.ndown;
-            inverse_b_inverse<NM>(t, L, inv, brow, ycol, [&](int k) { return t.identity_conf ? k : (int)cf[k]; }, zz);
+            inverse_b_inverse<NM>(t, L, inv, oc_, brow, ycol, [&](int k) { return t.identity_conf ? k : (int)cf[k]; }, zz);
             double rc = 0.0, oc = 0.0;
 #pragma unroll
             for (int c2 = 0; c2 < QMC_MAXCONF; ++c2)

@@ -128,6 +128,7 @@ __device__ __forceinline__ T ipow(T x, int k) {
 template <typename T, bool DERIV>
 __device__ __forceinline__ void cart_poly(T x, T y, T z, int kx, int ky, int kz, T& Y, T& Yx, T& Yy, T& Yz,
                                           T& Ylap) {
+#pragma clang fp contract(off)
     T px = ipow(x, kx), py = ipow(y, ky), pz = ipow(z, kz);
     Y = px * py * pz;
     if (DERIV) {
@@ -145,20 +146,20 @@ __device__ __forceinline__ void cart_poly(T x, T y, T z, int kx, int ky, int kz,
 }
 
 // ------------------------------------------------------------ AO -> MO row
-// Evaluates the AOs of one electron group by group and contracts them into
-// the MO row on the fly (the AO row never leaves registers).
+// Evaluates the AOs of one electron shell by shell and contracts them into the
+// MO row on the fly (the AO row never leaves registers).  With the moments
+// m_j = sum_p K_p a_p^j e_p of a shell's primitives, e_p = exp(-a_p r^2) (GTO,
+// radial_functions.py:241-320) or exp(-a_p r) (STO, radial_functions.py:6-123),
+//   AO = v Y,  grad AO = v grad Y + c Y r,  lap AO = Y (A + L B) + v lap Y:
+//   GTO  v = m0, c = -2 m1, A = 4 r^2 m2 - 6 m1, B = -4 m1;
+//   STO  R = r^n:  v = R m0, c = R (n m0 / r^2 - m1 / r),
+//        A = R (n (n+1) m0 / r^2 - 2 (n+1) m1 / r + m2), B = 2 c
+// (L the total Cartesian power), shared by the shell's 1, 3 or 6 entries.
 //
-//   GTO (radial_functions.py:241-320): with S_k = sum_p K_p a_p^k exp(-a_p r^2)
-//     AO = Y S0,  grad AO = S0 grad Y - 2 S1 Y r,
-//     lap AO = Y (4 r^2 S2 - (6 + 4L) S1) + S0 lap Y          (L = kx+ky+kz)
-//   STO (radial_functions.py:6-123): R_p = r^n exp(-a r), q = n/r^2 - a/r,
-//     AO = Y sum K R,  grad AO = (sum K R) grad Y + Y (sum K R q) r,
-//     lap AO = Y sum K R (n(n+1)/r^2 - 2a(n+1)/r + a^2 + 2Lq) + (sum K R) lap Y
-//
-// sink(i, mu, ao, gx, gy, gz, lap) is called once per AO entry i (AO mu); entries of one
+// sink(i, mu, ao, gx, gy, gz, lap) is called once per AO entry i; entries of one
 // AO that were split across groups are delivered separately (all consumers
-// are linear in the AO).  The primitive count of a group selects a fully
-// unrolled instance (no predicated slots).
+// are linear in the AO).
+
 // exponents gathered in group-primitive order, in the evaluation precision
 template <typename T>
 __device__ __forceinline__ const T* group_exponents(const QmcParams& prm);
@@ -183,63 +184,6 @@ __device__ __forceinline__ void group_prims_from(const T* gexp, int p0, T r2, T 
     }
 }
 
-// AO entry i (AO mu, Cartesian powers kx, ky, kz) of a group from its
-// primitive exponentials; hands value, gradient and Laplacian to the sink.
-// kcoef(p) is the contraction coefficient K_p of primitive p, rpow(p) its STO
-// r power (unused for Gaussians): read from the plan tables, or written into a
-// generated row as literals.
-template <typename T, int RAD, bool DERIV, int NP, typename KF, typename NF, typename Sink>
-__device__ __forceinline__ void ao_entry_with(KF kcoef, NF rpow, int i, int mu, int kx, int ky, int kz,
-                                              const T (&E)[NP], const T (&A)[NP], T dx, T dy, T dz, T r2, T r,
-                                              T ir, Sink& sink) {
-    T Y, Yx = 0, Yy = 0, Yz = 0, Yl = 0;
-    cart_poly<T, DERIV>(dx, dy, dz, kx, ky, kz, Y, Yx, Yy, Yz, Yl);
-    T s0 = 0, s1 = 0, s2 = 0;
-    if (RAD == QMC_RADIAL_GTO_PURE) {
-#pragma unroll
-        for (int p = 0; p < NP; ++p) {
-            const T ke = kcoef(p) * E[p];
-            s0 += ke;
-            if (DERIV) {
-                s1 += ke * A[p];
-                s2 += ke * A[p] * A[p];
-            }
-        }
-        const T ao = Y * s0;
-        if (DERIV) {
-            const T L = T(kx + ky + kz);
-            const T c = T(-2) * s1 * Y;
-            sink(i, mu, ao, s0 * Yx + c * dx, s0 * Yy + c * dy, s0 * Yz + c * dz,
-                 Y * (T(4) * r2 * s2 - (T(6) + T(4) * L) * s1) + s0 * Yl);
-        } else {
-            sink(i, mu, ao, T(0), T(0), T(0), T(0));
-        }
-    } else {
-        const T L = T(kx + ky + kz);
-#pragma unroll
-        for (int p = 0; p < NP; ++p) {
-            const double np_ = rpow(p);
-            const T n = (T)np_;
-            const int ni = (int)np_;
-            const T kr = kcoef(p) * ipow(r, ni) * E[p];
-            s0 += kr;
-            if (DERIV) {
-                const T a = A[p];
-                const T q = n * ir * ir - a * ir;
-                s1 += kr * q;
-                s2 += kr * (n * (n + T(1)) * ir * ir - T(2) * a * (n + T(1)) * ir + a * a + T(2) * L * q);
-            }
-        }
-        const T ao = Y * s0;
-        if (DERIV) {
-            const T c = Y * s1;
-            sink(i, mu, ao, s0 * Yx + c * dx, s0 * Yy + c * dy, s0 * Yz + c * dz, Y * s2 + s0 * Yl);
-        } else {
-            sink(i, mu, ao, T(0), T(0), T(0), T(0));
-        }
-    }
-}
-
 // ----------------------------------------------- table-driven AO row by shells
 // The row of the kernels for any basis layout.  The plan describes it as
 // records of up to three shells that share their primitives:
@@ -251,15 +195,8 @@ __device__ __forceinline__ void ao_entry_with(KF kcoef, NF rpow, int i, int mu, 
 // its use, and the loads it leads to (exponents, coefficients, W rows) are
 // issued together: walking the group and entry tables instead cost four
 // dependent scalar loads per group and three per entry, and every entry
-// selected its Cartesian powers at run time.  With the primitives' moments
-// m_j = sum_p K_p a_p^j e_p, e_p = exp(-a_p r^2) or exp(-a_p r), a shell's
-// radial part is
-//   value v, gradient  v grad Y + c Y r,  Laplacian  Y (A + L B) + v lap Y:
-//   GTO  v = m0, c = -2 m1, A = 4 r^2 m2 - 6 m1, B = -4 m1;
-//   STO  R = r^n:  v = R m0, c = R (n m0 / r^2 - m1 / r),
-//        A = R (n (n+1) m0 / r^2 - 2 (n+1) m1 / r + m2), B = 2 c
-// (L the total Cartesian power), shared by its 1, 3 or 6 entries.  Two waters
-// (20 electrons, 50 AOs, FP64), 2047 walkers x 50 steps: 1.411 -> 1.181 ms.
+// selected its Cartesian powers at run time.  Two waters (20 electrons, 50 AOs,
+// FP64), 2047 walkers x 50 steps: 1.411 -> 1.181 ms.
 constexpr int kRecWords = 8;
 constexpr int kRecShells = 3;  // shells per record at most
 enum ShellType { kShellS = 0, kShellP = 1, kShellD = 2, kShellOne = 3 };  // D: xx xy xz yy yz zz; One: one entry
@@ -275,30 +212,103 @@ __device__ __forceinline__ const QMC_CONST double* record_coeffs<double>(const T
     return t.rec_K;
 }
 
-// moments m[shell][j] (j = 0, with DERIV also 1 and 2) of a record's NP primitives
+// The pieces of a shell below say themselves where a product and a sum share
+// one rounding: left to the compiler, a table-driven and a generated row would
+// round differently, and near a node of the determinant FP32 rows that differ by
+// one rounding differ by 1e-3 in log|psi|.
+
+template <typename T>
+__device__ __forceinline__ T norm2(T x, T y, T z) {
+    return fma(z, z, fma(y, y, x * x));
+}
+
+// moments of a shell (m1 and m2 with DERIV) from its primitives' exponentials
+template <typename T, bool DERIV, int NP, typename KF>
+__device__ __forceinline__ void shell_moments(KF kcoef, const T (&E)[NP], const T (&A)[NP], T& m0, T& m1, T& m2) {
+#pragma clang fp contract(off)
+    m0 = m1 = m2 = T(0);
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        const T k = kcoef(p);
+        m0 = fma(k, E[p], m0);
+        if (DERIV) {
+            const T kea = k * E[p] * A[p];
+            m1 += kea;
+            m2 = fma(kea, A[p], m2);
+        }
+    }
+}
+
+// radial part of a shell from its moments; n: STO r power
+template <typename T>
+struct ShellRadial {
+    T v, c, A, B;
+};
+template <typename T, int RAD, bool DERIV>
+__device__ __forceinline__ ShellRadial<T> shell_radial(T m0, T m1, T m2, int n, T r2, T r, T ir) {
+#pragma clang fp contract(off)
+    ShellRadial<T> s{m0, T(0), T(0), T(0)};
+    if (RAD == QMC_RADIAL_GTO_PURE) {
+        if (DERIV) {
+            s.c = T(-2) * m1;
+            s.A = fma(T(4) * r2, m2, T(-6) * m1);
+            s.B = T(-4) * m1;
+        }
+    } else {
+        const T R = ipow(r, n);
+        s.v = R * m0;
+        if (DERIV) {
+            const T fn = T(n);
+            s.c = R * fma(fn * m0 * ir, ir, -(m1 * ir));
+            s.A = R * (fma(fn * (fn + T(1)) * m0 * ir, ir, T(-2) * (fn + T(1)) * m1 * ir) + m2);
+            s.B = T(2) * s.c;
+        }
+    }
+    return s;
+}
+
+// the entries of a shell from i on; f: normalisation of d_xy relative to d_xx;
+// kx, ky, kz: the powers of a single entry
+template <typename T, bool DERIV, int TYPE, typename Sink>
+__device__ __forceinline__ void shell_entries(int i, const ShellRadial<T>& s, T x, T y, T z, T f, int kx, int ky,
+                                              int kz, Sink& sink) {
+#pragma clang fp contract(off)
+    const T v = s.v, c = s.c;
+    if (TYPE == kShellS) {
+        sink(i, 0, v, c * x, c * y, c * z, s.A);
+    } else if (TYPE == kShellP) {
+        const T l = s.A + s.B, cx = c * x, cy = c * y, cz = c * z;
+        sink(i + 0, 0, v * x, fma(cx, x, v), cx * y, cx * z, l * x);
+        sink(i + 1, 0, v * y, cy * x, fma(cy, y, v), cy * z, l * y);
+        sink(i + 2, 0, v * z, cz * x, cz * y, fma(cz, z, v), l * z);
+    } else if (TYPE == kShellD) {
+        const T l = fma(T(2), s.B, s.A), vf = v * f, cf = c * f, lf = l * f, v2 = v + v;
+        const T xx = x * x, xy = x * y, xz = x * z, yy = y * y, yz = y * z, zz = z * z;
+        sink(i + 0, 0, v * xx, x * fma(c, xx, v2), c * xx * y, c * xx * z, fma(l, xx, v2));
+        sink(i + 1, 0, vf * xy, y * fma(cf, xx, vf), x * fma(cf, yy, vf), cf * xy * z, lf * xy);
+        sink(i + 2, 0, vf * xz, z * fma(cf, xx, vf), cf * xz * y, x * fma(cf, zz, vf), lf * xz);
+        sink(i + 3, 0, v * yy, c * yy * x, y * fma(c, yy, v2), c * yy * z, fma(l, yy, v2));
+        sink(i + 4, 0, vf * yz, cf * yz * x, z * fma(cf, yy, vf), y * fma(cf, zz, vf), lf * yz);
+        sink(i + 5, 0, v * zz, c * zz * x, c * zz * y, z * fma(c, zz, v2), fma(l, zz, v2));
+    } else {
+        T Y, Yx = 0, Yy = 0, Yz = 0, Yl = 0;
+        cart_poly<T, DERIV>(x, y, z, kx, ky, kz, Y, Yx, Yy, Yz, Yl);
+        const T cY = c * Y;
+        sink(i, 0, v * Y, fma(cY, x, v * Yx), fma(cY, y, v * Yy), fma(cY, z, v * Yz),
+             fma(v, Yl, Y * fma(T(kx + ky + kz), s.B, s.A)));
+    }
+}
+
+// moments m[shell][j] of a record's nk shells and NP primitives
 template <typename T, int RAD, bool DERIV, int NP>
 __device__ __forceinline__ void record_moments(const T* gexp, const QMC_CONST T* K, int nk, T r2, T r,
                                                T (&m)[kRecShells][3]) {
     T E[NP], A[NP];
     group_prims_from<T, RAD, NP>(gexp, 0, r2, r, E, A);
 #pragma unroll
-    for (int q = 0; q < kRecShells; ++q) {
-        if (q < nk) {
-            T m0 = 0, m1 = 0, m2 = 0;
-#pragma unroll
-            for (int p = 0; p < NP; ++p) {
-                const T ke = K[q * (NP + 1) + p] * E[p];
-                m0 += ke;
-                if (DERIV) {
-                    m1 += ke * A[p];
-                    m2 += ke * A[p] * A[p];
-                }
-            }
-            m[q][0] = m0;
-            m[q][1] = m1;
-            m[q][2] = m2;
-        }
-    }
+    for (int q = 0; q < kRecShells; ++q)
+        if (q < nk)
+            shell_moments<T, DERIV, NP>([&](int p) { return K[q * (NP + 1) + p]; }, E, A, m[q][0], m[q][1], m[q][2]);
 }
 
 template <typename T, int RAD, bool DERIV, typename Sink>
@@ -318,7 +328,7 @@ __device__ __forceinline__ void ao_shells(const Tables& t, const QmcParams& prm,
             x = (T)(ex - ldc(prm.atom_coords, 3 * at + 0));
             y = (T)(ey - ldc(prm.atom_coords, 3 * at + 1));
             z = (T)(ez - ldc(prm.atom_coords, 3 * at + 2));
-            r2 = x * x + y * y + z * z;
+            r2 = norm2(x, y, z);
             if (RAD == QMC_RADIAL_STO) {
                 r = fsqrt(r2);
                 ir = T(1) / r;
@@ -343,56 +353,21 @@ __device__ __forceinline__ void ao_shells(const Tables& t, const QmcParams& prm,
             const int word = q == 0 ? w[4] : (q == 1 ? w[5] : w[6]);
             const int type = word & 15;
             const T m0 = q == 0 ? m[0][0] : (q == 1 ? m[1][0] : m[2][0]);
-            T v = m0, c = 0, A = 0, B = 0;
-            if (RAD == QMC_RADIAL_GTO_PURE) {
-                if (DERIV) {
-                    const T m1 = q == 0 ? m[0][1] : (q == 1 ? m[1][1] : m[2][1]);
-                    const T m2 = q == 0 ? m[0][2] : (q == 1 ? m[1][2] : m[2][2]);
-                    c = T(-2) * m1;
-                    A = T(4) * r2 * m2 - T(6) * m1;
-                    B = T(-4) * m1;
-                }
-            } else {
-                const int n = word >> 16;
-                const T R = ipow(r, n);
-                v = R * m0;
-                if (DERIV) {
-                    const T m1 = q == 0 ? m[0][1] : (q == 1 ? m[1][1] : m[2][1]);
-                    const T m2 = q == 0 ? m[0][2] : (q == 1 ? m[1][2] : m[2][2]);
-                    const T fn = T(n);
-                    c = R * (fn * m0 * ir * ir - m1 * ir);
-                    A = R * (fn * (fn + T(1)) * m0 * ir * ir - T(2) * (fn + T(1)) * m1 * ir + m2);
-                    B = T(2) * c;
-                }
-            }
+            const T m1 = q == 0 ? m[0][1] : (q == 1 ? m[1][1] : m[2][1]);
+            const T m2 = q == 0 ? m[0][2] : (q == 1 ? m[1][2] : m[2][2]);
+            const ShellRadial<T> s = shell_radial<T, RAD, DERIV>(m0, m1, m2, word >> 16, r2, r, ir);
             if (type == kShellS) {
-                sink(i, 0, v, c * x, c * y, c * z, A);
+                shell_entries<T, DERIV, kShellS>(i, s, x, y, z, T(0), 0, 0, 0, sink);
                 i += 1;
             } else if (type == kShellP) {
-                const T l = A + B, cx = c * x, cy = c * y, cz = c * z;
-                sink(i + 0, 0, v * x, v + cx * x, cx * y, cx * z, l * x);
-                sink(i + 1, 0, v * y, cy * x, v + cy * y, cy * z, l * y);
-                sink(i + 2, 0, v * z, cz * x, cz * y, v + cz * z, l * z);
+                shell_entries<T, DERIV, kShellP>(i, s, x, y, z, T(0), 0, 0, 0, sink);
                 i += 3;
             } else if (type == kShellD) {
-                const T f = K[q * (np + 1) + np];  // normalisation of xy relative to xx
-                const T l = A + T(2) * B, vf = v * f, cf = c * f, lf = l * f;
-                const T xx = x * x, xy = x * y, xz = x * z, yy = y * y, yz = y * z, zz = z * z;
-                const T v2 = v + v;
-                sink(i + 0, 0, v * xx, x * (v2 + c * xx), c * xx * y, c * xx * z, l * xx + v2);
-                sink(i + 1, 0, vf * xy, y * (vf + cf * xx), x * (vf + cf * yy), cf * xy * z, lf * xy);
-                sink(i + 2, 0, vf * xz, z * (vf + cf * xx), cf * xz * y, x * (vf + cf * zz), lf * xz);
-                sink(i + 3, 0, v * yy, c * yy * x, y * (v2 + c * yy), c * yy * z, l * yy + v2);
-                sink(i + 4, 0, vf * yz, cf * yz * x, z * (vf + cf * yy), y * (vf + cf * zz), lf * yz);
-                sink(i + 5, 0, v * zz, c * zz * x, c * zz * y, z * (v2 + c * zz), l * zz + v2);
+                shell_entries<T, DERIV, kShellD>(i, s, x, y, z, K[q * (np + 1) + np], 0, 0, 0, sink);
                 i += 6;
             } else {
-                const int kx = (word >> 4) & 15, ky = (word >> 8) & 15, kz = (word >> 12) & 15;
-                T Y, Yx = 0, Yy = 0, Yz = 0, Yl = 0;
-                cart_poly<T, DERIV>(x, y, z, kx, ky, kz, Y, Yx, Yy, Yz, Yl);
-                const T cY = c * Y;
-                sink(i, 0, v * Y, v * Yx + cY * x, v * Yy + cY * y, v * Yz + cY * z,
-                     Y * (A + T(kx + ky + kz) * B) + v * Yl);
+                shell_entries<T, DERIV, kShellOne>(i, s, x, y, z, T(0), (word >> 4) & 15, (word >> 8) & 15,
+                                                   (word >> 12) & 15, sink);
                 i += 1;
             }
         }
@@ -401,13 +376,12 @@ __device__ __forceinline__ void ao_shells(const Tables& t, const QmcParams& prm,
 
 // AO evaluation policies of the kernels: AoGeneric walks the shell records
 // above; a generated policy (qmc_spec_*.hip) walks one basis layout with every
-// group, entry, primitive offset and Cartesian power a compile-time constant,
-// built from the atom_geo / group_prims / ao_entry pieces above in the same
-// order of entries, so both give the same values up to rounding.
+// shell, primitive offset and coefficient a compile-time constant, built from
+// the same pieces in the same order, so both give the same values.
 struct AoGeneric {
     static constexpr int kEntries = 0;    // AO entries of the row: known at run time only
     static constexpr int kRowBlocks = 4;  // 16-lane row blocks of the MFMA contraction: all
-    template <typename T, int RAD, bool DERIV, bool TIGHT, typename Sink>
+    template <typename T, int RAD, bool DERIV, typename Sink>
     static __device__ __forceinline__ void row(const Tables& t, const QmcParams& prm, double ex, double ey, double ez,
                                                Sink&& sink) {
         ao_shells<T, RAD, DERIV>(t, prm, ex, ey, ez, sink);
@@ -425,7 +399,7 @@ __device__ __forceinline__ AtomGeo<T> atom_geo(double dxd, double dyd, double dz
     g.dx = (T)dxd;
     g.dy = (T)dyd;
     g.dz = (T)dzd;
-    g.r2 = g.dx * g.dx + g.dy * g.dy + g.dz * g.dz;
+    g.r2 = norm2(g.dx, g.dy, g.dz);
     g.r = g.ir = T(0);
     if (RAD == QMC_RADIAL_STO) {
         g.r = fsqrt(g.r2);
@@ -756,27 +730,21 @@ __device__ __forceinline__ void lane_det_lds(double (&a)[NM], int n, int nmax, i
     logdet = singular ? -INFINITY : log_mantissa(mant) + 0.6931471805599453 * (double)expo;
 }
 
-// ------------------------------------------------ augmented elimination (LDS)
-// lane_gauss_jordan<NM, true> with the pivot row passed through LDS and, above
-// 8 columns, the pivot found by seg_pivot: same arithmetic, same outputs up to
-// the choice between pivots equal to 15 mantissa bits, for matrices a whose
-// columns n..NM-1 are zero on entry (gathered configurations).
-// rowbuf is the group's n * NM doubles (the lane_det_lds buffer).  Up to
-// NM = 16 the pivot lane stores its b[0..NM) at rowbuf[0..NM) and its a[j],
-// k < j < n, at rowbuf[NM - 1 + j] (at most NM + n - 1 doubles, so it fits
-// for every n <= NM); readers take the a-part only for j < n (the columns
-// past n stay zero, as in the shuffle version, where the pivot row's entries
-// there are zero).  For the larger buckets, where unmasked loads of whole b
-// rows raise the register pressure, b must also be zero past n: the row is
-// b[0..n) at rowbuf[0..n) and a[j] at rowbuf[n - 1 + j], both read for j < n
-// only (at most 2n - 1 doubles).  The loads of the masked columns may read up
-// to 2 NM - 2 doubles past rowbuf, which the buffer's tail padding keeps in
-// bounds.
+// ------------------------------------------------------ in-place inverse (LDS)
+// Gauss-Jordan inversion of the n x n matrix whose row r lives in lane
+// gbase + r, in the NM registers of the row: after the step of column k with
+// pivot row p, storage column k holds the inverse's column of row p.  On exit
+// the lane that pivoted column k (my_col = k) holds row k of A^-1 with the
+// entry of row i in storage column (my_col of row i's lane); log|det| and sign
+// as lane_det_lds, pivots chosen by seg_pivot.  NM multiply-adds per column and
+// row, where eliminating [A | I] or [A | B] took up to 2 NM and twice the
+// registers.  rowbuf: the group's row buffer (NM doubles used).
 template <int NM>
-__device__ __forceinline__ void lane_gj_lds(double (&a)[NM], double (&b)[NM], int n, int nmax, int myrow, int gbase,
-                                            int spin, uint64_t gmask, bool may_store, double* rowbuf, double& logdet,
-                                            double& sgn, double& trace_part, int& my_col) {
-    if constexpr (NM > 8) seg_pivot_init(myrow, gbase, may_store);
+__device__ __forceinline__ void lane_invert_lds(double (&a)[NM], int n, int nmax, int myrow, int gbase,
+                                                uint64_t gmask, bool may_store, double* rowbuf, double& logdet,
+                                                double& sgn, int& my_col) {
+    seg_pivot_init(myrow, gbase, may_store);
+    double* const pivot = det_recips() + gbase;  // the column's pivot
     bool done = false;
     my_col = -1;
     sgn = 1.0;
@@ -784,63 +752,44 @@ __device__ __forceinline__ void lane_gj_lds(double (&a)[NM], double (&b)[NM], in
     bool singular = false;
     double mant = 1.0;  // |det| = mant * 2^expo, renormalised after every pivot
     int expo = 0;
-    constexpr bool kFullB = NM <= 16;
-    double* const ra = rowbuf + ((kFullB ? NM : n) - 1);  // a-part: ra[j] for k < j < n
 #pragma unroll
     for (int k = 0; k < NM; ++k) {
         if (k < nmax) {
             const bool colk = k < n;
-            int br;
-            if constexpr (NM <= 8) {
-                const double cand = (!done && colk && myrow < n) ? fabs(a[k]) : -1.0;
-                double c[NM];
-#pragma unroll
-                for (int s = 0; s < NM; ++s) c[s] = __shfl(cand, gbase + (s < n ? s : 0));
-                double bb = -1.0;
-                br = 0;
-#pragma unroll
-                for (int s = 0; s < NM; ++s) {
-                    if (s < n && c[s] > bb) {
-                        bb = c[s];
-                        br = s;
-                    }
-                }
-            } else {
-                br = seg_pivot<NM>(k, !done && colk && myrow < n, a[k], myrow, gbase, may_store);
-            }
-            const int plane = gbase + br;
+            const bool cand = !done && colk && myrow < n;
+            seg_pivot_post<NM>(k, cand, a[k], myrow, gbase, may_store);
+            // the reciprocal of every candidate is formed while the search runs
+            double rk = (a[k] != 0.0) ? 1.0 / a[k] : 0.0;
+            asm volatile("" : "+v"(rk));
+            const int br = seg_pivot_get(k, gbase);
             const uint64_t bal = __ballot(!done && myrow < br);
             if (colk) inversions += __popcll(bal & gmask);
-            const double piv = __shfl(a[k], plane);
             const bool is_piv = colk && (myrow == br);
-            if (colk) {
-                singular = singular || (piv == 0.0);
-                int ex;
-                mant = frexp(mant * fabs(piv), &ex);
-                expo += ex;
-                sgn *= (piv < 0.0) ? -1.0 : 1.0;
-            }
-            const double ip = (piv != 0.0) ? 1.0 / piv : 0.0;
-            const double f = (colk && !is_piv) ? a[k] * ip : 0.0;
-            wave_lds_sync();  // the previous column's reads are done
+            wave_lds_sync();  // the previous column's reads come first
             if (is_piv && may_store) {
+                // the pivot row over its pivot, the reciprocal in its own column
 #pragma unroll
-                for (int j = 0; j < NM; ++j)
-                    if (kFullB || j < n) rowbuf[j] = b[j];
-#pragma unroll
-                for (int j = k + 1; j < NM; ++j)
-                    if (j < n) ra[j] = a[j];
+                for (int j = 0; j < NM; ++j) rowbuf[j] = j == k ? rk : a[j] * rk;
+                *pivot = a[k];
             }
             wave_lds_sync();
-#pragma unroll
-            for (int j = k + 1; j < NM; ++j) {
-                const double pa = (j < n) ? ra[j] : 0.0;
-                a[j] = is_piv ? a[j] * ip : a[j] - f * pa;
+            {
+                // past this group's n nobody stores: colk is false, nothing is used
+                const double pv = colk ? *pivot : 1.0;
+                singular = singular || (pv == 0.0);
+                int ex;
+                mant = frexp(mant * fabs(pv), &ex);
+                expo += ex;
+                sgn *= (pv < 0.0) ? -1.0 : 1.0;
             }
+            const double f = colk ? a[k] : 0.0;
 #pragma unroll
             for (int j = 0; j < NM; ++j) {
-                const double pb = (kFullB || j < n) ? rowbuf[j] : 0.0;
-                b[j] = is_piv ? b[j] * ip : b[j] - f * pb;
+                const double p = rowbuf[j];
+                if (j == k)
+                    a[k] = is_piv ? p : (colk ? -f * p : a[k]);
+                else
+                    a[j] = is_piv ? p : fma(-f, p, a[j]);
             }
             if (is_piv) {
                 done = true;
@@ -850,10 +799,6 @@ __device__ __forceinline__ void lane_gj_lds(double (&a)[NM], double (&b)[NM], in
     }
     if (inversions & 1) sgn = -sgn;
     logdet = singular ? -INFINITY : log_mantissa(mant) + 0.6931471805599453 * (double)expo;
-    trace_part = 0.0;
-#pragma unroll
-    for (int j = 0; j < NM; ++j)
-        if (j == my_col) trace_part = b[j];
 }
 
 }  // namespace qmc

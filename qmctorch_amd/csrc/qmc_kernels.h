@@ -159,6 +159,35 @@ struct MoSink {
     }
 };
 
+// MO row and kinetic row of one electron for the local energy: with g and l2 =
+// (lap J) / J of this electron known, the kinetic operator acts on the AO,
+//   b = lap AO + 2 g . grad AO + l2 AO,   mo[m] += AO W[m],   bk[m] += b W[m],
+// two multiply-adds per column instead of the five of value, gradient and
+// Laplacian rows combined afterwards, and two rows of registers instead of
+// five: E_L of water, 65536 walkers, 90 -> 69 us.
+template <int NM>
+struct KinSink {
+    const double* __restrict__ W;  // entry-ordered W rows, stride NM
+    double gx2, gy2, gz2, l2;      // 2 g, (lap J) / J
+    double* mo;
+    double* bk;
+    __device__ __forceinline__ void fence() {}
+    template <typename P>
+    __device__ __forceinline__ const P* pace(const P* p) const {
+        return p;
+    }
+    __device__ __forceinline__ void operator()(int i, int, double ao, double ax, double ay, double az, double al) const {
+        const QMC_CONST double* wr = (const QMC_CONST double*)W + (size_t)i * NM;
+        const double b = fma(gx2, ax, fma(gy2, ay, fma(gz2, az, fma(l2, ao, al))));
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            const double w = wr[m];
+            mo[m] = fma(ao, w, mo[m]);
+            bk[m] = fma(b, w, bk[m]);
+        }
+    }
+};
+
 // AO -> MO contraction on the matrix cores for the large register buckets
 // (molecular_orbitals.py:79-95): MO = AO W with the wavefront's 64 lanes as the
 // rows of AO (one electron each), the AO entries as K and the bucket's columns
@@ -566,15 +595,14 @@ __device__ __forceinline__ T jastrow_value(const Tables& t, const QmcParams& prm
 }
 
 // Row buffer of this wavefront: NM doubles per lane (64 * NM), shared by the
-// eliminations and the row transposes of the kernel instance; 2 NM doubles of
-// tail padding keep the masked loads of lane_gj_lds in bounds.
+// eliminations and the row transposes of the kernel instance.
 template <int NM>
 __device__ __forceinline__ double* wave_rowbuf() {
-    __shared__ double rows[kBlockWaves * 64 * NM + 2 * NM];
+    __shared__ double rows[kBlockWaves * 64 * NM];
     return rows + (threadIdx.x >> 6) * 64 * NM;
 }
 
-// Pivot-row buffer of lane_det_lds / lane_gj_lds for the group of this lane:
+// Pivot-row buffer of lane_det_lds / lane_invert_lds for the group of this lane:
 // the NM-double rows of the group's lanes gbase .. gbase + n - 1, so any lane
 // layout fits.  Lanes past the wavefront's last walker compute a throw-away
 // group and do not store.
@@ -583,18 +611,27 @@ __device__ __forceinline__ double* det_rowbuf(const WalkerLane& L) {
     return wave_rowbuf<NM>() + L.gbase * NM;
 }
 
-// Augmented elimination [A | B] of this lane's group: the shuffle version up to
-// 8 rows (faster for 5 x 5 blocks: H2O E_L 32.9 vs 33.9 us, HMC launch 1.10 vs
-// 1.20 ms), the LDS pivot-row version above (the benzene adjoint kernel spills
-// 360 instead of 1145 VGPRs).
+// Column of the inverse for this lane's row, inv[k] = (A^-1)[k][row] (zero past
+// the group's n), log|det A| and its sign, of the group matrix whose rows are
+// the lanes' a (destroyed): the in-place inversion, then a transpose through the
+// wavefront's row buffer, which afterwards holds A^-1 of every group: entry
+// (k, row of lane l) at [(gbase + k) NM + the lane's returned column].
 template <int NM>
-__device__ __forceinline__ void lane_gj(const WalkerLane& L, int nmax, double (&a)[NM], double (&b)[NM], double& lg,
-                                        double& sg, double& tp, int& col) {
-    if constexpr (NM <= 8)
-        lane_gauss_jordan<NM, true>(a, b, L.n_sig, nmax, L.myrow, L.gbase, L.gmask, lg, sg, tp, col);
-    else
-        lane_gj_lds<NM>(a, b, L.n_sig, nmax, L.myrow, L.gbase, L.spin, L.gmask, L.lane_real, det_rowbuf<NM>(L), lg, sg,
-                        tp, col);
+__device__ __forceinline__ int lane_inverse(const WalkerLane& L, int nmax, double (&a)[NM], double& lg, double& sg,
+                                            double (&inv)[NM]) {
+    int col;
+    lane_invert_lds<NM>(a, L.n_sig, nmax, L.myrow, L.gbase, L.gmask, L.lane_real, det_rowbuf<NM>(L), lg, sg, col);
+    double* rb = wave_rowbuf<NM>();
+    wave_lds_sync();  // the elimination's loads come first
+    if (L.lane_real && col >= 0) {
+#pragma unroll
+        for (int j = 0; j < NM; ++j) rb[(L.gbase + col) * NM + j] = a[j];
+    }
+    wave_lds_sync();
+    const int c = col < 0 ? 0 : col;
+#pragma unroll
+    for (int k = 0; k < NM; ++k) inv[k] = k < L.n_sig ? rb[(L.gbase + (k < L.n_sig ? k : 0)) * NM + c] : 0.0;
+    return c;
 }
 
 // ---------------------------------------------- small matrices (minors)
@@ -699,8 +736,8 @@ __device__ __forceinline__ double log_abs_product(double d1, double d2, int ex) 
 // and (INV) y[k] = (A_c^-1)[k][this row], the coefficient of configuration
 // column k, zero past the group's n.  own_ex: this lane's row exponent.
 template <int N, int NM, bool SCALE, bool INV, typename Col>
-__device__ __forceinline__ void minor_det_n(const WalkerLane& L, const double* rows, int own_ex, Col col, double& lg,
-                                            double& sg, double (&y)[NM]) {
+__device__ __forceinline__ void minor_det_n(const WalkerLane& L, const double* rows, int own_ex, int nmax, Col col,
+                                            double& lg, double& sg, double (&y)[NM]) {
     double a[N], c[N];
     bool flip;
     int ex;
@@ -717,13 +754,30 @@ __device__ __forceinline__ void minor_det_n(const WalkerLane& L, const double* r
 #pragma unroll
         for (int k = 0; k < NM; ++k) y[k] = k < N ? c[k < N ? k : 0] * id : 0.0;
     }
+    if constexpr (SCALE) {
+        const bool weak = !(fabs(D) >= kWeakDet);
+        if (__any(weak && L.lane_real)) {  // eliminate (qmc_minors.h)
+            double aw[NM], inv[NM], lw, sw;
+#pragma unroll
+            for (int k = 0; k < NM; ++k) aw[k] = k < N ? a[k < N ? k : 0] : 0.0;
+            lane_inverse<NM>(L, nmax, aw, lw, sw, inv);
+            if (weak) {
+                lg = lw + 0.6931471805599453 * (double)(ex + own_ex);
+                sg = sw;
+                if constexpr (INV) {
+#pragma unroll
+                    for (int k = 0; k < NM; ++k) y[k] = ldexp(inv[k], -own_ex);
+                }
+            }
+        }
+    }
 }
 
 template <int NM, bool SCALE, bool INV>
 __device__ __forceinline__ void minor_det(const Tables& t, const WalkerLane& L, const double* rows, int own_ex, int c,
                                           double& lg, double& sg, double (&y)[NM]) {
     if (t.identity_conf) {
-        minor_det_n<NM, NM, SCALE, INV>(L, rows, own_ex, [](int k) { return k; }, lg, sg, y);
+        minor_det_n<NM, NM, SCALE, INV>(L, rows, own_ex, t.nsig_max, [](int k) { return k; }, lg, sg, y);
         return;
     }
     const int nconf = L.spin == 0 ? t.nconf_up : t.nconf_dn;
@@ -734,7 +788,7 @@ __device__ __forceinline__ void minor_det(const Tables& t, const WalkerLane& L, 
     auto col = [&](int k) { return (int)conf[k < L.n_sig ? k : 0]; };
     static_for<1, NM + 1>([&](auto nc) {
         constexpr int N = decltype(nc)::value;
-        if (t.nsig_max == N) minor_det_n<N, NM, SCALE, INV>(L, rows, own_ex, col, lg, sg, y);
+        if (t.nsig_max == N) minor_det_n<N, NM, SCALE, INV>(L, rows, own_ex, N, col, lg, sg, y);
     });
 }
 
@@ -782,6 +836,24 @@ __device__ __forceinline__ void slater_single_minors(const Tables& t, const QmcP
     const double c0 = ldc(prm.ci, 0);
     logabs = log_abs_product(du, dd, et) + logc0;
     sgn = (((du < 0.0) != (dd < 0.0)) != (c0 < 0.0)) ? -1.0 : 1.0;
+    if constexpr (SCALE) {
+        const double D = L.spin == 0 ? du : dd;
+        const bool weak = !(fabs(D) >= kWeakDet);
+        if (__any(weak && L.lane_real)) {  // eliminate (qmc_minors.h)
+            double inv[NM], lw, sw;
+            lane_inverse<NM>(L, t.nsig_max, a, lw, sw, inv);
+            if constexpr (INV) {
+#pragma unroll
+                for (int k = 0; k < NM; ++k) y[k] = weak ? ldexp(inv[k], -own_ex) : y[k];
+            }
+            const double lg = weak ? lw + 0.6931471805599453 * (double)ex : log_abs_product(D, 1.0, ex);
+            const double sg = weak ? sw : (D < 0.0 ? -1.0 : 1.0);
+            const double lu = __shfl(lg, L.wbase), ld = __shfl(lg, dn_lane);
+            const double su = __shfl(sg, L.wbase), sd = __shfl(sg, dn_lane);
+            logabs = lu + (t.ndown > 0 ? ld : 0.0) + logc0;
+            sgn = su * (t.ndown > 0 ? sd : 1.0) * (c0 < 0.0 ? -1.0 : 1.0);
+        }
+    }
 }
 
 // Single configuration, single CI term: log|D_up D_dn| and its sign (ground state).
@@ -801,20 +873,18 @@ __device__ __forceinline__ void slater_single(const Tables& t, const QmcParams& 
     sgn = su * (t.ndown > 0 ? sdn : 1.0) * (c0 < 0.0 ? -1.0 : 1.0);
 }
 
-// slater_single with the kinetic ratio tr(A^-1 B) (eliminations of [A | B]).
+// slater_single with the kinetic ratio tr(A^-1 B), each lane's share of it the
+// product of its kinetic row and its inverse column.
 template <int NM>
 __device__ __forceinline__ void slater_single_kin(const Tables& t, const QmcParams& prm, const WalkerLane& L,
                                                   const double (&mo)[NM], const double (&bk)[NM], double& logabs,
                                                   double& sgn, double& kin) {
-    double a[NM], b[NM];
+    double a[NM], inv[NM], lg, sg, tp = 0.0;
 #pragma unroll
-    for (int j = 0; j < NM; ++j) {
-        a[j] = mo[j];
-        b[j] = bk[j];
-    }
-    double lg, sg, tp;
-    int col;
-    lane_gj<NM>(L, t.nsig_max, a, b, lg, sg, tp, col);
+    for (int j = 0; j < NM; ++j) a[j] = mo[j];
+    lane_inverse<NM>(L, t.nsig_max, a, lg, sg, inv);
+#pragma unroll
+    for (int k = 0; k < NM; ++k) tp += k < L.n_sig ? bk[k] * inv[k] : 0.0;
     kin = seg_sum(tp, L.wbase, t.nelec, t.nelec);
     const int dn_lane = L.wbase + (t.ndown > 0 ? t.nup : 0);
     const double lu = __shfl(lg, L.wbase), su = __shfl(sg, L.wbase);
@@ -890,10 +960,12 @@ __device__ __forceinline__ void slater_combine(const Tables& t, const QmcParams&
             lane_det_lds<NM>(a, L.n_sig, t.nsig_max, L.myrow, L.gbase, L.spin, L.gmask, L.lane_real,
                              det_rowbuf<NM>(L), lg, sg);
         } else {
-            int col;
+            double inv[NM];
             gather_conf<NM>(t, L, c, mo, a);
+            lane_inverse<NM>(L, t.nsig_max, a, lg, sg, inv);
             gather_conf<NM>(t, L, c, bk, b);
-            lane_gj<NM>(L, t.nsig_max, a, b, lg, sg, tp, col);
+#pragma unroll
+            for (int k = 0; k < NM; ++k) tp += k < L.n_sig ? b[k] * inv[k] : 0.0;
         }
         const double tr = KIN ? seg_sum(tp, L.gbase, L.n_sig, t.nsig_max) : 0.0;
 #pragma unroll
@@ -1471,29 +1543,32 @@ __device__ __forceinline__ void wf_walkers(const KArgs& a, const WalkerLane& L) 
     const double* p = a.pos + (size_t)L.wclamp * 3 * t.nelec + 3 * L.e;
     const double x = p[0], y = p[1], z = p[2];
 
-    // local energy: MO rows accumulated in FP64 from an FP64 W; AO groups with
-    // tight exponents in FP64 even when the bulk type T is float
-    using AT = typename std::conditional<ELOC, double, T>::type;
-    AT mo[NM], gx[NM], gy[NM], gz[NM], lp[NM];
-#pragma unroll
-    for (int m = 0; m < NM; ++m) mo[m] = gx[m] = gy[m] = gz[m] = lp[m] = AT(0);
-    MoSink<AT, NM, ELOC, AT> sink{(const AT*)a.p.entry_w, t.nmo, mo, gx, gy, gz, lp};
-    AO::template row<T, RAD, ELOC, ELOC>(t, a.p, x, y, z, sink);
-
     double kee, ken, jgx, jgy, jgz, jlap, vee, ven;
     jastrow_and_potential<ELOC>(t, a.p, L, x, y, z, kee, ken, jgx, jgy, jgz, jlap, vee, ven);
 
+    // local energy: everything in FP64
+    using AT = typename std::conditional<ELOC, double, T>::type;
+    AT mo[NM];
     double bk[NM];
-    if (ELOC) {
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+        mo[m] = AT(0);
+        bk[m] = 0.0;
+    }
+    if constexpr (ELOC) {
         const double l2 = jlap + jgx * jgx + jgy * jgy + jgz * jgz;  // (lap J)/J
+        KinSink<NM> sink{(const double*)a.p.entry_w, 2.0 * jgx, 2.0 * jgy, 2.0 * jgz, l2, mo, bk};
+        AO::template row<double, RAD, true>(t, a.p, x, y, z, sink);
 #pragma unroll
         for (int m = 0; m < NM; ++m) {
-            bk[m] = -0.5 * ((double)lp[m] + 2.0 * (jgx * (double)gx[m] + jgy * (double)gy[m] + jgz * (double)gz[m]) +
-                            l2 * (double)mo[m]);
+            bk[m] *= -0.5;
             // formed here: the compiler otherwise sinks the row and its whole AO
             // evaluation past the determinants, spilling what it holds meanwhile
             asm volatile("" : "+v"(bk[m]));
         }
+    } else {
+        MoSink<AT, NM, false, AT> sink{(const AT*)a.p.entry_w, t.nmo, mo, nullptr, nullptr, nullptr, nullptr};
+        AO::template row<T, RAD, false>(t, a.p, x, y, z, sink);
     }
     double logabs, sgn, kin = 0.0, logj, svee = 0.0, sven = 0.0;
     if constexpr (!EXC && !MULTI && use_minors<NM>()) {
@@ -1549,14 +1624,14 @@ __device__ __forceinline__ void wf_walkers(const KArgs& a, const WalkerLane& L) 
 }
 
 // Waves per SIMD the evaluation kernels are held to: what their registers allow
-// without spilling (168 VGPRs up to 5 columns, 256 up to 7).
-template <int NM>
+// without spilling (168 VGPRs up to 5 columns, 3 with table-driven rows).
+template <int NM, typename AO>
 constexpr int wf_waves() {
-    return NM <= 5 ? 3 : (NM <= 7 ? 2 : 1);
+    return NM <= (AO::kEntries > 0 ? 5 : 3) ? 3 : (NM <= 12 ? 2 : 1);
 }
 
 template <typename T, int NM, int RAD, bool ELOC, bool MULTI, typename AO = AoGeneric>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(wf_waves<NM>()))) void wf_kernel(KArgs a) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(wf_waves<NM, AO>()))) void wf_kernel(KArgs a) {
     const WalkerLane L = lane_layout(a.t, a.nw);
     if ((int64_t)L.wave * L.G >= a.nw) return;  // whole wavefront beyond the batch
     wf_walkers<T, NM, RAD, ELOC, MULTI, AO>(a, L);
@@ -1578,7 +1653,7 @@ struct WJob {
 };
 
 template <typename T, int NM, int RAD, bool ELOC, bool MULTI, typename AO = AoGeneric>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(wf_waves<NM>()))) void wf_batch_kernel(const WJob* __restrict__ jobs, int njobs, int nwaves) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(wf_waves<NM, AO>()))) void wf_batch_kernel(const WJob* __restrict__ jobs, int njobs, int nwaves) {
     const int wave = global_wave();
     if (wave >= nwaves) return;
     const int j = find_job(jobs, njobs, wave);
@@ -1623,13 +1698,13 @@ __device__ __forceinline__ double eval_logpsi(const Tables& t, const QmcParams& 
                                                MfmaPairSink<NM, WLDS>>::type;
         Sink sink;
         sink.init((const float*)w, t.nentry);
-        AO::template row<T, RAD, false, false>(t, prm, x, y, z, sink);
+        AO::template row<T, RAD, false>(t, prm, x, y, z, sink);
         sink.finish(mo);
     } else {
 #pragma unroll
         for (int m = 0; m < NM; ++m) mo[m] = T(0);
         MoSink<T, NM, false, T, false, WLDS> sink{w, t.nmo, mo, nullptr, nullptr, nullptr, nullptr};
-        AO::template row<T, RAD, false, false>(t, prm, x, y, z, sink);
+        AO::template row<T, RAD, false>(t, prm, x, y, z, sink);
     }
     const T kj = jastrow_value<T>(t, prm, L, x, y, z);
     double logabs;
@@ -1934,14 +2009,13 @@ __device__ __forceinline__ T jastrow_value_grad(const Tables& t, const QmcParams
 // every other plan): the per-configuration values live in registers.
 template <typename T, int NM, int RAD, int MC, typename AO = AoGeneric>
 __device__ __forceinline__ double eval_drift(const Tables& t, const QmcParams& prm, const WalkerLane& L, double x,
-                                             double y, double z, double logc0, double* lds, double& sgn,
-                                             double (&dr)[3]) {
+                                             double y, double z, double logc0, double& sgn, double (&dr)[3]) {
     T mo[NM], gx[NM], gy[NM], gz[NM];
 #pragma unroll
     for (int m = 0; m < NM; ++m) mo[m] = gx[m] = gy[m] = gz[m] = T(0);
     // values and gradients only: the row's Laplacian terms are dead code here
     MoSink<T, NM, true, T, false> sink{(const T*)prm.entry_w, t.nmo, mo, gx, gy, gz, nullptr};
-    AO::template row<T, RAD, true, false>(t, prm, x, y, z, sink);
+    AO::template row<T, RAD, true>(t, prm, x, y, z, sink);
     if constexpr (use_minors<NM>()) {
         // formed here, not sunk past the determinants (as the kinetic row of wf_walkers)
 #pragma unroll
@@ -1992,17 +2066,7 @@ __device__ __forceinline__ double eval_drift(const Tables& t, const QmcParams& p
             minor_det<NM, SCALE, true>(t, L, rows, own_ex, c, lg, sg, ib);
         } else {
             gather_conf<NM>(t, L, c, mo, aa);
-#pragma unroll
-            for (int j = 0; j < NM; ++j) ib[j] = (j == L.myrow) ? 1.0 : 0.0;
-            double tp;
-            int col;
-            lane_gj<NM>(L, t.nsig_max, aa, ib, lg, sg, tp, col);
-            wave_lds_sync();  // earlier reads of the row buffer are done
-            if (L.lane_real && col >= 0) {
-#pragma unroll
-                for (int j = 0; j < NM; ++j) lds[(L.gbase + col) * NM + j] = ib[j];
-            }
-            wave_lds_sync();
+            lane_inverse<NM>(L, t.nsig_max, aa, lg, sg, ib);
         }
         double ga[NM], gb[NM], gc[NM];
         gather_conf<NM>(t, L, c, gx, ga);
@@ -2012,7 +2076,7 @@ __device__ __forceinline__ double eval_drift(const Tables& t, const QmcParams& p
 #pragma unroll
         for (int k = 0; k < NM; ++k) {
             if (k < L.n_sig) {
-                const double inv = use_minors<NM>() ? ib[k] : lds[(L.gbase + k) * NM + L.myrow];
+                const double inv = ib[k];
                 v0 += inv * ga[k];
                 v1 += inv * gb[k];
                 v2 += inv * gc[k];
@@ -2114,7 +2178,7 @@ __device__ __forceinline__ double eval_drift_exc(const Tables& t, const QmcParam
 #pragma unroll
     for (int m = 0; m < NM; ++m) mo[m] = gx[m] = gy[m] = gz[m] = T(0);
     MoSink<T, NM, true, T, false> sink{(const T*)prm.entry_w, t.nmo, mo, gx, gy, gz, nullptr};
-    AoGeneric::template row<T, RAD, true, false>(t, prm, x, y, z, sink);
+    AoGeneric::template row<T, RAD, true>(t, prm, x, y, z, sink);
     T jg[3];
     const T kj = jastrow_value_grad<T>(t, prm, L, x, y, z, jg);
     const double logj = (double)seg_sum<T>(kj, L.wbase, t.nelec, t.nelec);
@@ -2158,13 +2222,6 @@ template <typename T, int NM, int RAD, int MC, typename AO = AoGeneric, bool EXC
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NM <= 8 ? 2 : 1))) void hmc_kernel(HArgs a) {
     const WalkerLane L = lane_layout(a.t, a.nw);
     if ((int64_t)L.wave * L.G >= a.nw) return;
-    double* lds;  // row transposes (above 8 rows also the pivot rows), or the exc_gamma rows
-    if constexpr (EXC)
-        lds = (double*)qmc_dyn_lds;
-    else if constexpr (use_minors<NM>())
-        lds = nullptr;
-    else
-        lds = wave_rowbuf<NM>();
     const Tables& t = a.t;
     const int Ne = t.nelec;
     double* pp = a.wk.pos + (size_t)L.wclamp * 3 * Ne + 3 * L.e;
@@ -2186,9 +2243,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NM <= 8 
         double sgn_n, gn[3];
         double lpn;
         if constexpr (EXC)
-            lpn = eval_drift_exc<T, NM, RAD>(t, a.p, L, qx, qy, qz, lds, sgn_n, gn);
+            lpn = eval_drift_exc<T, NM, RAD>(t, a.p, L, qx, qy, qz, (double*)qmc_dyn_lds, sgn_n, gn);
         else
-            lpn = eval_drift<T, NM, RAD, MC, AO>(t, a.p, L, qx, qy, qz, logc0, lds, sgn_n, gn);
+            lpn = eval_drift<T, NM, RAD, MC, AO>(t, a.p, L, qx, qy, qz, logc0, sgn_n, gn);
         if (s >= 0) {
             // momentum update at the new point: full step, or the closing half step
             const double f = (l + 1 < traj) ? 2.0 * eps : eps;  // p -= f/2 grad U, grad U = -2 drift
@@ -2332,31 +2389,17 @@ __device__ __forceinline__ int stage_conf_rows(const Tables& t, const WalkerLane
 
 // log|det| and sign of configuration c of this lane's spin and its inverse
 // column inv[k] = (A_c^-1)[k][this row], zero past the group's n (rows staged
-// by stage_conf_rows).  Above the minors' sizes the lane that pivoted column k
-// of [A | I] holds row k of A^-1, and the transpose goes through the
-// wavefront's row buffer, which then holds A_c^-1 of every group: (k, l) at
-// [(gbase + k) NM + l].
+// by stage_conf_rows).  Returns lane_inverse's column above the minors' sizes.
 template <int NM>
-__device__ __forceinline__ void conf_inverse(const Tables& t, const WalkerLane& L, int c, const double (&mo)[NM],
+__device__ __forceinline__ int conf_inverse(const Tables& t, const WalkerLane& L, int c, const double (&mo)[NM],
                                              int own_ex, double& lg, double& sg, double (&inv)[NM]) {
     if constexpr (use_minors<NM>()) {
         minor_det<NM, true, true>(t, L, wave_minor_rows<NM>(), own_ex, c, lg, sg, inv);
+        return 0;
     } else {
-        double aa[NM], bb[NM], tp;
-        int col;
+        double aa[NM];
         gather_conf<NM>(t, L, c, mo, aa);
-#pragma unroll
-        for (int j = 0; j < NM; ++j) bb[j] = (j == L.myrow) ? 1.0 : 0.0;
-        lane_gj<NM>(L, t.nsig_max, aa, bb, lg, sg, tp, col);
-        double* rb = wave_rowbuf<NM>();
-        wave_lds_sync();  // the elimination's loads come first
-        if (L.lane_real && col >= 0) {
-#pragma unroll
-            for (int j = 0; j < NM; ++j) rb[(L.gbase + col) * NM + j] = bb[j];
-        }
-        wave_lds_sync();
-#pragma unroll
-        for (int k = 0; k < NM; ++k) inv[k] = k < L.n_sig ? rb[(L.gbase + (k < L.n_sig ? k : 0)) * NM + L.myrow] : 0.0;
+        return lane_inverse<NM>(L, t.nsig_max, aa, lg, sg, inv);
     }
 }
 
@@ -2364,10 +2407,11 @@ __device__ __forceinline__ void conf_inverse(const Tables& t, const WalkerLane& 
 // Y_l the inverse column of row l and B_l its kinetic row,
 // zz = sum_l Y_l (B_l . inv).  B_l: row [lane][NM] of brow, column k of the
 // configuration at col(k); Y_l: ycol [lane][NM] (small matrices, written here)
-// or the row buffer left by conf_inverse.
+// or the row buffer left by conf_inverse, whose columns are own_col of the lanes.
 template <int NM, typename Col>
 __device__ __forceinline__ void inverse_b_inverse(const Tables& t, const WalkerLane& L, const double (&inv)[NM],
-                                                  const double* brow, double* ycol, Col col, double (&zz)[NM]) {
+                                                  int own_col, const double* brow, double* ycol, Col col,
+                                                  double (&zz)[NM]) {
     const double* rb = nullptr;
     if constexpr (use_minors<NM>()) {
         wave_lds_sync();  // the previous configuration's loads come first
@@ -2386,9 +2430,10 @@ __device__ __forceinline__ void inverse_b_inverse(const Tables& t, const WalkerL
         for (int k = 0; k < NM; ++k)
             if (k < L.n_sig) tl += brow[lane_l * NM + col(k)] * inv[k];
         if (l >= L.n_sig) tl = 0.0;
+        const int cl = use_minors<NM>() ? 0 : __shfl(own_col, lane_l);
 #pragma unroll
         for (int k = 0; k < NM; ++k)
-            if (k < L.n_sig) zz[k] += tl * (use_minors<NM>() ? ycol[lane_l * NM + k] : rb[k * NM + ll]);
+            if (k < L.n_sig) zz[k] += tl * (use_minors<NM>() ? ycol[lane_l * NM + k] : rb[k * NM + cl]);
     }
 }
 
@@ -2823,10 +2868,10 @@ __global__ __launch_bounds__(kBlock) void eloc_grad_kernel(EArgs a) {
 #pragma unroll 1
     for (int c = 0; c < t.nconf_max; ++c) {
         double lg, sg, inv[NM], zz[NM];
-        conf_inverse<NM>(t, L, c, mo, own_ex, lg, sg, inv);
+        const int oc_ = conf_inverse<NM>(t, L, c, mo, own_ex, lg, sg, inv);
         const int nc = L.spin == 0 ? t.nconf_up : t.nconf_dn, cc = c < nc ? c : nc - 1;
         const QMC_CONST int* cf = L.spin == 0 ? t.conf_up + cc * t.nup : t.conf_dn + cc * t.ndown;
-        inverse_b_inverse<NM>(t, L, inv, brow, ycol, [&](int k) { return t.identity_conf ? k : (int)cf[k]; }, zz);
+        inverse_b_inverse<NM>(t, L, inv, oc_, brow, ycol, [&](int k) { return t.identity_conf ? k : (int)cf[k]; }, zz);
         double rc = 0.0, oc = 0.0;
 #pragma unroll
         for (int c2 = 0; c2 < QMC_MAXCONF; ++c2)

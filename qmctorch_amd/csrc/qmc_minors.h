@@ -23,8 +23,15 @@ namespace qmc {
 // off from an 80-bit elimination by 6.1e-15 / 1.2e-12 (99 % / 99.99 % quantile,
 // relative to E_L) where a pivoted FP64 elimination is off by 9.6e-15 /
 // 3.0e-12; N2: 1.2e-14 / 3.5e-12 against 1.5e-14 / 8.6e-12.  With each lane's
-// own determinant it was 2.8e-14 / 6.8e-12 and 6.9e-14 / 5.8e-11.
+// own determinant it was 2.8e-14 / 6.8e-12 and 6.9e-14 / 5.8e-11.  A block with
+// several small singular values (walkers far outside the molecule) loses more
+// than an elimination does, so FP64 blocks whose determinant, of rows scaled to
+// a largest entry of 1/2 to 1, is below kWeakDet are eliminated instead: 1e-5
+// of the groups above, and the quantiles stay at or below the elimination's
+// for walkers spread two and four times as far.
 constexpr int kMaxMinors = 7;
+
+constexpr double kWeakDet = 1e-6;
 
 template <int I, int E, typename F>
 QMC_MINORS_FN void static_for(F&& f) {

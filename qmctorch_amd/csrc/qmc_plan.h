@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <cstring>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -18,15 +19,37 @@ struct QmcPlan {
     ~QmcPlan() {
         for (void* p : allocs) (void)hipFree(p);
     }
+    // Tables are placed in chunks of device memory through host mirrors, copied
+    // once by upload_done(): an allocation and a copy per table took most of the
+    // plan's creation.
+    struct Chunk {
+        char* dev;
+        size_t size;
+        std::vector<char> host;
+    };
+    std::vector<Chunk> chunks;
     template <typename X>
     const X* upload(const X* host, size_t n) {
         if (n == 0 || host == nullptr) return nullptr;
-        void* d = nullptr;
-        if (hipMalloc(&d, n * sizeof(X)) != hipSuccess) throw std::runtime_error("hipMalloc failed");
-        allocs.push_back(d);
-        if (hipMemcpy(d, host, n * sizeof(X), hipMemcpyHostToDevice) != hipSuccess)
-            throw std::runtime_error("hipMemcpy failed");
-        return (const X*)d;
+        const size_t bytes = n * sizeof(X), kChunk = 256 * 1024, kAlign = 256;
+        if (chunks.empty() || (chunks.back().host.size() + kAlign - 1) / kAlign * kAlign + bytes > chunks.back().size) {
+            const size_t size = bytes > kChunk ? bytes : kChunk;
+            void* d = nullptr;
+            if (hipMalloc(&d, size) != hipSuccess) throw std::runtime_error("hipMalloc failed");
+            allocs.push_back(d);
+            chunks.push_back(Chunk{(char*)d, size, {}});
+        }
+        Chunk& c = chunks.back();
+        const size_t at = (c.host.size() + kAlign - 1) / kAlign * kAlign;
+        c.host.resize(at + bytes);
+        std::memcpy(c.host.data() + at, host, bytes);
+        return (const X*)(c.dev + at);
+    }
+    void upload_done() {
+        for (auto& c : chunks)
+            if (hipMemcpy(c.dev, c.host.data(), c.host.size(), hipMemcpyHostToDevice) != hipSuccess)
+                throw std::runtime_error("hipMemcpy failed");
+        chunks.clear();
     }
 };
 

@@ -68,6 +68,42 @@ def nm_bucket_fine(nmo: int, nup: int, ndown: int) -> int:
     return -1
 
 
+P_POWERS = [0x001, 0x010, 0x100]  # kx | ky << 4 | kz << 8 of x, y, z
+D_POWERS = [0x002, 0x011, 0x101, 0x020, 0x110, 0x200]  # xx xy xz yy yz zz
+
+
+def shells(tab, g: int) -> List[Tuple[int, str, int, float]]:
+    """(first entry, type, r power, d_xy / d_xx ratio) of the shells of group g:
+    the merging of shell_records in qmc_abi.hip."""
+    npr, i, i1 = int(tab.grp_nprim[g]), int(tab.grp_ao0[g]), int(tab.grp_ao0[g] + tab.grp_nao[g])
+    sto = int(tab.radial) == 1
+    K = lambda j: tab.gao_K[j, :npr]
+    rpow = lambda j: int(tab.gao_n[j, 0]) if sto else 0
+    scaled = lambda a, b, f: bool(np.all(np.abs(K(b) - f * K(a)) <= 8e-16 * np.abs(K(b))))
+
+    def matches(i, powers):
+        return i + len(powers) <= i1 and all(int(tab.gao_k[i + j]) == k and rpow(i + j) == rpow(i)
+                                             for j, k in enumerate(powers))
+
+    if sto and any(len(set(tab.gao_n[j, :npr])) > 1 for j in range(i, i1)):
+        raise ValueError("a generated layout needs one r power per entry")
+    out = []
+    while i < i1:
+        if matches(i, P_POWERS) and scaled(i, i + 1, 1.0) and scaled(i, i + 2, 1.0):
+            out.append((i, "P", rpow(i), 0.0))
+            i += 3
+            continue
+        if matches(i, D_POWERS) and K(i)[0] != 0.0:
+            f = float(K(i + 1)[0] / K(i)[0])
+            if scaled(i, i + 3, 1.0) and scaled(i, i + 5, 1.0) and all(scaled(i, i + j, f) for j in (1, 2, 4)):
+                out.append((i, "D", rpow(i), f))
+                i += 6
+                continue
+        out.append((i, "S" if int(tab.gao_k[i]) == 0 else "One", rpow(i), 0.0))
+        i += 1
+    return out
+
+
 def row_source(tab) -> str:
     """Body of AoSpec::row for the layout of ``tab``."""
     lines = ["        const double* ac = prm.atom_coords;"]
@@ -85,41 +121,25 @@ def row_source(tab) -> str:
             p0 = int(tab.grp_prim0[g])
             i0 = int(tab.grp_ao0[g])
             nao = int(tab.grp_nao[g])
-            tight = int(tab.grp_tight[g]) if len(tab.grp_tight) else 0
-
-            def block(T, geo):
-                out = ["%s E[%d], A[%d];" % (T, npr, npr),
-                       "group_prims_from<%s, RAD, %d>(sink.pace(group_exponents<%s>(prm)), %d, %s.r2, %s.r, E, A);"
-                       % (T, npr, T, p0, geo, geo)]
-                for i in range(i0, i0 + nao):
-                    k = int(tab.gao_k[i])
-                    kc = ", ".join(repr(float(v)) for v in tab.gao_K[i, :npr])
-                    nc = ", ".join(repr(float(v)) for v in tab.gao_n[i, :npr])
-                    out.append("{")
-                    out.append("    constexpr double K[%d] = {%s};" % (npr, kc))
-                    out.append("    constexpr double N[%d] = {%s};" % (npr, nc))
-                    out.append("    ao_entry_with<%s, RAD, DERIV, %d>([&](int p) { return (%s)K[p]; }, "
-                               "[&](int p) { return N[p]; }, %d, %d, %d, %d, %d, E, A, %s.dx, %s.dy, %s.dz, "
-                               "%s.r2, %s.r, %s.ir, sink);"
-                               % (T, npr, T, i, int(tab.gao_mu[i]), k & 15, (k >> 4) & 15, (k >> 8) & 15,
-                                  geo, geo, geo, geo, geo, geo))
-                    out.append("}")
-                return out
 
             lines.append("            sink.fence();")
-            lines.append("            // group %d: %d primitives from %d, entries %d..%d%s"
-                         % (g, npr, p0, i0, i0 + nao - 1, ", FP64 in the mixed local energy" if tight else ""))
-            if tight:
-                lines.append("            if (TIGHT) {")
-                lines.append("                const AtomGeo<double> D = atom_geo<double, RAD>(dxd, dyd, dzd);")
-                lines += ["                " + x for x in block("double", "D")]
-                lines.append("            } else {")
-                lines += ["                " + x for x in block("T", "G")]
-                lines.append("            }")
-            else:
-                lines.append("            {")
-                lines += ["                " + x for x in block("T", "G")]
-                lines.append("            }")
+            lines.append("            // group %d: %d primitives from %d, entries %d..%d" % (g, npr, p0, i0, i0 + nao - 1))
+            lines.append("            {")
+            body = ["T E[%d], A[%d];" % (npr, npr),
+                    "group_prims_from<T, RAD, %d>(sink.pace(group_exponents<T>(prm)), %d, G.r2, G.r, E, A);" % (npr, p0)]
+            for i, kind, rpow, ratio in shells(tab, g):
+                k = int(tab.gao_k[i])
+                kc = ", ".join(repr(float(v)) for v in tab.gao_K[i, :npr])
+                body += ["{",
+                         "    constexpr double K[%d] = {%s};" % (npr, kc),
+                         "    T m0, m1, m2;",
+                         "    shell_moments<T, DERIV, %d>([&](int p) { return (T)K[p]; }, E, A, m0, m1, m2);" % npr,
+                         "    const ShellRadial<T> S = shell_radial<T, RAD, DERIV>(m0, m1, m2, %d, G.r2, G.r, G.ir);" % rpow,
+                         "    shell_entries<T, DERIV, kShell%s>(%d, S, G.dx, G.dy, G.dz, T(%r), %d, %d, %d, sink);"
+                         % (kind, i, ratio, k & 15, (k >> 4) & 15, (k >> 8) & 15),
+                         "}"]
+            lines += ["                " + x for x in body]
+            lines.append("            }")
             g += 1
         lines.append("        }")
     return "\n".join(lines)
@@ -135,7 +155,7 @@ namespace {
 struct AoSpec {
     static constexpr int kEntries = %(nentry)d;
     static constexpr int kRowBlocks = %(rowblocks)d;  // 16-lane row blocks holding the catalog molecule's walkers
-    template <typename T, int RAD, bool DERIV, bool TIGHT, typename Sink>
+    template <typename T, int RAD, bool DERIV, typename Sink>
     static __device__ __forceinline__ void row(const Tables& t, const QmcParams& prm, double ex, double ey,
                                                double ez, Sink&& sink) {
 %(body)s
@@ -173,6 +193,21 @@ int spec_%(name)s_hmc(const HArgs& a, int prec, hipStream_t s) {
     hipLaunchKernelGGL((hmc_kernel<float, kNM, kRAD, kMC, AoSpec>), grid_for(a.t, a.nw), dim3(kBlock), 0, s, a);
     return 0;
 }
+
+}  // namespace qmc
+'''
+
+# Layouts up to this many W elements get a generated local-energy kernel: the
+# straight-line row of a larger one (benzene: 120 entries x 24 columns) is
+# executed once per wavefront and waits for its instructions, where the
+# table-driven row is a loop that stays in the instruction cache: E_L of 1021
+# walkers 309 us generated, 180 us table-driven; water (24 entries x 5 columns),
+# 65536 walkers, is fastest with its generated row.
+ELOC_MAX_W = 512
+
+NO_ELOC = '''
+int spec_%(name)s_wf(const KArgs&, int, int, hipStream_t) { return -1; }
+int spec_%(name)s_wf_batch(const WJob*, int, int, int, int, hipStream_t) { return -1; }
 
 }  // namespace qmc
 '''
@@ -246,7 +281,8 @@ def unit_sources(name: str, tab, nm: int, mc: int = 1) -> Dict[str, str]:
     single, batch = sweep_launch(len(tab.gao_mu), nm)
     sweep = SWEEP % dict(name=name, launch=single, launch_batch=batch)
     return {"qmc_spec_%s_sweep.hip" % name: head + sweep,
-            "qmc_spec_%s_eloc.hip" % name: head + ELOC % dict(name=name),
+            "qmc_spec_%s_eloc.hip" % name: head + (ELOC if len(tab.gao_mu) * nm <= ELOC_MAX_W else NO_ELOC) % dict(
+                name=name),
             "qmc_spec_%s_hmc.hip" % name: head + HMC % dict(name=name, mc=mc)}
 
 
