@@ -614,9 +614,9 @@ __device__ __forceinline__ int seg_pivot(int k, bool cand, double v, int myrow, 
 }
 
 // ------------------------------------------------- determinant-only elimination
-// log|det| and sign of the n x n matrix whose row r lives in lane gbase + r,
-// with the row arithmetic of lane_gauss_jordan<NM, false> but fewer cross-lane
-// moves per column:
+// Determinant det 2^ex2 (det 0 or a signed mantissa) of the n x n matrix whose
+// row r lives in lane gbase + r, with the row arithmetic of
+// lane_gauss_jordan<NM, false> but fewer cross-lane moves per column:
 //  * the pivot (largest |a_rk| among the rows not used yet, first one on ties,
 //    compared through seg_pivot's 32-bit keys): up to 8 columns from the n
 //    keys gathered into every lane by shuffles; for the larger buckets by
@@ -633,12 +633,11 @@ __device__ __forceinline__ int seg_pivot(int k, bool cand, double v, int myrow, 
 // still to be eliminated are written.
 template <int NM>
 __device__ __forceinline__ void lane_det_lds(double (&a)[NM], int n, int nmax, int myrow, int gbase, int spin,
-                                             uint64_t gmask, bool may_store, double* rowbuf, double& logdet,
-                                             double& sgn) {
+                                             uint64_t gmask, bool may_store, double* rowbuf, double& det, int& ex2) {
     if constexpr (NM > 8) seg_pivot_init(myrow, gbase, may_store);
     double* const recip = det_recips() + gbase;  // the group's pivot reciprocal
     bool done = false;
-    sgn = 1.0;
+    double sgn = 1.0;
     int inversions = 0;
     bool singular = false;
     double mant = 1.0;  // |det| = mant * 2^expo, renormalised after every pivot
@@ -727,7 +726,8 @@ __device__ __forceinline__ void lane_det_lds(double (&a)[NM], int n, int nmax, i
         }
     }
     if (inversions & 1) sgn = -sgn;
-    logdet = singular ? -INFINITY : log_mantissa(mant) + 0.6931471805599453 * (double)expo;
+    det = singular ? 0.0 : sgn * mant;
+    ex2 = expo;
 }
 
 // ------------------------------------------------------ in-place inverse (LDS)
@@ -735,19 +735,19 @@ __device__ __forceinline__ void lane_det_lds(double (&a)[NM], int n, int nmax, i
 // gbase + r, in the NM registers of the row: after the step of column k with
 // pivot row p, storage column k holds the inverse's column of row p.  On exit
 // the lane that pivoted column k (my_col = k) holds row k of A^-1 with the
-// entry of row i in storage column (my_col of row i's lane); log|det| and sign
-// as lane_det_lds, pivots chosen by seg_pivot.  NM multiply-adds per column and
+// entry of row i in storage column (my_col of row i's lane); det and ex2 as
+// lane_det_lds, pivots chosen by seg_pivot.  NM multiply-adds per column and
 // row, where eliminating [A | I] or [A | B] took up to 2 NM and twice the
 // registers.  rowbuf: the group's row buffer (NM doubles used).
 template <int NM>
 __device__ __forceinline__ void lane_invert_lds(double (&a)[NM], int n, int nmax, int myrow, int gbase,
-                                                uint64_t gmask, bool may_store, double* rowbuf, double& logdet,
-                                                double& sgn, int& my_col) {
+                                                uint64_t gmask, bool may_store, double* rowbuf, double& det,
+                                                int& ex2, int& my_col) {
     seg_pivot_init(myrow, gbase, may_store);
     double* const pivot = det_recips() + gbase;  // the column's pivot
     bool done = false;
     my_col = -1;
-    sgn = 1.0;
+    double sgn = 1.0;
     int inversions = 0;
     bool singular = false;
     double mant = 1.0;  // |det| = mant * 2^expo, renormalised after every pivot
@@ -798,7 +798,8 @@ __device__ __forceinline__ void lane_invert_lds(double (&a)[NM], int n, int nmax
         }
     }
     if (inversions & 1) sgn = -sgn;
-    logdet = singular ? -INFINITY : log_mantissa(mant) + 0.6931471805599453 * (double)expo;
+    det = singular ? 0.0 : sgn * mant;
+    ex2 = expo;
 }
 
 }  // namespace qmc

@@ -612,15 +612,15 @@ __device__ __forceinline__ double* det_rowbuf(const WalkerLane& L) {
 }
 
 // Column of the inverse for this lane's row, inv[k] = (A^-1)[k][row] (zero past
-// the group's n), log|det A| and its sign, of the group matrix whose rows are
+// the group's n), and det A = d 2^ex, of the group matrix whose rows are
 // the lanes' a (destroyed): the in-place inversion, then a transpose through the
 // wavefront's row buffer, which afterwards holds A^-1 of every group: entry
 // (k, row of lane l) at [(gbase + k) NM + the lane's returned column].
 template <int NM>
-__device__ __forceinline__ int lane_inverse(const WalkerLane& L, int nmax, double (&a)[NM], double& lg, double& sg,
+__device__ __forceinline__ int lane_inverse(const WalkerLane& L, int nmax, double (&a)[NM], double& d, int& ex,
                                             double (&inv)[NM]) {
     int col;
-    lane_invert_lds<NM>(a, L.n_sig, nmax, L.myrow, L.gbase, L.gmask, L.lane_real, det_rowbuf<NM>(L), lg, sg, col);
+    lane_invert_lds<NM>(a, L.n_sig, nmax, L.myrow, L.gbase, L.gmask, L.lane_real, det_rowbuf<NM>(L), d, ex, col);
     double* rb = wave_rowbuf<NM>();
     wave_lds_sync();  // the elimination's loads come first
     if (L.lane_real && col >= 0) {
@@ -732,38 +732,37 @@ __device__ __forceinline__ double log_abs_product(double d1, double d2, int ex) 
     return (d1 == 0.0 || d2 == 0.0) ? -INFINITY : l;
 }
 
-// Configuration c of this lane's spin from the staged rows: log|det|, its sign
-// and (INV) y[k] = (A_c^-1)[k][this row], the coefficient of configuration
+// Configuration c of this lane's spin from the staged rows: its determinant
+// d 2^ex and (INV) y[k] = (A_c^-1)[k][this row], the coefficient of configuration
 // column k, zero past the group's n.  own_ex: this lane's row exponent.
 template <int N, int NM, bool SCALE, bool INV, typename Col>
 __device__ __forceinline__ void minor_det_n(const WalkerLane& L, const double* rows, int own_ex, int nmax, Col col,
-                                            double& lg, double& sg, double (&y)[NM]) {
+                                            double& d, int& ex, double (&y)[NM]) {
     double a[N], c[N];
     bool flip;
-    int ex;
     group_cofactors<N, NM, SCALE>(L, rows, col, a, c, flip, ex);
-    double d = 0.0;
+    ex += own_ex;
+    d = 0.0;
 #pragma unroll
     for (int k = 0; k < N; ++k) d = fma(a[k], c[k], d);
     // one determinant for the group (qmc_minors.h): its first lane's
-    const double D = __shfl(flip ? -d : d, L.gbase);
-    lg = log_abs_product(D, 1.0, ex + own_ex);
-    sg = D < 0.0 ? -1.0 : 1.0;
+    d = __shfl(flip ? -d : d, L.gbase);
     if constexpr (INV) {
-        const double id = ldexp(1.0 / (flip ? -D : D), -own_ex);
+        const double id = ldexp(1.0 / (flip ? -d : d), -own_ex);
 #pragma unroll
         for (int k = 0; k < NM; ++k) y[k] = k < N ? c[k < N ? k : 0] * id : 0.0;
     }
     if constexpr (SCALE) {
-        const bool weak = !(fabs(D) >= kWeakDet);
+        const bool weak = !(fabs(d) >= kWeakDet);
         if (__any(weak && L.lane_real)) {  // eliminate (qmc_minors.h)
-            double aw[NM], inv[NM], lw, sw;
+            double aw[NM], inv[NM], dw;
+            int ew;
 #pragma unroll
             for (int k = 0; k < NM; ++k) aw[k] = k < N ? a[k < N ? k : 0] : 0.0;
-            lane_inverse<NM>(L, nmax, aw, lw, sw, inv);
+            lane_inverse<NM>(L, nmax, aw, dw, ew, inv);
             if (weak) {
-                lg = lw + 0.6931471805599453 * (double)(ex + own_ex);
-                sg = sw;
+                d = dw;
+                ex += ew;
                 if constexpr (INV) {
 #pragma unroll
                     for (int k = 0; k < NM; ++k) y[k] = ldexp(inv[k], -own_ex);
@@ -775,9 +774,9 @@ __device__ __forceinline__ void minor_det_n(const WalkerLane& L, const double* r
 
 template <int NM, bool SCALE, bool INV>
 __device__ __forceinline__ void minor_det(const Tables& t, const WalkerLane& L, const double* rows, int own_ex, int c,
-                                          double& lg, double& sg, double (&y)[NM]) {
+                                          double& d, int& ex, double (&y)[NM]) {
     if (t.identity_conf) {
-        minor_det_n<NM, NM, SCALE, INV>(L, rows, own_ex, t.nsig_max, [](int k) { return k; }, lg, sg, y);
+        minor_det_n<NM, NM, SCALE, INV>(L, rows, own_ex, t.nsig_max, [](int k) { return k; }, d, ex, y);
         return;
     }
     const int nconf = L.spin == 0 ? t.nconf_up : t.nconf_dn;
@@ -788,13 +787,16 @@ __device__ __forceinline__ void minor_det(const Tables& t, const WalkerLane& L, 
     auto col = [&](int k) { return (int)conf[k < L.n_sig ? k : 0]; };
     static_for<1, NM + 1>([&](auto nc) {
         constexpr int N = decltype(nc)::value;
-        if (t.nsig_max == N) minor_det_n<N, NM, SCALE, INV>(L, rows, own_ex, N, col, lg, sg, y);
+        if (t.nsig_max == N) minor_det_n<N, NM, SCALE, INV>(L, rows, own_ex, N, col, d, ex, y);
     });
 }
 
 // Single configuration, single CI term: log|D_up D_dn| and its sign in every
 // lane, and (INV) this lane's inverse column y; ksum: the sum of kj over the
 // walker's lanes, in lane order, exchanged together with the rows.
+__device__ __forceinline__ void single_product(const Tables& t, const WalkerLane& L, double d, int ex, double logc0,
+                                               double c0, double& logabs, double& sgn);
+
 template <int NM, bool INV, typename T, typename KT>
 __device__ __forceinline__ void slater_single_minors(const Tables& t, const QmcParams& prm, const WalkerLane& L,
                                                      const T (&mo)[NM], double logc0, KT kj, double& logabs,
@@ -840,37 +842,40 @@ __device__ __forceinline__ void slater_single_minors(const Tables& t, const QmcP
         const double D = L.spin == 0 ? du : dd;
         const bool weak = !(fabs(D) >= kWeakDet);
         if (__any(weak && L.lane_real)) {  // eliminate (qmc_minors.h)
-            double inv[NM], lw, sw;
-            lane_inverse<NM>(L, t.nsig_max, a, lw, sw, inv);
+            double inv[NM], dw;
+            int ew;
+            lane_inverse<NM>(L, t.nsig_max, a, dw, ew, inv);
             if constexpr (INV) {
 #pragma unroll
                 for (int k = 0; k < NM; ++k) y[k] = weak ? ldexp(inv[k], -own_ex) : y[k];
             }
-            const double lg = weak ? lw + 0.6931471805599453 * (double)ex : log_abs_product(D, 1.0, ex);
-            const double sg = weak ? sw : (D < 0.0 ? -1.0 : 1.0);
-            const double lu = __shfl(lg, L.wbase), ld = __shfl(lg, dn_lane);
-            const double su = __shfl(sg, L.wbase), sd = __shfl(sg, dn_lane);
-            logabs = lu + (t.ndown > 0 ? ld : 0.0) + logc0;
-            sgn = su * (t.ndown > 0 ? sd : 1.0) * (c0 < 0.0 ? -1.0 : 1.0);
+            single_product(t, L, weak ? dw : D, weak ? ex + ew : ex, logc0, c0, logabs, sgn);
         }
     }
+}
+
+// log|c0 D_up D_dn| and its sign in every lane, from the groups' determinants
+// d 2^ex (one logarithm for the product).
+__device__ __forceinline__ void single_product(const Tables& t, const WalkerLane& L, double d, int ex, double logc0,
+                                               double c0, double& logabs, double& sgn) {
+    const int dn_lane = L.wbase + (t.ndown > 0 ? t.nup : 0);
+    const double du = __shfl(d, L.wbase), dd_ = __shfl(d, dn_lane);
+    const int eu = __shfl(ex, L.wbase), ed = __shfl(ex, dn_lane);
+    const double dd = t.ndown > 0 ? dd_ : 1.0;
+    logabs = log_abs_product(du, dd, eu + (t.ndown > 0 ? ed : 0)) + logc0;
+    sgn = (((du < 0.0) != (dd < 0.0)) != (c0 < 0.0)) ? -1.0 : 1.0;
 }
 
 // Single configuration, single CI term: log|D_up D_dn| and its sign (ground state).
 template <int NM, typename T>
 __device__ __forceinline__ void slater_single(const Tables& t, const QmcParams& prm, const WalkerLane& L,
                                               const T (&mo)[NM], double logc0, double& logabs, double& sgn) {
-    double a[NM];
+    double a[NM], d;
+    int ex;
 #pragma unroll
     for (int j = 0; j < NM; ++j) a[j] = (double)mo[j];
-    double lg, sg;
-    lane_det_lds<NM>(a, L.n_sig, t.nsig_max, L.myrow, L.gbase, L.spin, L.gmask, L.lane_real, det_rowbuf<NM>(L), lg, sg);
-    const int dn_lane = L.wbase + (t.ndown > 0 ? t.nup : 0);
-    const double lu = __shfl(lg, L.wbase), su = __shfl(sg, L.wbase);
-    const double ldn = __shfl(lg, dn_lane), sdn = __shfl(sg, dn_lane);
-    const double c0 = ldc(prm.ci, 0);
-    logabs = lu + (t.ndown > 0 ? ldn : 0.0) + logc0;
-    sgn = su * (t.ndown > 0 ? sdn : 1.0) * (c0 < 0.0 ? -1.0 : 1.0);
+    lane_det_lds<NM>(a, L.n_sig, t.nsig_max, L.myrow, L.gbase, L.spin, L.gmask, L.lane_real, det_rowbuf<NM>(L), d, ex);
+    single_product(t, L, d, ex, logc0, ldc(prm.ci, 0), logabs, sgn);
 }
 
 // slater_single with the kinetic ratio tr(A^-1 B), each lane's share of it the
@@ -879,19 +884,16 @@ template <int NM>
 __device__ __forceinline__ void slater_single_kin(const Tables& t, const QmcParams& prm, const WalkerLane& L,
                                                   const double (&mo)[NM], const double (&bk)[NM], double& logabs,
                                                   double& sgn, double& kin) {
-    double a[NM], inv[NM], lg, sg, tp = 0.0;
+    double a[NM], inv[NM], d, tp = 0.0;
+    int ex;
 #pragma unroll
     for (int j = 0; j < NM; ++j) a[j] = mo[j];
-    lane_inverse<NM>(L, t.nsig_max, a, lg, sg, inv);
+    lane_inverse<NM>(L, t.nsig_max, a, d, ex, inv);
 #pragma unroll
     for (int k = 0; k < NM; ++k) tp += k < L.n_sig ? bk[k] * inv[k] : 0.0;
     kin = seg_sum(tp, L.wbase, t.nelec, t.nelec);
-    const int dn_lane = L.wbase + (t.ndown > 0 ? t.nup : 0);
-    const double lu = __shfl(lg, L.wbase), su = __shfl(sg, L.wbase);
-    const double ldn = __shfl(lg, dn_lane), sdn = __shfl(sg, dn_lane);
     const double c0 = ldc(prm.ci, 0);
-    logabs = lu + (t.ndown > 0 ? ldn : 0.0) + log(fabs(c0));
-    sgn = su * (t.ndown > 0 ? sdn : 1.0) * (c0 < 0.0 ? -1.0 : 1.0);
+    single_product(t, L, d, ex, log(fabs(c0)), c0, logabs, sgn);
 }
 
 // Gather row entries of configuration c from an MO-like row (uniform c).
@@ -924,116 +926,98 @@ __device__ __forceinline__ void gather_conf(const Tables& t, const WalkerLane& L
 // first lane (slater_pooling.py:64-111, 262-409; slater_jastrow.py:312-344).
 // Returns log|sum_n c_n D_n| and its sign in every lane of the walker, and the
 // Jacobi kinetic ratio sum_n c_n (tr_up + tr_dn) D_n / sum_n c_n D_n.
+// The groups' determinants d 2^ex and traces meet in a wave-local LDS table
+// ([configuration][group's first lane]), which every lane of a walker reads per
+// CI term: two products a term and one logarithm for the sum, instead of a
+// logarithm per configuration, an exponential per term and an eight-way
+// register selection per read: LiH in a Slater basis, four determinants,
+// FP64, 1000 walkers x 100 steps, 1243 -> 872 us.  The configurations of minors
+// share ex (their row scales) unless one was weak; otherwise, and for eliminated
+// blocks, the terms are taken relative to the largest power of two among them,
+// so that no ratio of determinants leaves the range.
 template <int NM, bool KIN, typename T>
 __device__ __forceinline__ void slater_combine(const Tables& t, const QmcParams& prm, const WalkerLane& L,
                                                const T (&mo)[NM], const double (&bk)[NM], double& logabs,
                                                double& sgn, double& kin) {
-    double ld[QMC_MAXCONF], sd[QMC_MAXCONF], td[QMC_MAXCONF];
-#pragma unroll
-    for (int c = 0; c < QMC_MAXCONF; ++c) {
-        ld[c] = 0.0;
-        sd[c] = 1.0;
-        td[c] = 0.0;
-    }
+    __shared__ double dsh[kBlockWaves * QMC_MAXCONF * 64], tsh[KIN ? kBlockWaves * QMC_MAXCONF * 64 : 1];
+    __shared__ int esh[kBlockWaves * QMC_MAXCONF * 64];
+    double* dt = dsh + (threadIdx.x >> 6) * QMC_MAXCONF * 64;
+    int* et = esh + (threadIdx.x >> 6) * QMC_MAXCONF * 64;
+    double* tt = KIN ? tsh + (threadIdx.x >> 6) * QMC_MAXCONF * 64 : nullptr;
     constexpr bool SCALE = std::is_same<T, double>::value;
     double* rows = nullptr;
-    int own_ex = 0;
+    int own_ex = 0, eref = 0;
+    bool common = true;
+    wave_lds_sync();  // the previous evaluation's loads come first
     if constexpr (use_minors<NM>()) {
         rows = wave_minor_rows<NM>();
-        wave_lds_sync();  // the previous evaluation's loads come first
         own_ex = stage_minor_row<NM, SCALE>(L, mo, minors_full<NM>(t), rows);
         wave_lds_sync();
     }
 #pragma unroll 1
     for (int c = 0; c < t.nconf_max; ++c) {
-        double a[NM], b[NM];
-        double lg, sg, tp = 0.0;
+        double a[NM], d, tp = 0.0;
+        int ex;
         if constexpr (use_minors<NM>()) {
-            minor_det<NM, SCALE, KIN>(t, L, rows, own_ex, c, lg, sg, a);
-            if constexpr (KIN) {
-                gather_conf<NM>(t, L, c, bk, b);
-#pragma unroll
-                for (int k = 0; k < NM; ++k) tp += k < L.n_sig ? b[k] * a[k] : 0.0;
-            }
+            minor_det<NM, SCALE, KIN>(t, L, rows, own_ex, c, d, ex, a);
         } else if constexpr (!KIN) {
             gather_conf<NM>(t, L, c, mo, a);
             lane_det_lds<NM>(a, L.n_sig, t.nsig_max, L.myrow, L.gbase, L.spin, L.gmask, L.lane_real,
-                             det_rowbuf<NM>(L), lg, sg);
+                             det_rowbuf<NM>(L), d, ex);
         } else {
-            double inv[NM];
-            gather_conf<NM>(t, L, c, mo, a);
-            lane_inverse<NM>(L, t.nsig_max, a, lg, sg, inv);
+            double r[NM];
+            gather_conf<NM>(t, L, c, mo, r);
+            lane_inverse<NM>(L, t.nsig_max, r, d, ex, a);
+        }
+        if (c == 0) eref = ex;
+        common = common && ex == eref;
+        const bool first = L.lane_real && L.myrow == 0;
+        if (first) {
+            dt[c * 64 + L.lane] = d;
+            et[c * 64 + L.lane] = ex;
+        }
+        if constexpr (KIN) {
+            double b[NM];
             gather_conf<NM>(t, L, c, bk, b);
 #pragma unroll
-            for (int k = 0; k < NM; ++k) tp += k < L.n_sig ? b[k] * inv[k] : 0.0;
-        }
-        const double tr = KIN ? seg_sum(tp, L.gbase, L.n_sig, t.nsig_max) : 0.0;
-#pragma unroll
-        for (int c2 = 0; c2 < QMC_MAXCONF; ++c2) {
-            if (c2 == c) {
-                ld[c2] = lg;
-                sd[c2] = sg;
-                td[c2] = tr;
-            }
+            for (int k = 0; k < NM; ++k) tp += k < L.n_sig ? b[k] * a[k] : 0.0;
+            const double tr = seg_sum(tp, L.gbase, L.n_sig, t.nsig_max);
+            if (first) tt[c * 64 + L.lane] = tr;
         }
     }
-    // exchange: every lane fetches the up values (lane wbase) and the down
-    // values (lane wbase + nup) of its walker
+    wave_lds_sync();
     const int up_lane = L.wbase, dn_lane = L.wbase + (t.ndown > 0 ? t.nup : 0);
-    double lu[QMC_MAXCONF], su[QMC_MAXCONF], tu[QMC_MAXCONF];
-    double lo[QMC_MAXCONF], so[QMC_MAXCONF], to[QMC_MAXCONF];
-#pragma unroll
-    for (int c = 0; c < QMC_MAXCONF; ++c) {
-        if (c < t.nconf_max) {
-            lu[c] = __shfl(ld[c], up_lane);
-            su[c] = __shfl(sd[c], up_lane);
-            lo[c] = __shfl(ld[c], dn_lane);
-            so[c] = __shfl(sd[c], dn_lane);
-            if (KIN) {
-                tu[c] = __shfl(td[c], up_lane);
-                to[c] = __shfl(td[c], dn_lane);
-            }
-        }
-        if (t.ndown == 0) {
-            lo[c] = 0.0;
-            so[c] = 1.0;
-            to[c] = 0.0;
-        }
-    }
-    double lmax = -INFINITY;
-    for (int n = 0; n < t.nci; ++n) {
-        const int cu = t.ci_up[n], cd = t.ci_dn[n];
-        double l = 0.0;
-#pragma unroll
-        for (int c = 0; c < QMC_MAXCONF; ++c) {
-            if (c == cu) l += lu[c];
-            if (c == cd) l += lo[c];
-        }
-        lmax = fmax(lmax, l);
-    }
-    if (!(lmax > -INFINITY)) lmax = 0.0;
+    const bool down = t.ndown > 0;
+    int emax = et[up_lane] + (down ? et[dn_lane] : 0);
     double s = 0.0, st = 0.0;
-    for (int n = 0; n < t.nci; ++n) {
-        const int cu = t.ci_up[n], cd = t.ci_dn[n];
-        double l = 0.0, sg = 1.0, tr = 0.0;
-#pragma unroll
-        for (int c = 0; c < QMC_MAXCONF; ++c) {
-            if (c == cu) {
-                l += lu[c];
-                sg *= su[c];
-                if (KIN) tr += tu[c];
-            }
-            if (c == cd) {
-                l += lo[c];
-                sg *= so[c];
-                if (KIN) tr += to[c];
-            }
-        }
-        const double dn = ldc(prm.ci, n) * sg * exp(l - lmax);
+    auto add = [&](int iu, int id, double dn) {
         s += dn;
-        if (KIN) st += tr * dn;
+        if constexpr (KIN) {
+            const double td = tt[id];
+            st += dn * (tt[iu] + (down ? td : 0.0));
+        }
+    };
+    if (!__any(!common && L.lane_real)) {
+#pragma unroll 4
+        for (int n = 0; n < t.nci; ++n) {
+            const int iu = t.ci_up[n] * 64 + up_lane, id = t.ci_dn[n] * 64 + dn_lane;
+            const double dd = dt[id];
+            add(iu, id, ldc(prm.ci, n) * dt[iu] * (down ? dd : 1.0));
+        }
+    } else {
+        emax = -(1 << 30);
+        for (int n = 0; n < t.nci; ++n) {
+            const int iu = t.ci_up[n] * 64 + up_lane, id = t.ci_dn[n] * 64 + dn_lane;
+            const bool zero = dt[iu] == 0.0 || (down && dt[id] == 0.0);
+            emax = zero ? emax : max(emax, et[iu] + (down ? et[id] : 0));
+        }
+        for (int n = 0; n < t.nci; ++n) {
+            const int iu = t.ci_up[n] * 64 + up_lane, id = t.ci_dn[n] * 64 + dn_lane;
+            const double dd = dt[id];
+            add(iu, id, ldexp(ldc(prm.ci, n) * dt[iu] * (down ? dd : 1.0), et[iu] + (down ? et[id] : 0) - emax));
+        }
     }
-    logabs = lmax + log(fabs(s));
+    logabs = log_abs_product(s, 1.0, emax);
     sgn = s < 0.0 ? -1.0 : 1.0;
     kin = KIN ? st / s : 0.0;
 }
@@ -2060,18 +2044,19 @@ __device__ __forceinline__ double eval_drift(const Tables& t, const QmcParams& p
     }
 #pragma unroll 1
     for (int c = 0; c < t.nconf_max; ++c) {
-        double aa[NM], ib[NM];
-        double lg, sg;
+        double aa[NM], ib[NM], d;
+        int ex;
         if constexpr (use_minors<NM>()) {
-            minor_det<NM, SCALE, true>(t, L, rows, own_ex, c, lg, sg, ib);
+            minor_det<NM, SCALE, true>(t, L, rows, own_ex, c, d, ex, ib);
         } else {
             gather_conf<NM>(t, L, c, mo, aa);
-            lane_inverse<NM>(L, t.nsig_max, aa, lg, sg, ib);
+            lane_inverse<NM>(L, t.nsig_max, aa, d, ex, ib);
         }
         double ga[NM], gb[NM], gc[NM];
         gather_conf<NM>(t, L, c, gx, ga);
         gather_conf<NM>(t, L, c, gy, gb);
         gather_conf<NM>(t, L, c, gz, gc);
+        const double lg = log_abs_product(d, 1.0, ex), sg = d < 0.0 ? -1.0 : 1.0;
         double v0 = 0.0, v1 = 0.0, v2 = 0.0;
 #pragma unroll
         for (int k = 0; k < NM; ++k) {
@@ -2393,14 +2378,18 @@ __device__ __forceinline__ int stage_conf_rows(const Tables& t, const WalkerLane
 template <int NM>
 __device__ __forceinline__ int conf_inverse(const Tables& t, const WalkerLane& L, int c, const double (&mo)[NM],
                                              int own_ex, double& lg, double& sg, double (&inv)[NM]) {
+    double d;
+    int ex, col = 0;
     if constexpr (use_minors<NM>()) {
-        minor_det<NM, true, true>(t, L, wave_minor_rows<NM>(), own_ex, c, lg, sg, inv);
-        return 0;
+        minor_det<NM, true, true>(t, L, wave_minor_rows<NM>(), own_ex, c, d, ex, inv);
     } else {
         double aa[NM];
         gather_conf<NM>(t, L, c, mo, aa);
-        return lane_inverse<NM>(L, t.nsig_max, aa, lg, sg, inv);
+        col = lane_inverse<NM>(L, t.nsig_max, aa, d, ex, inv);
     }
+    lg = log_abs_product(d, 1.0, ex);
+    sg = d < 0.0 ? -1.0 : 1.0;
+    return col;
 }
 
 // zz = column of A^-1 B A^-1 for this lane's row, inv its column of A^-1: with
@@ -2449,12 +2438,18 @@ __device__ __forceinline__ void conf_dets(const Tables& t, const WalkerLane& L, 
         double aa[NM], lg, sg;
         if constexpr (INV) {
             conf_inverse<NM>(t, L, c, mo, own_ex, lg, sg, aa);
-        } else if constexpr (use_minors<NM>()) {
-            minor_det<NM, true, false>(t, L, wave_minor_rows<NM>(), own_ex, c, lg, sg, aa);
         } else {
-            gather_conf<NM>(t, L, c, mo, aa);
-            lane_det_lds<NM>(aa, L.n_sig, t.nsig_max, L.myrow, L.gbase, L.spin, L.gmask, L.lane_real,
-                             det_rowbuf<NM>(L), lg, sg);
+            double d;
+            int ex;
+            if constexpr (use_minors<NM>()) {
+                minor_det<NM, true, false>(t, L, wave_minor_rows<NM>(), own_ex, c, d, ex, aa);
+            } else {
+                gather_conf<NM>(t, L, c, mo, aa);
+                lane_det_lds<NM>(aa, L.n_sig, t.nsig_max, L.myrow, L.gbase, L.spin, L.gmask, L.lane_real,
+                                 det_rowbuf<NM>(L), d, ex);
+            }
+            lg = log_abs_product(d, 1.0, ex);
+            sg = d < 0.0 ? -1.0 : 1.0;
         }
 #pragma unroll
         for (int c2 = 0; c2 < QMC_MAXCONF; ++c2)

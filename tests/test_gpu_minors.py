@@ -69,3 +69,44 @@ def test_rows_far_from_the_nuclei(n):
     ok = bound < 1e-3  # the others' determinants have no correct digits in double
     assert int(ok.sum()) >= 20
     assert ((la.cpu() - ref).abs() <= bound)[ok].all() and torch.equal(sg.cpu()[ok], (su * sd)[ok])
+
+
+@pytest.mark.parametrize("n", [6, 8, 16])
+def test_ci_terms_far_from_the_nuclei(n):
+    """The configurations' determinants, all below the double range and of
+    different powers of two (at n = 16 eliminated, with one exponent each), meet in
+    the CI sum without leaving it."""
+    print("case minors CI far H%d" % n, flush=True)
+    mol = _chain(n)
+    wf, orc = helpers.make_pair(mol, configs="cas(2,2)", w_ee=1.0, w_en=1.0)
+    ci = torch.linspace(1.0, 0.1, wf.nci, dtype=torch.float64)
+    with torch.no_grad():
+        wf.fc.weight.copy_(ci.view(1, -1))
+    rng = np.random.default_rng(n)
+    d = rng.standard_normal((33, n, 3))
+    d *= 40.0 / np.linalg.norm(d, axis=2, keepdims=True)
+    pos = torch.as_tensor((d + np.asarray(mol.atom_coords)[None]).reshape(33, 3 * n))
+    la, sg = wf.log_psi(pos.cuda())
+    mo = orc.mo(orc.ao(pos)).detach()
+    scale = mo.abs().amax(-1, keepdim=True)
+    rows = mo / scale
+    lg, s, cond = [], [], 0.0
+    for cu, cd in zip(*wf.configs):
+        up, dn = rows[:, :mol.nup][..., cu.long()], rows[:, mol.nup:][..., cd.long()]
+        (su, lu), (sd, ld) = torch.linalg.slogdet(up), torch.linalg.slogdet(dn)
+        lg.append(lu + ld)
+        s.append(su * sd)
+        cond = cond + torch.linalg.cond(up) + torch.linalg.cond(dn)
+    lg, s = torch.stack(lg, 1), torch.stack(s, 1)
+    top = lg.amax(1, keepdim=True)
+    terms = ci * s * (lg - top).exp()
+    tot = terms.sum(1)
+    ref = tot.abs().log() + top.view(-1) + scale.log().sum((1, 2)) + orc.jastrow(pos).detach().view(-1).log()
+    assert float(ref.max()) < -745.0
+    # as above, carried through each determinant and a sum that may cancel
+    bound = 5e-14 * n * cond * terms.abs().sum(1) / tot.abs()
+    ok = bound < 1e-3
+    print("  log|psi| from %.0f to %.0f, %d walkers compared, largest difference %.1e"
+          % (ref.min(), ref.max(), int(ok.sum()), (la.cpu() - ref).abs()[ok].max()), flush=True)
+    assert int(ok.sum()) >= 5
+    assert ((la.cpu() - ref).abs() <= bound)[ok].all() and torch.equal(sg.cpu()[ok], tot.sign()[ok])
