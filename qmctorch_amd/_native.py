@@ -209,6 +209,8 @@ class NativeLibraryMissing(RuntimeError):
 def load(path: str = LIBPATH):
     """Load the library (once).  Raises if it is not built."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib
@@ -239,7 +241,9 @@ def ptr(t) -> int:
 
 
 def current_stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """hipStream_t of torch's current stream on the current device (without the
+    Stream object that torch.cuda.current_stream builds: 0.3 us a call, 4 us with it)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def require_device(t: torch.Tensor, what: str = "input") -> None:

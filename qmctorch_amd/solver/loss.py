@@ -19,9 +19,11 @@ class Loss(nn.Module):
     def forward(self, pos: torch.Tensor, no_grad: bool = False, deactivate_weight: bool = False):
         with (torch.no_grad() if no_grad else torch.enable_grad()):
             local_energies = self.wf.local_energy_autodiff(pos)
-            mask = self.get_clipping_mask(local_energies)
             weight = self.get_sampling_weights(pos, deactivate_weight)
-            loss = self.loss_fn((weight * local_energies)[mask])
+            weighted = weight * local_energies
+            if self.clip:  # a boolean selection waits for the device to count its elements
+                weighted = weighted[self.get_clipping_mask(local_energies)]
+            loss = self.loss_fn(weighted)
         return loss, local_energies
 
     def get_clipping_mask(self, local_energies: torch.Tensor) -> torch.Tensor:

@@ -174,15 +174,14 @@ class Solver(SolverBase):
         # parameter gradients do not need d psi / d x, so it is not formed
         psi = self.wf(lpos.detach())
         norm = 1.0 / len(psi)
-        weight = eloc.clone()
-        weight -= torch.mean(eloc)
-        weight /= psi.detach().clone()
+        energy = torch.mean(eloc)
+        weight = eloc - energy
+        weight /= psi.detach()
         weight *= 2.0 * norm
-        clip_mask = self.loss.get_clipping_mask(eloc)
         if self.loss.clip:
-            weight = weight * clip_mask
+            weight = weight * self.loss.get_clipping_mask(eloc)
         psi.backward(weight)
-        return torch.mean(eloc), eloc
+        return energy, eloc
 
     def log_data_opt(self, nepoch, task):
         log.info("")

@@ -42,4 +42,4 @@ def f64(t: torch.Tensor) -> torch.Tensor:
     t = t.detach()
     if t.dtype != torch.float64:
         t = t.to(torch.float64)
-    return t.contiguous()
+    return t if t.is_contiguous() else t.contiguous()

@@ -160,31 +160,34 @@ class SlaterJastrow(WaveFunction):
         self._plan_key = key
         return self._plan
 
-    def _params(self, precision: str):
+    def _params(self, precision: str, plan: Optional[DevicePlan] = None):
         """Parameter views handed to the kernels: one gather launch refreshes W
         and the grouped exponents from the live parameters; the remaining
-        pointers are the parameters themselves (float64)."""
+        pointers are the parameters themselves (float64).  ``plan`` is the
+        caller's device_plan(), if it has just taken it."""
         ee, en = self._jastrow_terms()
-        plan = self.device_plan()
-        mod = f64(self.mo.mo_modifier)
+        if plan is None:
+            plan = self.device_plan()
+        mo, ao = self.mo, self.ao
+        mod = f64(mo.mo_modifier)
         dev = mod.device
         pv = getattr(self, "_pviews", None)
         if pv is None or pv.plan is not plan or pv.mo_w64.device != dev:
             pv = self._pviews = ParamViews(plan, dev)
-        mo_scf = self.mo.mo_scf  # a constant of the MO layer (not a parameter)
+        mo_scf = mo.mo_scf  # a constant of the MO layer (not a parameter)
         if mo_scf.device != dev or mo_scf.dtype != torch.float64 or not mo_scf.is_contiguous():
             c = getattr(self, "_mo_scf64", None)
             if c is None or c.device != dev or c.shape != mo_scf.shape:
                 c = self._mo_scf64 = mo_scf.to(dev, torch.float64).contiguous()
             mo_scf = c
-        bas_exp = f64(self.ao.bas_exp)
+        bas_exp = f64(ao.bas_exp)
         pv.gather(mo_scf, mod, bas_exp)
         mixed = precision == "mixed"
         keep = {
             "mo_modifier": mod,
             "bas_exp": bas_exp,
-            "atom_coords": f64(self.ao.atom_coords),
-            "ci": f64(self.fc.weight).reshape(-1),
+            "atom_coords": f64(ao.atom_coords),
+            "ci": f64(self.fc.weight),
             "w_ee": f64(ee.jastrow_kernel.weight) if ee is not None else None,
             "w_en": f64(en.jastrow_kernel.weight) if en is not None else None,
             "views": pv,
@@ -203,16 +206,19 @@ class SlaterJastrow(WaveFunction):
             raise ValueError("positions must have shape (Nbatch, %d)" % (self.nelec * 3))
         return pos.detach().to(torch.float64).contiguous()
 
-    def _eval(self, pos: torch.Tensor, mode: int, precision: Optional[str] = None):
+    def _eval(self, pos: torch.Tensor, mode: int, precision: Optional[str] = None, want=None):
+        """Outputs of one qmc_wf_eval (those named in ``want``, or all of the
+        mode: an output that is not wanted is neither allocated nor stored)."""
         precision = precision or (self.precision if mode == N.QMC_EVAL_PSI else self.eloc_precision)
         x = self._check_pos(pos)
         nw = x.shape[0]
         plan = self.device_plan()
         # the local-energy kernel reads W in FP64 in both precisions
-        prm, keep = self._params(precision if mode == N.QMC_EVAL_PSI else "fp64")
-        out = {k: torch.empty(nw, dtype=torch.float64, device=x.device)
-               for k in (("psi", "logabs", "sign") if mode == N.QMC_EVAL_PSI
-                         else ("psi", "logabs", "sign", "kinetic", "eloc", "epot"))}
+        prm, keep = self._params(precision if mode == N.QMC_EVAL_PSI else "fp64", plan)
+        if want is None:
+            want = (("psi", "logabs", "sign") if mode == N.QMC_EVAL_PSI
+                    else ("psi", "logabs", "sign", "kinetic", "eloc", "epot"))
+        out = {k: torch.empty(nw, dtype=torch.float64, device=x.device) for k in want}
         if nw == 0:  # an empty batch (its tensors have no storage to hand over)
             return out
         o = N.QmcWfOut()
@@ -243,12 +249,12 @@ class SlaterJastrow(WaveFunction):
     def pdf(self, pos: torch.Tensor, return_grad: Optional[bool] = False) -> torch.Tensor:
         if return_grad:
             return self.gradients(pos, pdf=True)
-        psi = self._eval(pos, N.QMC_EVAL_PSI)["psi"]
+        psi = self._eval(pos, N.QMC_EVAL_PSI, want=("psi",))["psi"]
         return (psi * psi).to(torch.get_default_dtype())
 
     def log_psi(self, pos: torch.Tensor, precision: Optional[str] = None):
         """(log|psi|, sign(psi)) in float64, shape (Nbatch,)."""
-        out = self._eval(pos, N.QMC_EVAL_PSI, precision)
+        out = self._eval(pos, N.QMC_EVAL_PSI, precision, ("logabs", "sign"))
         return out["logabs"], out["sign"]
 
     def kinetic_energy_autograd(self, x: torch.Tensor) -> torch.Tensor:
@@ -257,11 +263,11 @@ class SlaterJastrow(WaveFunction):
 
     def kinetic_energy_jacobi(self, x: torch.Tensor, **kwargs) -> torch.Tensor:
         """-1/2 lap(psi)/psi by the Jacobi formula, (Nbatch, 1) (slater_jastrow.py:312-344)."""
-        return self._eval(x, N.QMC_EVAL_ELOC)["kinetic"].to(torch.get_default_dtype()).view(-1, 1)
+        return self._eval(x, N.QMC_EVAL_ELOC, want=("kinetic",))["kinetic"].to(torch.get_default_dtype()).view(-1, 1)
 
     def local_energy(self, pos: torch.Tensor) -> torch.Tensor:
         """T + V_en + V_ee + V_nn, (Nbatch, 1) (wf_base.py:184-215)."""
-        return self._eval(pos, N.QMC_EVAL_ELOC)["eloc"].to(torch.get_default_dtype()).view(-1, 1)
+        return self._eval(pos, N.QMC_EVAL_ELOC, want=("eloc",))["eloc"].to(torch.get_default_dtype()).view(-1, 1)
 
     def local_energy_parts(self, pos: torch.Tensor, precision: Optional[str] = None):
         """All outputs of one local-energy evaluation (float64 dict)."""
@@ -310,7 +316,7 @@ class SlaterJastrow(WaveFunction):
         x = self._check_pos(pos)
         nw = x.shape[0]
         plan = self.device_plan()
-        prm, keep = self._params(precision)
+        prm, keep = self._params(precision, plan)
         dr = torch.empty(nw, self.nelec, 3, dtype=torch.float64, device=x.device)
         la = torch.empty(nw, dtype=torch.float64, device=x.device)
         sg = torch.empty(nw, dtype=torch.float64, device=x.device)
@@ -365,8 +371,7 @@ class _PsiFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, wf, x, mo_mod, ci, bas_exp, w_ee, w_en):
-        out = wf._eval(x, N.QMC_EVAL_PSI)
-        psi = out["psi"]
+        psi = wf._eval(x, N.QMC_EVAL_PSI, want=("psi",))["psi"]
         ctx.wf = wf
         ctx.save_for_backward(x.detach(), psi)
         return psi.to(torch.get_default_dtype()).view(-1, 1)
@@ -392,9 +397,14 @@ def _param_grads(wf, r, needs):
     dt = torch.get_default_dtype()
     d_mod = d_ci = d_exp = d_ee = d_en = None
     if needs[2]:
-        full = torch.zeros_like(wf.mo.mo_modifier, dtype=torch.float64)
-        full[:, : r["w"].shape[1]] = r["w"]
-        d_mod = (full * wf.mo.mo_scf.to(full)).to(wf.mo.mo_modifier.dtype)
+        mod, w = wf.mo.mo_modifier, r["w"]
+        scf = wf.mo.mo_scf.detach().to(w)
+        if w.shape[1] == mod.shape[1]:
+            d_mod = w * scf
+        else:  # orbitals that no configuration occupies have no gradient
+            d_mod = torch.zeros_like(mod, dtype=torch.float64)
+            torch.mul(w, scf[:, : w.shape[1]], out=d_mod[:, : w.shape[1]])
+        d_mod = d_mod.to(mod.dtype)
     if needs[3]:
         d_ci = r["ci"].view(1, -1).to(wf.fc.weight.dtype)
     if needs[4] and r.get("exp") is not None:
@@ -415,7 +425,7 @@ def adjoint_reduce(wf: SlaterJastrow, pos: torch.Tensor, weights: torch.Tensor, 
     x = wf._check_pos(pos)
     nw = x.shape[0]
     plan = wf.device_plan()
-    prm, keep = wf._params("fp64")
+    prm, keep = wf._params("fp64", plan)
     dev, f64_ = x.device, torch.float64
     sz = plan.sizes()
     lib = N.load()
@@ -477,7 +487,7 @@ class _ELocFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, wf, x, mo_mod, ci, bas_exp, w_ee, w_en):
-        el = wf._eval(x, N.QMC_EVAL_ELOC)["eloc"]
+        el = wf._eval(x, N.QMC_EVAL_ELOC, want=("eloc",))["eloc"]
         ctx.wf = wf
         ctx.save_for_backward(x.detach())
         return el.to(torch.get_default_dtype()).view(-1, 1)
