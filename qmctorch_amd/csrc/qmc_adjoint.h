@@ -52,31 +52,101 @@ __device__ __forceinline__ void red_zero_slot(const RedSlots& r, int nentry, int
         if (red_owner(o) == lane) s[o] = 0.0;
 }
 
+// Sums over the 64 lanes of outputs that every lane contributes to, eight
+// outputs (an aligned block of the slot) per exchange: the contributions are
+// stored in LDS rows, lane l adds lanes 8 q .. 8 q + 7 (q = l / 8) of row
+// l mod 8, the eight partial sums meet by three xor shuffles, and the owner
+// lane adds the result to the slot.  A butterfly and a dependent read of the
+// slot per output took 12 shuffles and a memory round trip each (log|psi| adjoint
+// kernel: water, 8192 walkers, 81 -> 46 us; LiH with 93 CI terms and exponents,
+// 2048 walkers, 217 -> 181 us).
+struct RedBatch {
+    static constexpr int kRow = 65;
+    double* buf;  // this wave's [8][65]
+    double* slot;
+    int lane, base, mask;
+    __device__ __forceinline__ RedBatch(double* b, double* s, int l) : buf(b), slot(s), lane(l), base(-1), mask(0) {
+        wave_lds_sync();  // earlier loads of the buffer come first
+    }
+    __device__ __forceinline__ void put(int o, double v) {
+        const int b = o & ~7;
+        if (b != base) {
+            flush();
+            base = b;
+        }
+        buf[(o & 7) * kRow + lane] = v;
+        mask |= 1 << (o & 7);
+    }
+    __device__ __forceinline__ void flush() {
+        if (mask == 0) return;
+        const int c = lane & 7, q = lane >> 3, o = base + c;
+        const bool mine = ((mask >> c) & 1) != 0 && red_owner(o) == lane;
+        const double old = mine ? slot[o] : 0.0;
+        wave_lds_sync();
+        double acc = 0.0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) acc += buf[c * kRow + 8 * q + k];
+        wave_lds_sync();
+        acc += __shfl_xor(acc, 8);
+        acc += __shfl_xor(acc, 16);
+        acc += __shfl_xor(acc, 32);
+        if (mine) slot[o] = old + acc;
+        mask = 0;
+    }
+};
+
+// Sums of a[0..7] over the lanes with the same l mod 8, output m = l / 8 to each
+// lane: recursive halving, 4 + 2 + 1 exchanges for the eight sums.
+__device__ __forceinline__ double red_scatter8(const double (&a)[8], int lane) {
+    const int q = lane >> 3;
+    double b[4], d[2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const double lo = a[i], hi = a[4 + i];
+        b[i] = ((q & 4) ? hi : lo) + __shfl_xor((q & 4) ? lo : hi, 32);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) d[i] = ((q & 2) ? b[2 + i] : b[i]) + __shfl_xor((q & 2) ? b[i] : b[2 + i], 16);
+    return ((q & 1) ? d[1] : d[0]) + __shfl_xor((q & 1) ? d[0] : d[1], 8);
+}
+
 // Accumulates sum over lanes r of x[r][i] * G[r][m] (+ y[r][i] * H[r][m]) for
 // the AO entries i of a chunk staged in LDS (column i mod 8 of the wave's
-// stage rows, 9 doubles per lane), every m < nmo.  Lane l combines rows
-// 8 q .. 8 q + 7 (q = l / 8) of column l mod 8, the eight partial sums meet
-// by three xor shuffles, and the owner lane adds the result to the slot.
+// stage rows, 9 doubles per lane), every m < nmo; G (and H) staged in LDS by
+// column, [m][64].  Lane l combines rows 8 q .. 8 q + 7 (q = l / 8) of column
+// l mod 8, the partial sums of eight m meet by red_scatter8 at their owner
+// lanes, which read the slot before and write it after the sums.
 template <int NM, bool TWO>
 __device__ __forceinline__ void red_flush_w(double* slot, int i0, int ncol, int nmo, const double* xs,
-                                            const double* ys, const double (&G)[NM], const double (&H)[NM],
-                                            int lane) {
+                                            const double* ys, const double* G, const double* H, int lane) {
     const int c = lane & 7, q = lane >> 3;
+    constexpr int kSets = (NM + 7) / 8;
+    double old[kSets], x[8], y[8];
 #pragma unroll
-    for (int m = 0; m < NM; ++m) {
-        if (m < nmo) {
-            double acc = 0.0;
+    for (int j = 0; j < kSets; ++j)
+        old[j] = (c < ncol && 8 * j + q < nmo) ? slot[(i0 + c) * nmo + 8 * j + q] : 0.0;
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const int r = 8 * q + k;
-                acc += xs[r * (kRedCols + 1) + c] * __shfl(G[m], r);
-                if (TWO) acc += ys[r * (kRedCols + 1) + c] * __shfl(H[m], r);
+    for (int k = 0; k < 8; ++k) {
+        x[k] = xs[(8 * q + k) * (kRedCols + 1) + c];
+        y[k] = TWO ? ys[(8 * q + k) * (kRedCols + 1) + c] : 0.0;
+    }
+#pragma unroll
+    for (int j = 0; j < kSets; ++j) {
+        double a[8];
+#pragma unroll
+        for (int m8 = 0; m8 < 8; ++m8) {
+            const int m = 8 * j + m8;
+            a[m8] = 0.0;
+            if (m < NM) {
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    a[m8] = fma(x[k], G[m * 64 + 8 * q + k], a[m8]);
+                    if (TWO) a[m8] = fma(y[k], H[m * 64 + 8 * q + k], a[m8]);
+                }
             }
-            acc += __shfl_xor(acc, 8);
-            acc += __shfl_xor(acc, 16);
-            acc += __shfl_xor(acc, 32);
-            if (c < ncol && red_owner_w(i0 + c, m) == lane) slot[(i0 + c) * nmo + m] += acc;
         }
+        const double sum = red_scatter8(a, lane);
+        if (c < ncol && 8 * j + q < nmo) slot[(i0 + c) * nmo + 8 * j + q] = old[j] + sum;
     }
 }
 
@@ -88,8 +158,8 @@ struct RedStage {
     double* ys;  // second stage (the kinetic b rows) when TWO
     double* slot;
     int lane, nmo, i0, ncol;
-    const double (*G)[NM];
-    const double (*H)[NM];
+    const double* G;  // [m][64] coefficient columns of the wavefront
+    const double* H;
     __device__ __forceinline__ void put(int i, double x, double y) {
         if (i - i0 >= kRedCols) flush();
         if (ncol == 0) i0 = i - (i & (kRedCols - 1));  // chunks start at multiples of 8
@@ -108,7 +178,7 @@ struct RedStage {
     __device__ __forceinline__ void flush() {
         if (ncol == 0) return;
         wave_lds_sync();
-        red_flush_w<NM, TWO>(slot, i0, ncol, nmo, xs, ys, *G, *H, lane);
+        red_flush_w<NM, TWO>(slot, i0, ncol, nmo, xs, ys, G, H, lane);
         wave_lds_sync();
         clear();
         wave_lds_sync();
@@ -116,6 +186,13 @@ struct RedStage {
         ncol = 0;
     }
 };
+
+// Coefficient columns [m][64] of red_flush_w for this wavefront.
+template <int NM, int WAVES>
+__device__ __forceinline__ double* red_coeff_rows() {
+    __shared__ double g[WAVES * NM * 64];
+    return g + (WAVES > 1 ? (threadIdx.x >> 6) * NM * 64 : 0);
+}
 
 // CI combination of a walker from the per-lane unique-configuration values
 // (the lanes' spins, shared through the walker's first up and down lanes):
@@ -221,17 +298,18 @@ __device__ __forceinline__ void logpsi_adjoint_reduce(const GRedArgs& a, const W
         const int blk = t.nsig_max * NM;
         const double* Mu = xlds + (size_t)(L.wl * 2) * 3 * blk;
         const double* Md = Mu + 3 * blk;
+        RedBatch red(stage, slot, L.lane);
         for (int n = 0; n < t.nci; ++n) {
             double Ru, Rd = 1.0, q;
             exc_ratio<NM, false>(t.exc_up + 6 * t.ci_up[n], Mu, nullptr, t.nup, 0.0, Ru, q);
             if (t.ndown > 0) exc_ratio<NM, false>(t.exc_dn + 6 * t.ci_dn[n], Md, nullptr, t.ndown, 0.0, Rd, q);
-            const double sum = wave_sum((v && L.e == 0) ? gw * (Ru * Rd / S) : 0.0);
-            const int o = a.r.off_ci + n;
-            if (red_owner(o) == L.lane) slot[o] += sum;
+            red.put(a.r.off_ci + n, (v && L.e == 0) ? gw * (Ru * Rd / S) : 0.0);
         }
+        red.flush();
     } else if constexpr (!MULTI) {
-        const double sum = wave_sum((v && L.e == 0) ? gw / ldc(a.p.ci, 0) : 0.0);  // d log|psi| / d c = 1 / c
-        if (red_owner(a.r.off_ci) == L.lane) slot[a.r.off_ci] += sum;
+        RedBatch red(stage, slot, L.lane);
+        red.put(a.r.off_ci, (v && L.e == 0) ? gw / ldc(a.p.ci, 0) : 0.0);  // d log|psi| / d c = 1 / c
+        red.flush();
         double lg, sg;
         conf_inverse<NM>(t, L, 0, mo, stage_conf_rows<NM>(t, L, mo), lg, sg, gam);
     } else {
@@ -249,6 +327,7 @@ __device__ __forceinline__ void logpsi_adjoint_reduce(const GRedArgs& a, const W
         conf_dets<NM, false>(t, L, mo, own_ex, ld, sd, om, gam);
         CiTerms ct;
         ci_terms(t, a.p, L, ld, sd, td, ct);
+        RedBatch red(stage, slot, L.lane);
         for (int n = 0; n < t.nci; ++n) {
             double l, sg, tr;
             ct.term(t, n, l, sg, tr);
@@ -257,21 +336,18 @@ __device__ __forceinline__ void logpsi_adjoint_reduce(const GRedArgs& a, const W
 #pragma unroll
             for (int c = 0; c < QMC_MAXCONF; ++c)
                 if (c == mine) om[c] += ldc(a.p.ci, n) * dn_s;
-            const double sum = wave_sum((v && L.e == 0) ? gw * dn_s : 0.0);
-            const int o = a.r.off_ci + n;
-            if (red_owner(o) == L.lane) slot[o] += sum;
+            red.put(a.r.off_ci + n, (v && L.e == 0) ? gw * dn_s : 0.0);
         }
+        red.flush();
         conf_dets<NM, true>(t, L, mo, own_ex, ld, sd, om, gam);
     }
     // W: stage the recomputed AO row, contract with g * Gamma
-    double gG[NM], unused[NM];
-#pragma unroll
-    for (int m = 0; m < NM; ++m) {
-        gG[m] = v ? gw * gam[m] : 0.0;
-        unused[m] = 0.0;
-    }
     {
-        RedStage<NM, false> st{stage, nullptr, slot, L.lane, t.nmo, 0, 0, &gG, &unused};
+        double* G = red_coeff_rows<NM, EXC ? 1 : kBlockWaves>();
+        wave_lds_sync();  // the previous walkers' loads come first
+#pragma unroll
+        for (int m = 0; m < NM; ++m) G[m * 64 + L.lane] = v ? gw * gam[m] : 0.0;
+        RedStage<NM, false> st{stage, nullptr, slot, L.lane, t.nmo, 0, 0, G, nullptr};
         st.clear();
         wave_lds_sync();
         auto sink = [&](int i, int, double val, double, double, double, double) { st.put(i, v ? val : 0.0, 0.0); };
@@ -280,6 +356,7 @@ __device__ __forceinline__ void logpsi_adjoint_reduce(const GRedArgs& a, const W
     }
     // exponents: per term slot (entry i, primitive q) the walker sum of
     // g G_i d AO_i / d a_q (G_i = sum_m Gamma[m] W[mu_i][m]), as exp_adjoint
+    RedBatch red(stage, slot, L.lane);
     if (a.r.off_exp >= 0) {
         for (int g = 0; g < t.ngroup; ++g) {
             const int at = t.grp_atom[g];
@@ -307,9 +384,7 @@ __device__ __forceinline__ void logpsi_adjoint_reduce(const GRedArgs& a, const W
                         const int nn = (int)t.gao_n[(size_t)i * QMC_MAXP + q];
                         term = -r * K * ipow(r, nn) * exp(-al * r) * Y;
                     }
-                    const double sum = wave_sum(v ? gw * G * term : 0.0);
-                    const int o = a.r.off_exp + i * QMC_MAXP + q;
-                    if (red_owner(o) == L.lane) slot[o] += sum;
+                    red.put(a.r.off_exp + i * QMC_MAXP + q, v ? gw * G * term : 0.0);
                 }
             }
         }
@@ -335,12 +410,9 @@ __device__ __forceinline__ void logpsi_adjoint_reduce(const GRedArgs& a, const W
             den_ -= r2 * qq * qq;
         }
     }
-    const double sums[2] = {wave_sum(v ? gw * dee : 0.0), wave_sum(v ? gw * den_ : 0.0)};
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const int o = a.r.off_jas + k;
-        if (red_owner(o) == L.lane) slot[o] += sums[k];
-    }
+    red.put(a.r.off_jas + 0, v ? gw * dee : 0.0);
+    red.put(a.r.off_jas + 1, v ? gw * den_ : 0.0);
+    red.flush();
 }
 
 // Stage rows of the wavefronts of a block: NS x [64][9] doubles per wave.
@@ -456,11 +528,11 @@ __device__ __forceinline__ void eloc_adjoint_reduce(const ERedArgs& a, const Wal
         wave_lds_sync();
     }
     if constexpr (EXC) {
+        RedBatch red(stage, slot, L.lane);
         T = exc_eloc_gamma<NM>(t, a.p, L, mo, bk, xlds, GA, GB, [&](int nn, double val) {
-            const double sum = wave_sum((v && L.e == 0) ? gw * val : 0.0);
-            const int o = a.r.off_ci + nn;
-            if (red_owner(o) == L.lane) slot[o] += sum;
+            red.put(a.r.off_ci + nn, (v && L.e == 0) ? gw * val : 0.0);
         });
+        red.flush();
 #pragma unroll
         for (int m = 0; m < NM; ++m) {
             if (m < t.nmo) {
@@ -523,6 +595,8 @@ __device__ __forceinline__ void eloc_adjoint_reduce(const ERedArgs& a, const Wal
         double rho[QMC_MAXCONF], om[QMC_MAXCONF];
 #pragma unroll
         for (int c = 0; c < QMC_MAXCONF; ++c) rho[c] = om[c] = 0.0;
+        static_assert(!use_minors<NM>() || 2 * 64 * (kRedCols + 1) >= 64 * NM + 8 * RedBatch::kRow, "beside the kinetic rows");
+        RedBatch red(use_minors<NM>() ? ycol : stage, slot, L.lane);
         for (int n = 0; n < t.nci; ++n) {
             double lg, sg, tr;
             ct.term(t, n, lg, sg, tr);
@@ -535,10 +609,9 @@ __device__ __forceinline__ void eloc_adjoint_reduce(const ERedArgs& a, const Wal
                     rho[c] += wn * (tr - T);
                     om[c] += wn;
                 }
-            const double sum = wave_sum((v && L.e == 0) ? gw * dns * (tr - T) : 0.0);
-            const int o = a.r.off_ci + n;
-            if (red_owner(o) == L.lane) slot[o] += sum;
+            red.put(a.r.off_ci + n, (v && L.e == 0) ? gw * dns * (tr - T) : 0.0);
         }
+        red.flush();
 #pragma unroll
         for (int m = 0; m < NM; ++m) GA[m] = GB[m] = 0.0;
 #pragma unroll 1
@@ -579,13 +652,23 @@ __device__ __forceinline__ void eloc_adjoint_reduce(const ERedArgs& a, const Wal
     }
     // W: stage the recomputed AO and kinetic rows, contract with g GA and g GB
     {
-        double gA[NM], gB[NM];
+        // coefficient columns: their own LDS, or the inversion's and the kinetic
+        // rows' of the larger buckets (no longer read)
+        double *G, *H;
+        if constexpr (EXC || use_minors<NM>()) {
+            G = red_coeff_rows<2 * NM, EXC ? 1 : kBlockWaves>();
+            H = G + NM * 64;
+        } else {
+            G = wave_rowbuf<NM>();
+            H = brow;
+        }
+        wave_lds_sync();  // earlier loads come first
 #pragma unroll
         for (int m = 0; m < NM; ++m) {
-            gA[m] = v ? gw * GA[m] : 0.0;
-            gB[m] = v ? gw * GB[m] : 0.0;
+            G[m * 64 + L.lane] = v ? gw * GA[m] : 0.0;
+            H[m * 64 + L.lane] = v ? gw * GB[m] : 0.0;
         }
-        RedStage<NM, true> st{stage, stage + 64 * (kRedCols + 1), slot, L.lane, t.nmo, 0, 0, &gA, &gB};
+        RedStage<NM, true> st{stage, stage + 64 * (kRedCols + 1), slot, L.lane, t.nmo, 0, 0, G, H};
         st.clear();
         wave_lds_sync();
         auto sink = [&](int i, int, double ao, double ax, double ay, double az, double al) {
@@ -602,14 +685,10 @@ __device__ __forceinline__ void eloc_adjoint_reduce(const ERedArgs& a, const Wal
     }
     dte -= 0.5 * dle;
     dtn -= 0.5 * dln;
-    const double sdte = seg_sum(dte, L.wbase, t.nelec, t.nelec);
-    const double sdtn = seg_sum(dtn, L.wbase, t.nelec, t.nelec);
-    const double sums[2] = {wave_sum((v && L.e == 0) ? gw * sdte : 0.0), wave_sum((v && L.e == 0) ? gw * sdtn : 0.0)};
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const int o = a.r.off_jas + k;
-        if (red_owner(o) == L.lane) slot[o] += sums[k];
-    }
+    RedBatch red(stage, slot, L.lane);
+    red.put(a.r.off_jas + 0, v ? gw * dte : 0.0);
+    red.put(a.r.off_jas + 1, v ? gw * dtn : 0.0);
+    red.flush();
     if (a.eloc) {
         double kee, ken, d0, d1, d2, d3, vee, ven;
         jastrow_and_potential<true>(t, a.p, L, x, y, z, kee, ken, d0, d1, d2, d3, vee, ven);
