@@ -394,6 +394,7 @@ int qmc_plan_create(const QmcSystemDesc* d, QmcPlan** out) {
             std::vector<float> kf(r.K.begin(), r.K.end());
             t.nrec = (int)(r.rec.size() / kRecWords);
             t.rec = (decltype(t.rec))p->upload(r.rec.data(), r.rec.size());
+            t.nrec_K = (int)r.K.size();
             t.rec_K = (decltype(t.rec_K))p->upload(r.K.data(), r.K.size());
             t.rec_Kf = (decltype(t.rec_Kf))p->upload(kf.data(), kf.size());
         }

@@ -45,11 +45,10 @@ __device__ __forceinline__ double wave_sum(double v) {
 // Zero the outputs of this wavefront's slot owned by this lane.
 __device__ __forceinline__ void red_zero_slot(const RedSlots& r, int nentry, int nmo, int slot, int lane) {
     double* s = r.ws + (size_t)slot * r.stride;
-    for (int i = 0; i < nentry; ++i)
-        for (int m = 0; m < nmo; ++m)
-            if (red_owner_w(i, m) == lane) s[i * nmo + m] = 0.0;
-    for (int o = nentry * nmo; o < r.stride; ++o)
-        if (red_owner(o) == lane) s[o] = 0.0;
+    for (int i = lane & 7; i < nentry; i += 8)  // red_owner_w(i, m) == lane
+        for (int m = lane >> 3; m < nmo; m += 8) s[i * nmo + m] = 0.0;
+    const int o0 = nentry * nmo;
+    for (int o = o0 + ((lane - o0) & 63); o < r.stride; o += 64) s[o] = 0.0;  // red_owner(o) == lane
 }
 
 // Sums over the 64 lanes of outputs that every lane contributes to, eight

@@ -65,6 +65,7 @@ struct Tables {
     const QMC_CONST int* rec;
     const QMC_CONST double* rec_K;
     const QMC_CONST float* rec_Kf;
+    int nrec_K;  // their number
     const QMC_CONST int* ao_ptr;
     const QMC_CONST int* ao_ent;
     const QMC_CONST int* exp_ptr;
@@ -309,6 +310,21 @@ __device__ __forceinline__ void record_moments(const T* gexp, const QMC_CONST T*
     for (int q = 0; q < kRecShells; ++q)
         if (q < nk)
             shell_moments<T, DERIV, NP>([&](int p) { return K[q * (NP + 1) + p]; }, E, A, m[q][0], m[q][1], m[q][2]);
+}
+
+// One dword of each 128-byte line of [p, p + bytes), four loads in flight a lane.
+__device__ __forceinline__ uint32_t touch_lines(const void* p, int bytes, int lane) {
+    uint32_t acc = 0;
+    for (int b = lane * 128; b < bytes; b += 4 * 64 * 128) {
+        uint32_t v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int o = b + k * 64 * 128;
+            v[k] = o < bytes ? *(const uint32_t*)((const char*)p + o) : 0u;
+        }
+        acc |= (v[0] | v[1]) | (v[2] | v[3]);
+    }
+    return acc;
 }
 
 template <typename T, int RAD, bool DERIV, typename Sink>
