@@ -605,7 +605,7 @@ __device__ __forceinline__ void seg_pivot_init(int myrow, int gbase, bool real) 
 
 // seg_pivot_post issues column k's maximum (and the next column's clear);
 // seg_pivot_get waits for it, and for every LDS store the caller issued in
-// between, and returns the pivot row.  seg_pivot does both.
+// between, and returns the pivot row.
 template <int NM>
 __device__ __forceinline__ void seg_pivot_post(int k, bool cand, double v, int myrow, int gbase, bool real) {
     static_assert(NM <= 32, "five bits of row index");
@@ -623,20 +623,14 @@ __device__ __forceinline__ int seg_pivot_get(int k, int gbase) {
     return m ? 31 - (int)(m & 31u) : 0;
 }
 
-template <int NM>
-__device__ __forceinline__ int seg_pivot(int k, bool cand, double v, int myrow, int gbase, bool real) {
-    seg_pivot_post<NM>(k, cand, v, myrow, gbase, real);
-    return seg_pivot_get(k, gbase);
-}
-
 // ------------------------------------------------- determinant-only elimination
 // Determinant det 2^ex2 (det 0 or a signed mantissa) of the n x n matrix whose
 // row r lives in lane gbase + r, with the row arithmetic of
 // lane_gauss_jordan<NM, false> but fewer cross-lane moves per column:
 //  * the pivot (largest |a_rk| among the rows not used yet, first one on ties,
-//    compared through seg_pivot's 32-bit keys): up to 8 columns from the n
+//    compared through seg_pivot_post's 32-bit keys): up to 8 columns from the n
 //    keys gathered into every lane by shuffles; for the larger buckets by
-//    seg_pivot's LDS atomic maximum;
+//    its LDS atomic maximum;
 //  * the pivot row through LDS, read back as broadcast loads (two columns per
 //    load) instead of one shuffle pair per column, with the pivot itself and
 //    its reciprocal (det_recips()), which every candidate forms while the
@@ -699,7 +693,7 @@ __device__ __forceinline__ void lane_det_lds(double (&a)[NM], int n, int nmax, i
                 for (int j = k + 1; j < NM; ++j) a[j] = a[j] - f * rowbuf[j];
                 if (is_piv) done = true;
             } else {
-                // keys as in seg_pivot, gathered from the group's n lanes (reads
+                // keys as in seg_pivot_post, gathered from the group's n lanes (reads
                 // past the last row repeat it, which leaves the maximum alone);
                 // meanwhile every candidate row r publishes its remaining
                 // columns at rowbuf[r NM + k ..] and its pivot's reciprocal at
@@ -752,7 +746,7 @@ __device__ __forceinline__ void lane_det_lds(double (&a)[NM], int n, int nmax, i
 // pivot row p, storage column k holds the inverse's column of row p.  On exit
 // the lane that pivoted column k (my_col = k) holds row k of A^-1 with the
 // entry of row i in storage column (my_col of row i's lane); det and ex2 as
-// lane_det_lds, pivots chosen by seg_pivot.  NM multiply-adds per column and
+// lane_det_lds, pivots chosen by seg_pivot_post.  NM multiply-adds per column and
 // row, where eliminating [A | I] or [A | B] took up to 2 NM and twice the
 // registers.  rowbuf: the group's row buffer (NM doubles used).
 template <int NM>
