@@ -823,14 +823,14 @@ struct Group {
     bool multi;  // several configurations
     const SpecEntry* spec;
     std::vector<int> idx;
-    size_t lds;  // exc: the largest exc_lds_bytes of the group's jobs
+    size_t lds;  // largest of the group's jobs: exc_lds_bytes (exc), combine_table_bytes (multi)
 };
 
 // Groups the jobs by (radial type, register bucket, configuration kind, excitation
 // path, generated layout), costliest systems first inside a group.  Returns an error for jobs
 // without a bucket.
 template <typename JobT>
-int group_jobs(const JobT* jobs, int njobs, std::vector<Group>& groups) {
+int group_jobs(const JobT* jobs, int njobs, bool kin, std::vector<Group>& groups) {
     for (int j = 0; j < njobs; ++j) {
         const Tables& t = jobs[j].plan->t;
         const int bk = nm_bucket_fine(t);
@@ -845,7 +845,10 @@ int group_jobs(const JobT* jobs, int njobs, std::vector<Group>& groups) {
             g = &groups.back();
         }
         g->idx.push_back(j);
-        if (exc) g->lds = std::max(g->lds, exc_lds_bytes(t, bk));
+        if (exc)
+            g->lds = std::max(g->lds, exc_lds_bytes(t, bk));
+        else if (multi)
+            g->lds = std::max(g->lds, (size_t)combine_table_bytes(t, kin));
     }
     for (auto& g : groups)
         std::stable_sort(g.idx.begin(), g.idx.end(),
@@ -901,7 +904,7 @@ int qmc_metropolis_sweep_batch(QmcBatch* b, int32_t precision, const QmcSweepJob
     }
     if (live.empty()) return QMC_OK;
     std::vector<Group> groups;
-    int rc = group_jobs(live.data(), (int)live.size(), groups);
+    int rc = group_jobs(live.data(), (int)live.size(), false, groups);
     if (rc) return rc;
     int slot;
     rc = take_slot(b, slot);
@@ -942,10 +945,10 @@ int qmc_metropolis_sweep_batch(QmcBatch* b, int32_t precision, const QmcSweepJob
                 return fail(QMC_ERR_UNSUPPORTED, kNoExcBucket);
             continue;
         }
-        if (L.spec && L.spec->sweep_batch(dev + L.first, L.n, L.nwaves, precision, s) == 0) continue;
+        if (L.spec && L.spec->sweep_batch(dev + L.first, L.n, L.nwaves, (int)L.lds, precision, s) == 0) continue;
         const int r = precision == QMC_PREC_FP64
-                          ? QMC_BY_RAD(launch_sweep_batch_f64, L.rad, dev + L.first, L.n, L.nwaves, L.bucket, L.multi, s)
-                          : QMC_BY_RAD(launch_sweep_batch_f32, L.rad, dev + L.first, L.n, L.nwaves, L.bucket, L.multi, s);
+                          ? QMC_BY_RAD(launch_sweep_batch_f64, L.rad, dev + L.first, L.n, L.nwaves, L.bucket, (int)L.lds, L.multi, s)
+                          : QMC_BY_RAD(launch_sweep_batch_f32, L.rad, dev + L.first, L.n, L.nwaves, L.bucket, (int)L.lds, L.multi, s);
         if (r) return fail(QMC_ERR_UNSUPPORTED, kNoBucket);
     }
     QMC_HIP(hipGetLastError());
@@ -970,7 +973,7 @@ int qmc_wf_eval_batch(QmcBatch* b, int32_t precision, int32_t mode, const QmcEva
     }
     if (live.empty()) return QMC_OK;
     std::vector<Group> groups;
-    int rc = group_jobs(live.data(), (int)live.size(), groups);
+    int rc = group_jobs(live.data(), (int)live.size(), mode == QMC_EVAL_ELOC, groups);
     if (rc) return rc;
     int slot;
     rc = take_slot(b, slot);
@@ -1012,11 +1015,11 @@ int qmc_wf_eval_batch(QmcBatch* b, int32_t precision, int32_t mode, const QmcEva
                 return fail(QMC_ERR_UNSUPPORTED, kNoExcBucket);
             continue;
         }
-        if (L.spec && L.spec->wf_batch(dev + L.first, L.n, L.nwaves, precision, mode, s) == 0) continue;
+        if (L.spec && L.spec->wf_batch(dev + L.first, L.n, L.nwaves, (int)L.lds, precision, mode, s) == 0) continue;
         const int r =
             precision == QMC_PREC_FP64
-                ? QMC_BY_RAD(launch_wf_batch_f64, L.rad, dev + L.first, L.n, L.nwaves, L.bucket, L.multi, mode, s)
-                : QMC_BY_RAD(launch_wf_batch_f32, L.rad, dev + L.first, L.n, L.nwaves, L.bucket, L.multi, mode, s);
+                ? QMC_BY_RAD(launch_wf_batch_f64, L.rad, dev + L.first, L.n, L.nwaves, L.bucket, (int)L.lds, L.multi, mode, s)
+                : QMC_BY_RAD(launch_wf_batch_f32, L.rad, dev + L.first, L.n, L.nwaves, L.bucket, (int)L.lds, L.multi, mode, s);
         if (r) return fail(QMC_ERR_UNSUPPORTED, kNoBucket);
     }
     QMC_HIP(hipGetLastError());

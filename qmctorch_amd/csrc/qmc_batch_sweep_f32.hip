@@ -8,20 +8,20 @@
 namespace qmc {
 
 template <int NM, int RAD>
-static void go(const SJob* jobs, int njobs, int nwaves, bool multi, hipStream_t s) {
+static void go(const SJob* jobs, int njobs, int nwaves, int ctab, bool multi, hipStream_t s) {
     const dim3 g = grid_for_waves(nwaves);
     if (multi)
-        hipLaunchKernelGGL((sweep_batch_kernel<float, NM, RAD, true>), g, dim3(kBlock), 0, s, jobs, njobs, nwaves);
+        hipLaunchKernelGGL((sweep_batch_kernel<float, NM, RAD, true>), g, dim3(kBlock), kBlockWaves * ctab, s, jobs, njobs, nwaves, ctab);
     else
-        hipLaunchKernelGGL((sweep_batch_kernel<float, NM, RAD, false>), g, dim3(kBlock), 0, s, jobs, njobs, nwaves);
+        hipLaunchKernelGGL((sweep_batch_kernel<float, NM, RAD, false>), g, dim3(kBlock), kBlockWaves * ctab, s, jobs, njobs, nwaves, ctab);
 }
 
 template <>
-int launch_sweep_batch_f32<QMC_RAD>(const SJob* jobs, int njobs, int nwaves, int bucket, bool multi, hipStream_t s) {
+int launch_sweep_batch_f32<QMC_RAD>(const SJob* jobs, int njobs, int nwaves, int bucket, int ctab, bool multi, hipStream_t s) {
     switch (bucket) {
 #define QMC_CASE(K)                  \
     case K:                          \
-        go<K, QMC_RAD>(jobs, njobs, nwaves, multi, s); \
+        go<K, QMC_RAD>(jobs, njobs, nwaves, ctab, multi, s); \
         return 0;
         QMC_FINE_BUCKETS(QMC_CASE)
 #undef QMC_CASE

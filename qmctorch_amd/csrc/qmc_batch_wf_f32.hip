@@ -8,22 +8,22 @@
 namespace qmc {
 
 template <int NM, int RAD>
-static void go(const WJob* jobs, int njobs, int nwaves, bool multi, int mode, hipStream_t s) {
+static void go(const WJob* jobs, int njobs, int nwaves, int ctab, bool multi, int mode, hipStream_t s) {
     // psi only: local energies are evaluated by the FP64 kernels in every precision
     (void)mode;
     const dim3 g = grid_for_waves(nwaves);
     if (multi)
-        hipLaunchKernelGGL((wf_batch_kernel<float, NM, RAD, false, true>), g, dim3(kBlock), 0, s, jobs, njobs, nwaves);
+        hipLaunchKernelGGL((wf_batch_kernel<float, NM, RAD, false, true>), g, dim3(kBlock), kBlockWaves * ctab, s, jobs, njobs, nwaves, ctab);
     else
-        hipLaunchKernelGGL((wf_batch_kernel<float, NM, RAD, false, false>), g, dim3(kBlock), 0, s, jobs, njobs, nwaves);
+        hipLaunchKernelGGL((wf_batch_kernel<float, NM, RAD, false, false>), g, dim3(kBlock), kBlockWaves * ctab, s, jobs, njobs, nwaves, ctab);
 }
 
 template <>
-int launch_wf_batch_f32<QMC_RAD>(const WJob* jobs, int njobs, int nwaves, int bucket, bool multi, int mode, hipStream_t s) {
+int launch_wf_batch_f32<QMC_RAD>(const WJob* jobs, int njobs, int nwaves, int bucket, int ctab, bool multi, int mode, hipStream_t s) {
     switch (bucket) {
 #define QMC_CASE(K)                  \
     case K:                          \
-        go<K, QMC_RAD>(jobs, njobs, nwaves, multi, mode, s); \
+        go<K, QMC_RAD>(jobs, njobs, nwaves, ctab, multi, mode, s); \
         return 0;
         QMC_FINE_BUCKETS(QMC_CASE)
 #undef QMC_CASE

@@ -935,15 +935,24 @@ __device__ __forceinline__ void gather_conf(const Tables& t, const WalkerLane& L
 // share ex (their row scales) unless one was weak; otherwise, and for eliminated
 // blocks, the terms are taken relative to the largest power of two among them,
 // so that no ratio of determinants leaves the range.
+// The table is dynamic LDS, at byte coff of qmc_dyn_lds for this wavefront
+// (combine_table_bytes each): an entry per group and configuration.  Static
+// tables for the most any plan can have (64 groups, 8 configurations: 24 KB a
+// block, 40 KB with traces) cost the larger kernels a block a CU: benzene
+// CAS(2,2), FP64, 4096 walkers, psi 478 -> 230 us and 4 sweep steps 2345 -> 1294
+// us; E_L of water CAS(2,2), 131072 walkers, 462 -> 265 us.
+__host__ __device__ __forceinline__ int combine_table_bytes(const Tables& t, bool kin) {
+    return t.nconf_max * 2 * (64 / t.nelec) * (kin ? 20 : 12);
+}
+
 template <int NM, bool KIN, typename T>
-__device__ __forceinline__ void slater_combine(const Tables& t, const QmcParams& prm, const WalkerLane& L,
+__device__ __forceinline__ void slater_combine(const Tables& t, const QmcParams& prm, const WalkerLane& L, int coff,
                                                const T (&mo)[NM], const double (&bk)[NM], double& logabs,
                                                double& sgn, double& kin) {
-    __shared__ double dsh[kBlockWaves * QMC_MAXCONF * 64], tsh[KIN ? kBlockWaves * QMC_MAXCONF * 64 : 1];
-    __shared__ int esh[kBlockWaves * QMC_MAXCONF * 64];
-    double* dt = dsh + (threadIdx.x >> 6) * QMC_MAXCONF * 64;
-    int* et = esh + (threadIdx.x >> 6) * QMC_MAXCONF * 64;
-    double* tt = KIN ? tsh + (threadIdx.x >> 6) * QMC_MAXCONF * 64 : nullptr;
+    const int ngrp = 2 * L.G, nent = t.nconf_max * ngrp;  // entry [configuration][walker of the wavefront][spin]
+    double* dt = (double*)(qmc_dyn_lds + coff);
+    double* tt = dt + (KIN ? nent : 0);
+    int* et = (int*)(tt + nent);
     constexpr bool SCALE = std::is_same<T, double>::value;
     double* rows = nullptr;
     int own_ex = 0, eref = 0;
@@ -972,9 +981,10 @@ __device__ __forceinline__ void slater_combine(const Tables& t, const QmcParams&
         if (c == 0) eref = ex;
         common = common && ex == eref;
         const bool first = L.lane_real && L.myrow == 0;
+        const int at = c * ngrp + 2 * L.wl + L.spin;
         if (first) {
-            dt[c * 64 + L.lane] = d;
-            et[c * 64 + L.lane] = ex;
+            dt[at] = d;
+            et[at] = ex;
         }
         if constexpr (KIN) {
             double b[NM];
@@ -982,13 +992,14 @@ __device__ __forceinline__ void slater_combine(const Tables& t, const QmcParams&
 #pragma unroll
             for (int k = 0; k < NM; ++k) tp += k < L.n_sig ? b[k] * a[k] : 0.0;
             const double tr = seg_sum(tp, L.gbase, L.n_sig, t.nsig_max);
-            if (first) tt[c * 64 + L.lane] = tr;
+            if (first) tt[at] = tr;
         }
     }
     wave_lds_sync();
-    const int up_lane = L.wbase, dn_lane = L.wbase + (t.ndown > 0 ? t.nup : 0);
     const bool down = t.ndown > 0;
-    int emax = et[up_lane] + (down ? et[dn_lane] : 0);
+    // this walker's entries (a lane past the last walker reads another's)
+    const int up0 = 2 * (L.lane_real ? L.wl : 0), dn0 = up0 + (down ? 1 : 0);
+    int emax = et[up0] + (down ? et[dn0] : 0);
     double s = 0.0, st = 0.0;
     auto add = [&](int iu, int id, double dn) {
         s += dn;
@@ -1000,19 +1011,19 @@ __device__ __forceinline__ void slater_combine(const Tables& t, const QmcParams&
     if (!__any(!common && L.lane_real)) {
 #pragma unroll 4
         for (int n = 0; n < t.nci; ++n) {
-            const int iu = t.ci_up[n] * 64 + up_lane, id = t.ci_dn[n] * 64 + dn_lane;
+            const int iu = t.ci_up[n] * ngrp + up0, id = t.ci_dn[n] * ngrp + dn0;
             const double dd = dt[id];
             add(iu, id, ldc(prm.ci, n) * dt[iu] * (down ? dd : 1.0));
         }
     } else {
         emax = -(1 << 30);
         for (int n = 0; n < t.nci; ++n) {
-            const int iu = t.ci_up[n] * 64 + up_lane, id = t.ci_dn[n] * 64 + dn_lane;
+            const int iu = t.ci_up[n] * ngrp + up0, id = t.ci_dn[n] * ngrp + dn0;
             const bool zero = dt[iu] == 0.0 || (down && dt[id] == 0.0);
             emax = zero ? emax : max(emax, et[iu] + (down ? et[id] : 0));
         }
         for (int n = 0; n < t.nci; ++n) {
-            const int iu = t.ci_up[n] * 64 + up_lane, id = t.ci_dn[n] * 64 + dn_lane;
+            const int iu = t.ci_up[n] * ngrp + up0, id = t.ci_dn[n] * ngrp + dn0;
             const double dd = dt[id];
             add(iu, id, ldexp(ldc(prm.ci, n) * dt[iu] * (down ? dd : 1.0), et[iu] + (down ? et[id] : 0) - emax));
         }
@@ -1536,9 +1547,9 @@ __device__ __forceinline__ uint32_t touch_tables(const Tables& t, const QmcParam
 // psi / kinetic / local energy of the walkers of one wavefront.  MULTI: plans
 // of several configurations (up to QMC_MAXCONF unique ones per spin); without
 // it the plan is the ground-state determinant (identity_conf) and the kernel
-// holds none of their registers and code.
+// holds none of their registers and code.  coff: slater_combine's table.
 template <typename T, int NM, int RAD, bool ELOC, bool MULTI, typename AO = AoGeneric, bool EXC = false>
-__device__ __forceinline__ void wf_walkers(const KArgs& a, const WalkerLane& L) {
+__device__ __forceinline__ void wf_walkers(const KArgs& a, const WalkerLane& L, int coff = 0) {
     const Tables& t = a.t;
     const double* p = a.pos + (size_t)L.wclamp * 3 * t.nelec + 3 * L.e;
     const double x = p[0], y = p[1], z = p[2];
@@ -1597,7 +1608,7 @@ __device__ __forceinline__ void wf_walkers(const KArgs& a, const WalkerLane& L) 
         if constexpr (EXC)
             slater_exc<NM, ELOC>(t, a.p, L, mo, bk, (double*)qmc_dyn_lds, logabs, sgn, kin);
         else if constexpr (MULTI)
-            slater_combine<NM, ELOC>(t, a.p, L, mo, bk, logabs, sgn, kin);
+            slater_combine<NM, ELOC>(t, a.p, L, coff, mo, bk, logabs, sgn, kin);
         else if constexpr (ELOC)
             slater_single_kin<NM>(t, a.p, L, mo, bk, logabs, sgn, kin);
         else
@@ -1624,6 +1635,12 @@ __device__ __forceinline__ void wf_walkers(const KArgs& a, const WalkerLane& L) 
     }
 }
 
+// This wavefront's slater_combine table within the block's dynamic LDS, from
+// byte `from` on with wave_bytes a wavefront.
+__device__ __forceinline__ int combine_table(int from, int wave_bytes) {
+    return from + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * wave_bytes;
+}
+
 // Waves per SIMD the evaluation kernels are held to: what their registers allow
 // without spilling (168 VGPRs up to 5 columns, 3 with table-driven rows).
 template <int NM, typename AO>
@@ -1635,7 +1652,7 @@ template <typename T, int NM, int RAD, bool ELOC, bool MULTI, typename AO = AoGe
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(wf_waves<NM, AO>()))) void wf_kernel(KArgs a) {
     const WalkerLane L = lane_layout(a.t, a.nw);
     if ((int64_t)L.wave * L.G >= a.nw) return;  // whole wavefront beyond the batch
-    wf_walkers<T, NM, RAD, ELOC, MULTI, AO>(a, L);
+    wf_walkers<T, NM, RAD, ELOC, MULTI, AO>(a, L, MULTI ? combine_table(0, combine_table_bytes(a.t, ELOC)) : 0);
 }
 
 // Kernels of exc_mode plans: one wavefront per block, dynamic LDS of
@@ -1648,20 +1665,21 @@ __global__ __launch_bounds__(64) void wf_kernel_exc(KArgs a) {
 }
 
 // Many systems in one launch: job j owns global waves [wave0[j], wave0[j+1]).
+// ctab (MULTI): bytes per wavefront of the largest job's slater_combine table.
 struct WJob {
     KArgs a;
     int64_t wave0;
 };
 
 template <typename T, int NM, int RAD, bool ELOC, bool MULTI, typename AO = AoGeneric>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(wf_waves<NM, AO>()))) void wf_batch_kernel(const WJob* __restrict__ jobs, int njobs, int nwaves) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(wf_waves<NM, AO>()))) void wf_batch_kernel(const WJob* __restrict__ jobs, int njobs, int nwaves, int ctab) {
     const int wave = global_wave();
     if (wave >= nwaves) return;
     const int j = find_job(jobs, njobs, wave);
     const KArgs a = jobs[j].a;
     const WalkerLane L = lane_layout_w(a.t, a.nw, wave - (int)jobs[j].wave0);
     if ((int64_t)L.wave * L.G >= a.nw) return;
-    wf_walkers<T, NM, RAD, ELOC, MULTI, AO>(a, L);
+    wf_walkers<T, NM, RAD, ELOC, MULTI, AO>(a, L, MULTI ? combine_table(0, ctab) : 0);
 }
 
 // wf_batch_kernel for excitation plans: one wavefront per block (as
@@ -1685,11 +1703,12 @@ struct SArgs {
     int64_t nw;
 };
 
-// wlds: with WLDS, this wavefront's LDS copy of the entry-ordered W rows
+// wlds: with WLDS, this wavefront's LDS copy of the entry-ordered W rows; coff:
+// slater_combine's table
 template <typename T, int NM, int RAD, bool MULTI, typename AO = AoGeneric, bool WLDS = false, bool EXC = false>
 __device__ __forceinline__ double eval_logpsi(const Tables& t, const QmcParams& prm, const WalkerLane& L, double x,
                                               double y, double z, double logc0, double& sgn,
-                                              const T* wlds = nullptr) {
+                                              const T* wlds = nullptr, int coff = 0) {
     T mo[NM];
     const T* w = WLDS ? wlds : (const T*)prm.entry_w;
     // FP32 buckets of 16 and 24 columns contract on the matrix cores (a
@@ -1714,7 +1733,7 @@ __device__ __forceinline__ double eval_logpsi(const Tables& t, const QmcParams& 
         slater_exc<NM, false>(t, prm, L, mo, bk, (double*)qmc_dyn_lds, logabs, sgn, kin);
     } else if constexpr (MULTI) {
         double bk[NM], kin;
-        slater_combine<NM, false>(t, prm, L, mo, bk, logabs, sgn, kin);
+        slater_combine<NM, false>(t, prm, L, coff, mo, bk, logabs, sgn, kin);
     } else if constexpr (use_minors<NM>()) {
         T ksum;
         double y_[NM];
@@ -1730,7 +1749,8 @@ __device__ __forceinline__ double eval_logpsi(const Tables& t, const QmcParams& 
 // Persistent Metropolis sweep: nstep all-electron moves per launch, walker
 // state in registers (sampler/metropolis.py:134-165, 256-298).
 template <typename T, int NM, int RAD, bool MULTI, typename AO = AoGeneric, bool WLDS = false, bool EXC = false>
-__device__ __forceinline__ void sweep_walkers(const SArgs& a, const WalkerLane& L, const T* wlds = nullptr) {
+__device__ __forceinline__ void sweep_walkers(const SArgs& a, const WalkerLane& L, const T* wlds = nullptr,
+                                              int coff = 0) {
     const Tables& t = a.t;
     const int Ne = t.nelec;
     double* pp = a.wk.pos + (size_t)L.wclamp * 3 * Ne + 3 * L.e;
@@ -1743,7 +1763,7 @@ __device__ __forceinline__ void sweep_walkers(const SArgs& a, const WalkerLane& 
         asm volatile("" : : "v"(touched));
     }
     if (a.sw.init_logpsi) {
-        lp = eval_logpsi<T, NM, RAD, MULTI, AO, WLDS, EXC>(t, a.p, L, x, y, z, logc0, sgn, wlds);
+        lp = eval_logpsi<T, NM, RAD, MULTI, AO, WLDS, EXC>(t, a.p, L, x, y, z, logc0, sgn, wlds, coff);
     } else {
         lp = a.wk.logabs[L.wclamp];
         sgn = a.wk.sign[L.wclamp];
@@ -1809,7 +1829,8 @@ __device__ __forceinline__ void sweep_walkers(const SArgs& a, const WalkerLane& 
         }
         const double xn = x + nx, yn = y + ny, zn = z + nz;
         double sgn_n;
-        double lpn = eval_logpsi<T, NM, RAD, MULTI, AO, WLDS, EXC>(t, a.p, Ls, xn, yn, zn, logc0, sgn_n, wlds);
+        double lpn =
+            eval_logpsi<T, NM, RAD, MULTI, AO, WLDS, EXC>(t, a.p, Ls, xn, yn, zn, logc0, sgn_n, wlds, coff);
         if (lpn < lp_zero) lpn = lp_eps;
         // accept iff min(1, psi'^2/psi^2) >= U  <=>  2 (lpn - lp) >= log U; the
         // logarithm in the bulk precision (the hardware log2 in the mixed sweep,
@@ -1865,16 +1886,19 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NM >= 16
     SArgs a) {
     const WalkerLane L = lane_layout(a.t, a.nw);
     if ((int64_t)L.wave * L.G >= a.nw) return;
-    sweep_walkers<T, NM, RAD, MULTI, AO>(a, L);
+    sweep_walkers<T, NM, RAD, MULTI, AO>(a, L, nullptr, MULTI ? combine_table(0, combine_table_bytes(a.t, false)) : 0);
 }
 
 // sweep_kernel with the entry-ordered W rows staged in LDS once per block
-// (dynamic LDS of nentry * NM * sizeof(T) bytes, set by the launcher), for
+// (dynamic LDS of wlds_bytes(nentry * NM * sizeof(T)), set by the launcher, and
+// behind it the slater_combine tables of a MULTI instance), for
 // generated AO rows (whose fence() calls pace the W reads).  W values then
 // reach the MO accumulation by LDS broadcast reads instead of scalar loads,
 // which a 50-step loop otherwise hoists and spills to VGPR lanes.  Two waves
 // per SIMD are requested explicitly: the extra VGPRs of the LDS operands would
 // otherwise leave one.
+__host__ __device__ __forceinline__ constexpr int wlds_bytes(int w) { return (w + 15) / 16 * 16; }
+
 template <typename T, int NM, int RAD, bool MULTI, typename AO>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void sweep_kernel_wlds(SArgs a) {
     {
@@ -1886,7 +1910,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     }
     const WalkerLane L = lane_layout(a.t, a.nw);
     if ((int64_t)L.wave * L.G >= a.nw) return;
-    sweep_walkers<T, NM, RAD, MULTI, AO, true>(a, L, (const T*)qmc_dyn_lds);
+    const int from = wlds_bytes(a.t.nentry * NM * (int)sizeof(T));
+    sweep_walkers<T, NM, RAD, MULTI, AO, true>(
+        a, L, (const T*)qmc_dyn_lds, MULTI ? combine_table(from, combine_table_bytes(a.t, false)) : 0);
 }
 
 template <typename T, int NM, int RAD>
@@ -1919,22 +1945,23 @@ __global__ __launch_bounds__(64) void sweep_batch_kernel_exc(const SJob* __restr
 
 template <typename T, int NM, int RAD, bool MULTI, typename AO = AoGeneric>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NM >= 16 ? 2 : 1))) void sweep_batch_kernel(
-    const SJob* __restrict__ jobs, int njobs, int nwaves) {
+    const SJob* __restrict__ jobs, int njobs, int nwaves, int ctab) {
     const int wave = global_wave();
     if (wave >= nwaves) return;
     const int j = find_job(jobs, njobs, wave);
     const SArgs a = jobs[j].a;
     const WalkerLane L = lane_layout_w(a.t, a.nw, wave - (int)jobs[j].wave0);
     if ((int64_t)L.wave * L.G >= a.nw) return;
-    sweep_walkers<T, NM, RAD, MULTI, AO>(a, L);
+    sweep_walkers<T, NM, RAD, MULTI, AO>(a, L, nullptr, MULTI ? combine_table(0, ctab) : 0);
 }
 
 // sweep_batch_kernel with W in LDS: every wavefront stages the W rows of its
-// own job into its slice of wstride elements (dynamic LDS of 4 slices), so
+// own job into its slice of wstride elements (dynamic LDS of 4 slices, and
+// behind them the slater_combine tables of a MULTI instance), so
 // each walker runs the arithmetic of sweep_kernel_wlds exactly.
 template <typename T, int NM, int RAD, bool MULTI, typename AO>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void sweep_batch_kernel_wlds(
-    const SJob* __restrict__ jobs, int njobs, int nwaves, int wstride) {
+    const SJob* __restrict__ jobs, int njobs, int nwaves, int wstride, int ctab) {
     const int wave = global_wave();
     if (wave >= nwaves) return;
     const int j = find_job(jobs, njobs, wave);
@@ -1946,7 +1973,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     const int n = a.t.nentry * NM;  // <= wstride (one layout per launch)
     for (int i = L.lane; i < n; i += 64) w[i] = src[i];
     wave_lds_sync();
-    sweep_walkers<T, NM, RAD, MULTI, AO, true>(a, L, w);
+    const int from = wlds_bytes(kBlockWaves * wstride * (int)sizeof(T));
+    sweep_walkers<T, NM, RAD, MULTI, AO, true>(a, L, w, MULTI ? combine_table(from, ctab) : 0);
 }
 
 // ------------------------------------------------------------------ drift

@@ -64,15 +64,18 @@ int launch_wf_batch_exc(const WJob* jobs, int njobs, int nwaves, int bucket, siz
 // HMC / drift: MC = 1 for ground-state determinants, QMC_MAXCONF otherwise
 template <int RAD, int MC> int launch_hmc_f32(const HArgs& a, hipStream_t s);
 template <int RAD, int MC> int launch_hmc_f64(const HArgs& a, hipStream_t s);
-// batched launches: jobs (device) of one register bucket and configuration kind, nwaves in total
+// dynamic LDS of a kernel for several configurations: a slater_combine table per wavefront
+inline unsigned multi_lds(const Tables& t, bool kin) { return (unsigned)(kBlockWaves * combine_table_bytes(t, kin)); }
+// batched launches: jobs (device) of one register bucket and configuration kind, nwaves in total,
+// ctab the largest job's slater_combine table
 template <int RAD>
-int launch_sweep_batch_f32(const SJob* jobs, int njobs, int nwaves, int bucket, bool multi, hipStream_t s);
+int launch_sweep_batch_f32(const SJob* jobs, int njobs, int nwaves, int bucket, int ctab, bool multi, hipStream_t s);
 template <int RAD>
-int launch_sweep_batch_f64(const SJob* jobs, int njobs, int nwaves, int bucket, bool multi, hipStream_t s);
+int launch_sweep_batch_f64(const SJob* jobs, int njobs, int nwaves, int bucket, int ctab, bool multi, hipStream_t s);
 template <int RAD>
-int launch_wf_batch_f32(const WJob* jobs, int njobs, int nwaves, int bucket, bool multi, int mode, hipStream_t s);
+int launch_wf_batch_f32(const WJob* jobs, int njobs, int nwaves, int bucket, int ctab, bool multi, int mode, hipStream_t s);
 template <int RAD>
-int launch_wf_batch_f64(const WJob* jobs, int njobs, int nwaves, int bucket, bool multi, int mode, hipStream_t s);
+int launch_wf_batch_f64(const WJob* jobs, int njobs, int nwaves, int bucket, int ctab, bool multi, int mode, hipStream_t s);
 
 inline dim3 grid_for_waves(int nwaves) { return dim3((unsigned)((nwaves + (kBlock / 64) - 1) / (kBlock / 64))); }
 
@@ -98,9 +101,9 @@ struct SpecEntry {
     bool multi;          // built for several configurations (else for the ground-state determinant)
     const char* name;
     int (*sweep)(const SArgs& a, int precision, hipStream_t s);
-    int (*sweep_batch)(const SJob* jobs, int njobs, int nwaves, int precision, hipStream_t s);
+    int (*sweep_batch)(const SJob* jobs, int njobs, int nwaves, int ctab, int precision, hipStream_t s);
     int (*wf)(const KArgs& a, int precision, int mode, hipStream_t s);  // FP64 local energy
-    int (*wf_batch)(const WJob* jobs, int njobs, int nwaves, int precision, int mode, hipStream_t s);
+    int (*wf_batch)(const WJob* jobs, int njobs, int nwaves, int ctab, int precision, int mode, hipStream_t s);
     int (*hmc)(const HArgs& a, int precision, hipStream_t s);  // mixed HMC / drift
 };
 

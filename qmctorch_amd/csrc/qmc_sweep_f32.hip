@@ -12,7 +12,7 @@ static void go(const SArgs& a, hipStream_t s) {
     if (a.t.identity_conf)
         hipLaunchKernelGGL((sweep_kernel<float, NM, RAD, false>), grid_for(a.t, a.nw), dim3(kBlock), 0, s, a);
     else
-        hipLaunchKernelGGL((sweep_kernel<float, NM, RAD, true>), grid_for(a.t, a.nw), dim3(kBlock), 0, s, a);
+        hipLaunchKernelGGL((sweep_kernel<float, NM, RAD, true>), grid_for(a.t, a.nw), dim3(kBlock), multi_lds(a.t, false), s, a);
 }
 
 template <int RAD>

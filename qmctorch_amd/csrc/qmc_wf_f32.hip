@@ -14,7 +14,7 @@ static void go(const KArgs& a, int mode, hipStream_t s) {
     if (a.t.identity_conf)
         hipLaunchKernelGGL((wf_kernel<float, NM, RAD, false, false>), grid_for(a.t, a.nw), dim3(kBlock), 0, s, a);
     else
-        hipLaunchKernelGGL((wf_kernel<float, NM, RAD, false, true>), grid_for(a.t, a.nw), dim3(kBlock), 0, s, a);
+        hipLaunchKernelGGL((wf_kernel<float, NM, RAD, false, true>), grid_for(a.t, a.nw), dim3(kBlock), multi_lds(a.t, false), s, a);
 }
 
 template <int RAD>

@@ -12,11 +12,11 @@ static void go(const KArgs& a, int mode, hipStream_t s) {
     const dim3 g = grid_for(a.t, a.nw);
     const bool multi = !a.t.identity_conf;
     if (mode == QMC_EVAL_ELOC && multi)
-        hipLaunchKernelGGL((wf_kernel<double, NM, RAD, true, true>), g, dim3(kBlock), 0, s, a);
+        hipLaunchKernelGGL((wf_kernel<double, NM, RAD, true, true>), g, dim3(kBlock), multi_lds(a.t, true), s, a);
     else if (mode == QMC_EVAL_ELOC)
         hipLaunchKernelGGL((wf_kernel<double, NM, RAD, true, false>), g, dim3(kBlock), 0, s, a);
     else if (multi)
-        hipLaunchKernelGGL((wf_kernel<double, NM, RAD, false, true>), g, dim3(kBlock), 0, s, a);
+        hipLaunchKernelGGL((wf_kernel<double, NM, RAD, false, true>), g, dim3(kBlock), multi_lds(a.t, false), s, a);
     else
         hipLaunchKernelGGL((wf_kernel<double, NM, RAD, false, false>), g, dim3(kBlock), 0, s, a);
 }

@@ -176,7 +176,7 @@ int spec_%(name)s_sweep(const SArgs& a, int prec, hipStream_t s) {
     return 0;
 }
 
-int spec_%(name)s_sweep_batch(const SJob* jobs, int njobs, int nwaves, int prec, hipStream_t s) {
+int spec_%(name)s_sweep_batch(const SJob* jobs, int njobs, int nwaves, int ctab, int prec, hipStream_t s) {
     if (prec != QMC_PREC_MIXED) return -1;
 %(launch_batch)s
     return 0;
@@ -207,7 +207,7 @@ ELOC_MAX_W = 512
 
 NO_ELOC = '''
 int spec_%(name)s_wf(const KArgs&, int, int, hipStream_t) { return -1; }
-int spec_%(name)s_wf_batch(const WJob*, int, int, int, int, hipStream_t) { return -1; }
+int spec_%(name)s_wf_batch(const WJob*, int, int, int, int, int, hipStream_t) { return -1; }
 
 }  // namespace qmc
 '''
@@ -215,14 +215,15 @@ int spec_%(name)s_wf_batch(const WJob*, int, int, int, int, hipStream_t) { retur
 ELOC = '''
 int spec_%(name)s_wf(const KArgs& a, int prec, int mode, hipStream_t s) {
     if (prec != QMC_PREC_FP64 || mode != QMC_EVAL_ELOC) return -1;
-    hipLaunchKernelGGL((wf_kernel<double, kNM, kRAD, true, kMulti, AoSpec>), grid_for(a.t, a.nw), dim3(kBlock), 0, s, a);
+    hipLaunchKernelGGL((wf_kernel<double, kNM, kRAD, true, kMulti, AoSpec>), grid_for(a.t, a.nw), dim3(kBlock),
+                       kMulti ? multi_lds(a.t, true) : 0, s, a);
     return 0;
 }
 
-int spec_%(name)s_wf_batch(const WJob* jobs, int njobs, int nwaves, int prec, int mode, hipStream_t s) {
+int spec_%(name)s_wf_batch(const WJob* jobs, int njobs, int nwaves, int ctab, int prec, int mode, hipStream_t s) {
     if (prec != QMC_PREC_FP64 || mode != QMC_EVAL_ELOC) return -1;
-    hipLaunchKernelGGL((wf_batch_kernel<double, kNM, kRAD, true, kMulti, AoSpec>), grid_for_waves(nwaves), dim3(kBlock), 0,
-                       s, jobs, njobs, nwaves);
+    hipLaunchKernelGGL((wf_batch_kernel<double, kNM, kRAD, true, kMulti, AoSpec>), grid_for_waves(nwaves), dim3(kBlock),
+                       kBlockWaves * ctab, s, jobs, njobs, nwaves, ctab);
     return 0;
 }
 
@@ -260,15 +261,15 @@ def sweep_launch(nentry: int, nm: int) -> Tuple[str, str]:
     a walker's chain is the same alone and in a batch), else both without."""
     if nentry * nm * 4 <= WLDS_MAX_BYTES:
         single = ("    hipLaunchKernelGGL((sweep_kernel_wlds<float, kNM, kRAD, kMulti, AoSpec>), grid_for(a.t, a.nw), dim3(kBlock),\n"
-                  "                       (size_t)a.t.nentry * kNM * sizeof(float), s, a);")
+                  "                       wlds_bytes(a.t.nentry * kNM * (int)sizeof(float)) + (kMulti ? multi_lds(a.t, false) : 0), s, a);")
         batch = ("    hipLaunchKernelGGL((sweep_batch_kernel_wlds<float, kNM, kRAD, kMulti, AoSpec>), grid_for_waves(nwaves),\n"
-                 "                       dim3(kBlock), (kBlock / 64) * %d * sizeof(float), s, jobs, njobs, nwaves, %d);"
-                 % (nentry * nm, nentry * nm))
+                 "                       dim3(kBlock), wlds_bytes(kBlockWaves * %d * (int)sizeof(float)) + kBlockWaves * ctab, s,\n"
+                 "                       jobs, njobs, nwaves, %d, ctab);" % (nentry * nm, nentry * nm))
         return single, batch
-    single = ("    hipLaunchKernelGGL((sweep_kernel<float, kNM, kRAD, kMulti, AoSpec>), grid_for(a.t, a.nw), dim3(kBlock), 0, s, "
-              "a);")
-    batch = ("    hipLaunchKernelGGL((sweep_batch_kernel<float, kNM, kRAD, kMulti, AoSpec>), grid_for_waves(nwaves), dim3(kBlock), "
-             "0, s,\n                       jobs, njobs, nwaves);")
+    single = ("    hipLaunchKernelGGL((sweep_kernel<float, kNM, kRAD, kMulti, AoSpec>), grid_for(a.t, a.nw), dim3(kBlock),\n"
+              "                       kMulti ? multi_lds(a.t, false) : 0, s, a);")
+    batch = ("    hipLaunchKernelGGL((sweep_batch_kernel<float, kNM, kRAD, kMulti, AoSpec>), grid_for_waves(nwaves), dim3(kBlock),\n"
+             "                       kBlockWaves * ctab, s, jobs, njobs, nwaves, ctab);")
     return single, batch
 
 
@@ -290,9 +291,9 @@ def registry_source(layouts) -> str:
     decls, rows = "", ""
     for name, tab, nm, mc in layouts:
         decls += ("int spec_%(n)s_sweep(const SArgs&, int, hipStream_t);\n"
-                  "int spec_%(n)s_sweep_batch(const SJob*, int, int, int, hipStream_t);\n"
+                  "int spec_%(n)s_sweep_batch(const SJob*, int, int, int, int, hipStream_t);\n"
                   "int spec_%(n)s_wf(const KArgs&, int, int, hipStream_t);\n"
-                  "int spec_%(n)s_wf_batch(const WJob*, int, int, int, int, hipStream_t);\n"
+                  "int spec_%(n)s_wf_batch(const WJob*, int, int, int, int, int, hipStream_t);\n"
                   "int spec_%(n)s_hmc(const HArgs&, int, hipStream_t);\n" % dict(n=name))
         rows += ("        {0x%016xull, %d, %d, %s, \"%s\", &spec_%s_sweep, &spec_%s_sweep_batch, &spec_%s_wf, "
                  "&spec_%s_wf_batch, &spec_%s_hmc},\n" % (layout_signature(tab), nm, 16 * row_blocks(tab),
