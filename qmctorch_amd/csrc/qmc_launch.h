@@ -98,7 +98,7 @@ struct SpecEntry {
     uint64_t signature;  // layout_signature of the layout
     int nm;              // register bucket the kernels were built for
     int max_rows;        // lanes of real walkers per wavefront (G Ne) the sweeps' matrix tiles cover
-    bool multi;          // built for several configurations (else for the ground-state determinant)
+    bool single, multi;  // sweeps built for the ground-state determinant, for several configurations
     const char* name;
     int (*sweep)(const SArgs& a, int precision, hipStream_t s);
     int (*sweep_batch)(const SJob* jobs, int njobs, int nwaves, int ctab, int precision, hipStream_t s);
@@ -107,8 +107,8 @@ struct SpecEntry {
     int (*hmc)(const HArgs& a, int precision, hipStream_t s);  // mixed HMC / drift
 };
 
-// the generated layout with this signature, bucket and configuration kind
-// whose kernels cover `rows` lanes of real walkers per wavefront, or nullptr
+// the generated layout with this signature and bucket whose sweeps are built for
+// the configuration kind and cover `rows` lanes of real walkers per wavefront, or nullptr
 const SpecEntry* find_spec(uint64_t signature, int nm, int rows, bool multi);
 
 #define QMC_BY_RAD(fn, rad, ...) ((rad) == QMC_RADIAL_STO ? fn<QMC_RADIAL_STO>(__VA_ARGS__) : fn<QMC_RADIAL_GTO_PURE>(__VA_ARGS__))

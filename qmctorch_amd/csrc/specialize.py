@@ -189,7 +189,7 @@ HMC = '''
 constexpr int kMC = %(mc)d;
 
 int spec_%(name)s_hmc(const HArgs& a, int prec, hipStream_t s) {
-    if (prec != QMC_PREC_MIXED) return -1;
+    if (prec != QMC_PREC_MIXED || (a.t.identity_conf != 0) != (kMC == 1)) return -1;
     hipLaunchKernelGGL((hmc_kernel<float, kNM, kRAD, kMC, AoSpec>), grid_for(a.t, a.nw), dim3(kBlock), 0, s, a);
     return 0;
 }
@@ -214,14 +214,14 @@ int spec_%(name)s_wf_batch(const WJob*, int, int, int, int, int, hipStream_t) { 
 
 ELOC = '''
 int spec_%(name)s_wf(const KArgs& a, int prec, int mode, hipStream_t s) {
-    if (prec != QMC_PREC_FP64 || mode != QMC_EVAL_ELOC) return -1;
+    if (prec != QMC_PREC_FP64 || mode != QMC_EVAL_ELOC || (a.t.identity_conf == 0) != kMulti) return -1;
     hipLaunchKernelGGL((wf_kernel<double, kNM, kRAD, true, kMulti, AoSpec>), grid_for(a.t, a.nw), dim3(kBlock),
                        kMulti ? multi_lds(a.t, true) : 0, s, a);
     return 0;
 }
 
 int spec_%(name)s_wf_batch(const WJob* jobs, int njobs, int nwaves, int ctab, int prec, int mode, hipStream_t s) {
-    if (prec != QMC_PREC_FP64 || mode != QMC_EVAL_ELOC) return -1;
+    if (prec != QMC_PREC_FP64 || mode != QMC_EVAL_ELOC || (ctab > 0) != kMulti) return -1;
     hipLaunchKernelGGL((wf_batch_kernel<double, kNM, kRAD, true, kMulti, AoSpec>), grid_for_waves(nwaves), dim3(kBlock),
                        kBlockWaves * ctab, s, jobs, njobs, nwaves, ctab);
     return 0;
@@ -240,9 +240,9 @@ namespace qmc {
 #if !defined(__HIP_DEVICE_COMPILE__)
 const SpecEntry* find_spec(uint64_t signature, int nm, int rows, bool multi) {
     static const SpecEntry table[] = {
-%(rows)s        {0, 0, 0, false, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr}};
+%(rows)s        {0, 0, 0, false, false, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr}};
     for (const SpecEntry* e = table; e->name; ++e)
-        if (e->signature == signature && e->nm == nm && rows <= e->max_rows && multi == e->multi) return e;
+        if (e->signature == signature && e->nm == nm && rows <= e->max_rows && (multi ? e->multi : e->single)) return e;
     return nullptr;
 }
 #endif
@@ -255,22 +255,40 @@ const SpecEntry* find_spec(uint64_t signature, int nm, int rows, bool multi) {
 WLDS_MAX_BYTES = 8192
 
 
-def sweep_launch(nentry: int, nm: int) -> Tuple[str, str]:
-    """Launches of the single-system and batched sweeps: both with the W rows
-    staged in LDS when they fit (the two must run the same arithmetic, so that
-    a walker's chain is the same alone and in a batch), else both without."""
+def both_kinds(nm: int) -> bool:
+    """Whether ground states and expansions of a layout can share the bucket nm:
+    below the padded buckets each further orbital is a bucket of its own."""
+    return nm > 8
+
+
+def sweep_launch(nentry: int, nm: int, multi: bool) -> Tuple[str, str]:
+    """Launches of the single-system and batched sweeps of one configuration
+    kind: both with the W rows staged in LDS when they fit (the two must run the
+    same arithmetic, so that a walker's chain is the same alone and in a batch),
+    else both without."""
+    kind = "true" if multi else "false"
+    tables = ["multi_lds(a.t, false)", "kBlockWaves * ctab"] if multi else ["0", "0"]
     if nentry * nm * 4 <= WLDS_MAX_BYTES:
-        single = ("    hipLaunchKernelGGL((sweep_kernel_wlds<float, kNM, kRAD, kMulti, AoSpec>), grid_for(a.t, a.nw), dim3(kBlock),\n"
-                  "                       wlds_bytes(a.t.nentry * kNM * (int)sizeof(float)) + (kMulti ? multi_lds(a.t, false) : 0), s, a);")
-        batch = ("    hipLaunchKernelGGL((sweep_batch_kernel_wlds<float, kNM, kRAD, kMulti, AoSpec>), grid_for_waves(nwaves),\n"
-                 "                       dim3(kBlock), wlds_bytes(kBlockWaves * %d * (int)sizeof(float)) + kBlockWaves * ctab, s,\n"
-                 "                       jobs, njobs, nwaves, %d, ctab);" % (nentry * nm, nentry * nm))
-        return single, batch
-    single = ("    hipLaunchKernelGGL((sweep_kernel<float, kNM, kRAD, kMulti, AoSpec>), grid_for(a.t, a.nw), dim3(kBlock),\n"
-              "                       kMulti ? multi_lds(a.t, false) : 0, s, a);")
-    batch = ("    hipLaunchKernelGGL((sweep_batch_kernel<float, kNM, kRAD, kMulti, AoSpec>), grid_for_waves(nwaves), dim3(kBlock),\n"
-             "                       kBlockWaves * ctab, s, jobs, njobs, nwaves, ctab);")
+        rows = ["wlds_bytes(%d * (int)sizeof(float)) + " % (nentry * nm),
+                "wlds_bytes(kBlockWaves * %d * (int)sizeof(float)) + " % (nentry * nm)]
+        kernels, wstride = ["sweep_kernel_wlds", "sweep_batch_kernel_wlds"], "%d, " % (nentry * nm)
+    else:
+        rows, kernels, wstride = ["", ""], ["sweep_kernel", "sweep_batch_kernel"], ""
+    single = ("hipLaunchKernelGGL((%s<float, kNM, kRAD, %s, AoSpec>), grid_for(a.t, a.nw), dim3(kBlock),\n"
+              "                           %s, s, a);" % (kernels[0], kind, rows[0] + tables[0]))
+    batch = ("hipLaunchKernelGGL((%s<float, kNM, kRAD, %s, AoSpec>), grid_for_waves(nwaves), dim3(kBlock),\n"
+             "                           %s, s, jobs, njobs, nwaves, %sctab);" % (kernels[1], kind, rows[1] + tables[1], wstride))
     return single, batch
+
+
+def sweep_dispatch(nentry: int, nm: int, multi: bool) -> Tuple[str, str]:
+    """Bodies of the sweep launchers: the layout's own configuration kind, or both."""
+    own = sweep_launch(nentry, nm, multi)
+    if not both_kinds(nm):
+        return "    " + own[0], "    " + own[1]
+    # ground state : expansion (a batch of expansions has tables)
+    pairs = zip(sweep_launch(nentry, nm, False), sweep_launch(nentry, nm, True), ("a.t.identity_conf", "ctab == 0"))
+    return tuple("    if (%s)\n        %s\n    else\n        %s" % (test, g, e) for g, e, test in pairs)
 
 
 def unit_sources(name: str, tab, nm: int, mc: int = 1) -> Dict[str, str]:
@@ -279,7 +297,7 @@ def unit_sources(name: str, tab, nm: int, mc: int = 1) -> Dict[str, str]:
     instance (1, or QMC_MAXCONF)."""
     head = ROW % dict(name=name, ngroup=len(tab.grp_atom), nentry=len(tab.gao_mu), nm=nm, rad=int(tab.radial),
                       rowblocks=row_blocks(tab), body=row_source(tab), multi="true" if mc > 1 else "false")
-    single, batch = sweep_launch(len(tab.gao_mu), nm)
+    single, batch = sweep_dispatch(len(tab.gao_mu), nm, mc > 1)
     sweep = SWEEP % dict(name=name, launch=single, launch_batch=batch)
     return {"qmc_spec_%s_sweep.hip" % name: head + sweep,
             "qmc_spec_%s_eloc.hip" % name: head + (ELOC if len(tab.gao_mu) * nm <= ELOC_MAX_W else NO_ELOC) % dict(
@@ -295,10 +313,11 @@ def registry_source(layouts) -> str:
                   "int spec_%(n)s_wf(const KArgs&, int, int, hipStream_t);\n"
                   "int spec_%(n)s_wf_batch(const WJob*, int, int, int, int, int, hipStream_t);\n"
                   "int spec_%(n)s_hmc(const HArgs&, int, hipStream_t);\n" % dict(n=name))
-        rows += ("        {0x%016xull, %d, %d, %s, \"%s\", &spec_%s_sweep, &spec_%s_sweep_batch, &spec_%s_wf, "
+        single, multi = both_kinds(nm) or mc == 1, both_kinds(nm) or mc > 1
+        rows += ("        {0x%016xull, %d, %d, %s, %s, \"%s\", &spec_%s_sweep, &spec_%s_sweep_batch, &spec_%s_wf, "
                  "&spec_%s_wf_batch, &spec_%s_hmc},\n" % (layout_signature(tab), nm, 16 * row_blocks(tab),
-                                                           "true" if mc > 1 else "false", name, name, name, name, name,
-                                                           name))
+                                                           str(single).lower(), str(multi).lower(), name, name, name,
+                                                           name, name, name))
     return REGISTRY % dict(decls=decls, rows=rows)
 
 

@@ -15,7 +15,7 @@ import pytest
 import torch
 
 from qmctorch_amd import _native as N
-from qmctorch_amd.serving import catalog
+from qmctorch_amd.serving import BatchRunner, SystemContext, WalkerSet, catalog, sweep_each
 from tests import helpers
 
 pytestmark = pytest.mark.gpu
@@ -105,3 +105,31 @@ def test_generated_hmc_drift_matches_table_driven(system, configs, name):
     assert float(rel.median()) < 1e-6 and float(rel.max()) < 1e-4
     assert float((ls - lg).abs().max()) < 1e-4
     assert torch.equal(ss, sg)
+
+
+def test_generated_sweep_of_an_expansion_in_the_ground_states_bucket():
+    """Benzene CAS(2,2) has 22 columns, the ground state 21: one register bucket,
+    so the layout's generated sweep runs the expansion too, alone and in a batch
+    beside the ground state."""
+    _say("case generated sweep c6h6 cas(2,2)")
+    mol, wf = _wf("c6h6", "cas(2,2)")
+    plan = wf.device_plan()
+    assert plan.specialization == "c6h6"
+    pos = catalog.initial_positions(mol, 100, seed=7)
+    xs, ls, ns = _sweep(wf, pos, 20)
+    plan.set_specialized(False)
+    try:
+        xg, lg, ng = _sweep(wf, pos, 20)
+    finally:
+        plan.set_specialized(True)
+    same = (xs == xg).all(dim=1).double().mean().item()
+    _say("  walkers with identical trajectories %.4f, accept %d vs %d" % (same, int(ns.sum()), int(ng.sum())))
+    assert same >= 0.99
+    ctx = [SystemContext(w) for w in (wf, _wf("c6h6", "ground_state")[1])]
+    make = lambda: [WalkerSet(c, pos[:n].clone(), 5 + n) for c, n in zip(ctx, (33, 70))]
+    mix, alone = make(), make()
+    BatchRunner(4).sweep([(w, 6) for w in mix])
+    sweep_each([(w, 6) for w in alone])
+    torch.cuda.synchronize()
+    for a, b in zip(mix, alone):
+        assert torch.equal(a.pos, b.pos) and torch.equal(a.logabs, b.logabs) and int(a.naccept.sum()) > 0
