@@ -1880,9 +1880,18 @@ __device__ __forceinline__ void sweep_walkers(const SArgs& a, const WalkerLane& 
 
 // The 16- and 24-orbital buckets (one or two walkers per wavefront) are held to
 // two waves per SIMD, so a second wavefront covers the latency of the FP64
-// elimination; left alone the compiler keeps VGPRs and AGPRs for one.
+// elimination; left alone the compiler keeps VGPRs and AGPRs for one.  So are
+// expansions in 7 columns, whose minors take just over half of the registers:
+// water CAS(2,3), FP64, 131072 walkers x 8 steps 2980 -> 1970 us, 8192 walkers
+// 354 -> 272; 1000 walkers, which do not fill the chip, 222 -> 241 (57 VGPRs
+// spilled).
+template <int NM, bool MULTI>
+constexpr int sweep_waves() {
+    return NM >= 16 || (MULTI && NM == kMaxMinors) ? 2 : 1;
+}
+
 template <typename T, int NM, int RAD, bool MULTI, typename AO = AoGeneric>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NM >= 16 ? 2 : 1))) void sweep_kernel(
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sweep_waves<NM, MULTI>()))) void sweep_kernel(
     SArgs a) {
     const WalkerLane L = lane_layout(a.t, a.nw);
     if ((int64_t)L.wave * L.G >= a.nw) return;
@@ -1944,7 +1953,7 @@ __global__ __launch_bounds__(64) void sweep_batch_kernel_exc(const SJob* __restr
 }
 
 template <typename T, int NM, int RAD, bool MULTI, typename AO = AoGeneric>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NM >= 16 ? 2 : 1))) void sweep_batch_kernel(
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sweep_waves<NM, MULTI>()))) void sweep_batch_kernel(
     const SJob* __restrict__ jobs, int njobs, int nwaves, int ctab) {
     const int wave = global_wave();
     if (wave >= nwaves) return;
