@@ -936,20 +936,21 @@ __device__ __forceinline__ void gather_conf(const Tables& t, const WalkerLane& L
 // blocks, the terms are taken relative to the largest power of two among them,
 // so that no ratio of determinants leaves the range.
 // The table is dynamic LDS, at byte coff of qmc_dyn_lds for this wavefront
-// (combine_table_bytes each): an entry per group and configuration.  Static
+// (combine_table_bytes each): an entry per group and configuration, the groups
+// an odd number of entries apart (their walkers' reads meet in no LDS bank).  Static
 // tables for the most any plan can have (64 groups, 8 configurations: 24 KB a
 // block, 40 KB with traces) cost the larger kernels a block a CU: benzene
 // CAS(2,2), FP64, 4096 walkers, psi 478 -> 230 us and 4 sweep steps 2345 -> 1294
 // us; E_L of water CAS(2,2), 131072 walkers, 462 -> 265 us.
 __host__ __device__ __forceinline__ int combine_table_bytes(const Tables& t, bool kin) {
-    return t.nconf_max * 2 * (64 / t.nelec) * (kin ? 20 : 12);
+    return (t.nconf_max | 1) * 2 * (64 / t.nelec) * (kin ? 20 : 12);
 }
 
 template <int NM, bool KIN, typename T>
 __device__ __forceinline__ void slater_combine(const Tables& t, const QmcParams& prm, const WalkerLane& L, int coff,
                                                const T (&mo)[NM], const double (&bk)[NM], double& logabs,
                                                double& sgn, double& kin) {
-    const int ngrp = 2 * L.G, nent = t.nconf_max * ngrp;  // entry [configuration][walker of the wavefront][spin]
+    const int per = t.nconf_max | 1, nent = 2 * L.G * per;  // entry [walker of the wavefront][spin][configuration]
     double* dt = (double*)(qmc_dyn_lds + coff);
     double* tt = dt + (KIN ? nent : 0);
     int* et = (int*)(tt + nent);
@@ -981,7 +982,7 @@ __device__ __forceinline__ void slater_combine(const Tables& t, const QmcParams&
         if (c == 0) eref = ex;
         common = common && ex == eref;
         const bool first = L.lane_real && L.myrow == 0;
-        const int at = c * ngrp + 2 * L.wl + L.spin;
+        const int at = (2 * L.wl + L.spin) * per + c;
         if (first) {
             dt[at] = d;
             et[at] = ex;
@@ -998,7 +999,7 @@ __device__ __forceinline__ void slater_combine(const Tables& t, const QmcParams&
     wave_lds_sync();
     const bool down = t.ndown > 0;
     // this walker's entries (a lane past the last walker reads another's)
-    const int up0 = 2 * (L.lane_real ? L.wl : 0), dn0 = up0 + (down ? 1 : 0);
+    const int up0 = 2 * (L.lane_real ? L.wl : 0) * per, dn0 = up0 + (down ? per : 0);
     int emax = et[up0] + (down ? et[dn0] : 0);
     double s = 0.0, st = 0.0;
     auto add = [&](int iu, int id, double dn) {
@@ -1011,19 +1012,19 @@ __device__ __forceinline__ void slater_combine(const Tables& t, const QmcParams&
     if (!__any(!common && L.lane_real)) {
 #pragma unroll 4
         for (int n = 0; n < t.nci; ++n) {
-            const int iu = t.ci_up[n] * ngrp + up0, id = t.ci_dn[n] * ngrp + dn0;
+            const int iu = up0 + t.ci_up[n], id = dn0 + t.ci_dn[n];
             const double dd = dt[id];
             add(iu, id, ldc(prm.ci, n) * dt[iu] * (down ? dd : 1.0));
         }
     } else {
         emax = -(1 << 30);
         for (int n = 0; n < t.nci; ++n) {
-            const int iu = t.ci_up[n] * ngrp + up0, id = t.ci_dn[n] * ngrp + dn0;
+            const int iu = up0 + t.ci_up[n], id = dn0 + t.ci_dn[n];
             const bool zero = dt[iu] == 0.0 || (down && dt[id] == 0.0);
             emax = zero ? emax : max(emax, et[iu] + (down ? et[id] : 0));
         }
         for (int n = 0; n < t.nci; ++n) {
-            const int iu = t.ci_up[n] * ngrp + up0, id = t.ci_dn[n] * ngrp + dn0;
+            const int iu = up0 + t.ci_up[n], id = dn0 + t.ci_dn[n];
             const double dd = dt[id];
             add(iu, id, ldexp(ldc(prm.ci, n) * dt[iu] * (down ? dd : 1.0), et[iu] + (down ? et[id] : 0) - emax));
         }
@@ -1883,11 +1884,14 @@ __device__ __forceinline__ void sweep_walkers(const SArgs& a, const WalkerLane& 
 // elimination; left alone the compiler keeps VGPRs and AGPRs for one.  So are
 // expansions in 7 columns, whose minors take just over half of the registers:
 // water CAS(2,3), FP64, 131072 walkers x 8 steps 2980 -> 1970 us, 8192 walkers
-// 354 -> 272; 1000 walkers, which do not fill the chip, 222 -> 241 (57 VGPRs
-// spilled).
+// 354 -> 275; 1000 walkers, which do not fill the chip, 222 -> 242 (61 VGPRs
+// spilled).  Those of 4 and 8 columns are at the limit of three waves (169
+// VGPRs left alone, 168 fit): N2 CAS(2,2), FP64, 32768 walkers x 4 steps 471 us
+// with three, 566 with two.
 template <int NM, bool MULTI>
 constexpr int sweep_waves() {
-    return NM >= 16 || (MULTI && NM == kMaxMinors) ? 2 : 1;
+    if (NM >= 16 || (MULTI && NM == kMaxMinors)) return 2;
+    return MULTI && (NM <= 4 || NM == 8) ? 3 : 1;
 }
 
 template <typename T, int NM, int RAD, bool MULTI, typename AO = AoGeneric>
