@@ -16,6 +16,9 @@ static void go(const WJob* jobs, int njobs, int nwaves, int ctab, bool multi, in
         hipLaunchKernelGGL((wf_batch_kernel<double, NM, RAD, true, false>), g, dim3(kBlock), kBlockWaves * ctab, s, jobs, njobs, nwaves, ctab);
     else if (multi)
         hipLaunchKernelGGL((wf_batch_kernel<double, NM, RAD, false, true>), g, dim3(kBlock), kBlockWaves * ctab, s, jobs, njobs, nwaves, ctab);
+    else if (psi_may_eliminate<NM>() && psi_eliminates(nwaves))
+        hipLaunchKernelGGL((wf_batch_kernel<double, NM, RAD, false, false, AoGeneric, psi_may_eliminate<NM>()>), g,
+                           dim3(kBlock), kBlockWaves * ctab, s, jobs, njobs, nwaves, ctab);
     else
         hipLaunchKernelGGL((wf_batch_kernel<double, NM, RAD, false, false>), g, dim3(kBlock), kBlockWaves * ctab, s, jobs, njobs, nwaves, ctab);
 }

@@ -1549,7 +1549,9 @@ __device__ __forceinline__ uint32_t touch_tables(const Tables& t, const QmcParam
 // of several configurations (up to QMC_MAXCONF unique ones per spin); without
 // it the plan is the ground-state determinant (identity_conf) and the kernel
 // holds none of their registers and code.  coff: slater_combine's table.
-template <typename T, int NM, int RAD, bool ELOC, bool MULTI, typename AO = AoGeneric, bool EXC = false>
+// ELIM: psi of a single determinant by elimination where there are minors too.
+template <typename T, int NM, int RAD, bool ELOC, bool MULTI, typename AO = AoGeneric, bool EXC = false,
+          bool ELIM = false>
 __device__ __forceinline__ void wf_walkers(const KArgs& a, const WalkerLane& L, int coff = 0) {
     const Tables& t = a.t;
     const double* p = a.pos + (size_t)L.wclamp * 3 * t.nelec + 3 * L.e;
@@ -1584,7 +1586,7 @@ __device__ __forceinline__ void wf_walkers(const KArgs& a, const WalkerLane& L, 
         AO::template row<T, RAD, false>(t, a.p, x, y, z, sink);
     }
     double logabs, sgn, kin = 0.0, logj, svee = 0.0, sven = 0.0;
-    if constexpr (!EXC && !MULTI && use_minors<NM>()) {
+    if constexpr (!EXC && !MULTI && use_minors<NM>() && !ELIM) {
         double yc[NM];
         slater_single_minors<NM, ELOC>(t, a.p, L, mo, log(fabs(ldc(a.p.ci, 0))), 0.5 * kee + ken, logabs, sgn, logj, yc);
         if constexpr (ELOC) {
@@ -1649,11 +1651,12 @@ constexpr int wf_waves() {
     return NM <= (AO::kEntries > 0 ? 5 : 3) ? 3 : (NM <= 12 ? 2 : 1);
 }
 
-template <typename T, int NM, int RAD, bool ELOC, bool MULTI, typename AO = AoGeneric>
+template <typename T, int NM, int RAD, bool ELOC, bool MULTI, typename AO = AoGeneric, bool ELIM = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(wf_waves<NM, AO>()))) void wf_kernel(KArgs a) {
     const WalkerLane L = lane_layout(a.t, a.nw);
     if ((int64_t)L.wave * L.G >= a.nw) return;  // whole wavefront beyond the batch
-    wf_walkers<T, NM, RAD, ELOC, MULTI, AO>(a, L, MULTI ? combine_table(0, combine_table_bytes(a.t, ELOC)) : 0);
+    wf_walkers<T, NM, RAD, ELOC, MULTI, AO, false, ELIM>(
+        a, L, MULTI ? combine_table(0, combine_table_bytes(a.t, ELOC)) : 0);
 }
 
 // Kernels of exc_mode plans: one wavefront per block, dynamic LDS of
@@ -1672,7 +1675,7 @@ struct WJob {
     int64_t wave0;
 };
 
-template <typename T, int NM, int RAD, bool ELOC, bool MULTI, typename AO = AoGeneric>
+template <typename T, int NM, int RAD, bool ELOC, bool MULTI, typename AO = AoGeneric, bool ELIM = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(wf_waves<NM, AO>()))) void wf_batch_kernel(const WJob* __restrict__ jobs, int njobs, int nwaves, int ctab) {
     const int wave = global_wave();
     if (wave >= nwaves) return;
@@ -1680,7 +1683,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(wf_waves
     const KArgs a = jobs[j].a;
     const WalkerLane L = lane_layout_w(a.t, a.nw, wave - (int)jobs[j].wave0);
     if ((int64_t)L.wave * L.G >= a.nw) return;
-    wf_walkers<T, NM, RAD, ELOC, MULTI, AO>(a, L, MULTI ? combine_table(0, ctab) : 0);
+    wf_walkers<T, NM, RAD, ELOC, MULTI, AO, false, ELIM>(a, L, MULTI ? combine_table(0, ctab) : 0);
 }
 
 // wf_batch_kernel for excitation plans: one wavefront per block (as

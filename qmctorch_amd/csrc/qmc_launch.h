@@ -27,6 +27,21 @@ inline dim3 grid_for(const Tables& t, int64_t nw) {
     return dim3((unsigned)((waves + (kBlock / 64) - 1) / (kBlock / 64)));
 }
 
+// psi of a single determinant of 7 columns: its minors hold 200 to 235 VGPRs, two
+// waves a SIMD, where the elimination runs four, so the elimination takes over
+// once there are more waves than SIMDs (1024).  N2, minors / elimination, us:
+// mixed, 25 waves 13.9 / 15.7, 1024 waves 14.4 / 16.3, 4096 waves 29.6 / 23.8,
+// 16384 waves 99 / 67; FP64 16.7 / 18.1, 19.3 / 18.8, 37 / 31, 122 / 95.
+template <int NM>
+constexpr bool psi_may_eliminate() {
+    return NM == kMaxMinors;
+}
+inline bool psi_eliminates(int64_t waves) { return waves > 1024; }
+inline int64_t wave_count(const Tables& t, int64_t nw) {
+    const int G = 64 / t.nelec;
+    return (nw + G - 1) / G;
+}
+
 // Each family is compiled once per radial type (-DQMC_RAD=0 gto_pure, 1 sto);
 // the specialisations live in different translation units.
 template <int RAD> int launch_wf_f32(const KArgs& a, int mode, hipStream_t s);

@@ -11,10 +11,14 @@ template <int NM, int RAD>
 static void go(const KArgs& a, int mode, hipStream_t s) {
     // psi only: local energies are evaluated by the FP64 kernels in every precision
     (void)mode;
-    if (a.t.identity_conf)
-        hipLaunchKernelGGL((wf_kernel<float, NM, RAD, false, false>), grid_for(a.t, a.nw), dim3(kBlock), 0, s, a);
+    const dim3 g = grid_for(a.t, a.nw);
+    if (!a.t.identity_conf)
+        hipLaunchKernelGGL((wf_kernel<float, NM, RAD, false, true>), g, dim3(kBlock), multi_lds(a.t, false), s, a);
+    else if (psi_may_eliminate<NM>() && psi_eliminates(wave_count(a.t, a.nw)))
+        hipLaunchKernelGGL((wf_kernel<float, NM, RAD, false, false, AoGeneric, psi_may_eliminate<NM>()>), g,
+                           dim3(kBlock), 0, s, a);
     else
-        hipLaunchKernelGGL((wf_kernel<float, NM, RAD, false, true>), grid_for(a.t, a.nw), dim3(kBlock), multi_lds(a.t, false), s, a);
+        hipLaunchKernelGGL((wf_kernel<float, NM, RAD, false, false>), g, dim3(kBlock), 0, s, a);
 }
 
 template <int RAD>

@@ -17,6 +17,9 @@ static void go(const KArgs& a, int mode, hipStream_t s) {
         hipLaunchKernelGGL((wf_kernel<double, NM, RAD, true, false>), g, dim3(kBlock), 0, s, a);
     else if (multi)
         hipLaunchKernelGGL((wf_kernel<double, NM, RAD, false, true>), g, dim3(kBlock), multi_lds(a.t, false), s, a);
+    else if (psi_may_eliminate<NM>() && psi_eliminates(wave_count(a.t, a.nw)))
+        hipLaunchKernelGGL((wf_kernel<double, NM, RAD, false, false, AoGeneric, psi_may_eliminate<NM>()>), g,
+                           dim3(kBlock), 0, s, a);
     else
         hipLaunchKernelGGL((wf_kernel<double, NM, RAD, false, false>), g, dim3(kBlock), 0, s, a);
 }

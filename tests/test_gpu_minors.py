@@ -12,7 +12,7 @@ import pytest
 import torch
 
 from qmctorch_amd.scf import Molecule
-from tests import helpers
+from tests import helpers, systems
 
 pytestmark = pytest.mark.gpu
 
@@ -110,3 +110,24 @@ def test_ci_terms_far_from_the_nuclei(n):
           % (ref.min(), ref.max(), int(ok.sum()), (la.cpu() - ref).abs()[ok].max()), flush=True)
     assert int(ok.sum()) >= 5
     assert ((la.cpu() - ref).abs() <= bound)[ok].all() and torch.equal(sg.cpu()[ok], tot.sign()[ok])
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_psi_of_seven_columns_on_both_sides_of_the_wave_rule(precision):
+    """1024 wavefronts of N2 expand minors, 1025 eliminate: the same rows, so the
+    determinants differ by roundings times the condition of the blocks."""
+    print("case minors N2 wave rule", precision, flush=True)
+    mol = systems.n2()
+    wf, orc = helpers.make_pair(mol, w_ee=0.9, w_en=1.0)
+    pos = helpers.positions(mol, 4100, seed=2)
+    few, many = wf.log_psi(pos[:4096].cuda(), precision), wf.log_psi(pos.cuda(), precision)
+    mo = orc.mo(orc.ao(pos[:4096])).detach()
+    rows = mo / mo.abs().amax(-1, keepdim=True)
+    cond = torch.linalg.cond(rows[:, :7, :7]) + torch.linalg.cond(rows[:, 7:, :7])
+    # 7^2 roundings of 1.1e-16 in either way
+    assert ((few[0] - many[0][:4096]).abs().cpu() <= 2 * 49 * 1.1e-16 * cond).all()
+    ok = cond < 1e12
+    assert torch.equal(few[1].cpu()[ok], many[1][:4096].cpu()[ok]) and int(ok.sum()) > 4000
+    if precision == "fp64":
+        psi, psi_o = wf(pos.cuda()).detach().cpu().view(-1)[-300:], orc(pos[-300:]).detach().view(-1)
+        assert float(((psi - psi_o).abs() / psi_o.abs()).max()) < 1e-9
