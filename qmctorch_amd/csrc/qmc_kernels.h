@@ -671,7 +671,8 @@ __device__ __forceinline__ bool minors_full(const Tables& t) {
 // Stores this lane's row.  SCALE (FP64 rows): divided by a power of two that
 // brings its largest entry into [1/2, 1), so that products of N entries far
 // from every nucleus neither underflow nor overflow; returns that exponent.
-// FP32 rows need none (seven factors above 2^-149 stay above 2^-1074).
+// FP32 rows need none for one block (seven factors above 2^-149 stay above
+// 2^-1074); slater_combine, which multiplies two, scales their determinants.
 // With groups of fewer than NM rows (full = false) the unit rows follow.
 template <int NM, bool SCALE, typename S>
 __device__ __forceinline__ int stage_minor_row(const WalkerLane& L, const S (&mo)[NM], bool full, double* rows) {
@@ -932,9 +933,10 @@ __device__ __forceinline__ void gather_conf(const Tables& t, const WalkerLane& L
 // logarithm per configuration, an exponential per term and an eight-way
 // register selection per read: LiH in a Slater basis, four determinants,
 // FP64, 1000 walkers x 100 steps, 1243 -> 872 us.  The configurations of minors
-// share ex (their row scales) unless one was weak; otherwise, and for eliminated
-// blocks, the terms are taken relative to the largest power of two among them,
-// so that no ratio of determinants leaves the range.
+// share ex (their row scales; none for FP32 rows) unless one was weak, or one of
+// FP32 rows is far from 1; otherwise, and for eliminated blocks, the terms are
+// taken relative to the largest power of two among them, so that neither a
+// product nor a ratio of determinants leaves the range.
 // The table is dynamic LDS, at byte coff of qmc_dyn_lds for this wavefront
 // (combine_table_bytes each): an entry per group and configuration, the groups
 // an odd number of entries apart (their walkers' reads meet in no LDS bank).  Static
@@ -978,6 +980,14 @@ __device__ __forceinline__ void slater_combine(const Tables& t, const QmcParams&
             double r[NM];
             gather_conf<NM>(t, L, c, mo, r);
             lane_inverse<NM>(L, t.nsig_max, r, d, ex, a);
+        }
+        if constexpr (use_minors<NM>() && !SCALE) {
+            // determinants of unscaled FP32 rows: a product of two, times a CI
+            // weight, stays in range unless one is smaller or larger than this
+            const int e = __builtin_amdgcn_frexp_exp(d);  // 0 of zeros and non-numbers
+            const bool far = (unsigned)(e + 400) > 800u;
+            ex = far ? e : 0;
+            d = far ? __builtin_amdgcn_frexp_mant(d) : d;
         }
         if (c == 0) eref = ex;
         common = common && ex == eref;

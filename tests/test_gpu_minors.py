@@ -131,3 +131,44 @@ def test_psi_of_seven_columns_on_both_sides_of_the_wave_rule(precision):
     if precision == "fp64":
         psi, psi_o = wf(pos.cuda()).detach().cpu().view(-1)[-300:], orc(pos[-300:]).detach().view(-1)
         assert float(((psi - psi_o).abs() / psi_o.abs()).max()) < 1e-9
+
+def _beside_the_chain(mol, nw, rho, seed):
+    """Electrons of both spins alternating along the chain, each rho from its atom
+    and the chain's axis: far from every nucleus, their rows well apart."""
+    rng = np.random.default_rng(seed)
+    atom = np.empty(mol.nelec, dtype=int)
+    atom[:mol.nup], atom[mol.nup:] = np.arange(0, mol.nelec, 2), np.arange(1, mol.nelec, 2)
+    phi = rng.uniform(0, 2 * np.pi, (nw, mol.nelec))
+    d = np.stack([rho * np.cos(phi), rho * np.sin(phi), rng.uniform(-0.3, 0.3, phi.shape)], -1)
+    return torch.as_tensor((np.asarray(mol.atom_coords)[atom] + d).reshape(nw, -1))
+
+
+def test_mixed_ci_terms_whose_product_leaves_the_double_range():
+    """FP32 rows near 1e-30: each determinant of six is a double, no product of an
+    up and a down one is."""
+    print("case minors CI far H12 mixed", flush=True)
+    mol = _chain(12)
+    wf, orc = helpers.make_pair(mol, configs="cas(2,2)", w_ee=1.0, w_en=1.0)
+    ci = torch.linspace(1.0, 0.1, wf.nci, dtype=torch.float64)
+    with torch.no_grad():
+        wf.fc.weight.copy_(ci.view(1, -1))
+    pos = _beside_the_chain(mol, 33, 23.5, 1)
+    la, sg = (v.cpu() for v in wf.log_psi(pos.cuda(), "mixed"))
+    ref, ref_sg = (v.cpu() for v in wf.log_psi(pos.cuda(), "fp64"))
+    rows = orc.mo(orc.ao(pos)).detach()
+    rows = rows / rows.abs().amax(-1, keepdim=True)
+    cond, terms = 0.0, []
+    for c, cu, cd in zip(ci, *wf.configs):
+        up, dn = rows[:, :mol.nup][..., cu.long()], rows[:, mol.nup:][..., cd.long()]
+        cond = cond + torch.linalg.cond(up) + torch.linalg.cond(dn)
+        terms.append(c * torch.linalg.det(up) * torch.linalg.det(dn))
+    terms = torch.stack(terms, 1)
+    # an exponential of an FP32 argument near -67, itself good to 4 roundings, is
+    # good to 2e-5; carried through the determinants and the sum
+    bound = 2e-5 * mol.nelec * cond * terms.abs().sum(1) / terms.sum(1).abs()
+    ok = bound < 0.3
+    print("  log|psi| from %.0f to %.0f, %d walkers compared, largest difference %.1e"
+          % (ref.min(), ref.max(), int(ok.sum()), (la - ref).abs()[ok].max()), flush=True)
+    slater = ref - orc.jastrow(pos).detach().view(-1).log()
+    assert float(slater.max()) < -745.0 and int(ok.sum()) >= 15  # below the smallest double
+    assert ((la - ref).abs() <= bound)[ok].all() and torch.equal(sg[ok], ref_sg[ok])
