@@ -28,7 +28,8 @@ namespace qmc {
 // than an elimination does, so FP64 blocks whose determinant, of rows scaled to
 // a largest entry of 1/2 to 1, is below kWeakDet are eliminated instead: 1e-5
 // of the groups above, and the quantiles stay at or below the elimination's
-// for walkers spread two and four times as far.
+// for walkers spread two and four times as far.  FP32 rows are not scaled, and
+// their own rounding is larger than either way's.
 constexpr int kMaxMinors = 7;
 
 constexpr double kWeakDet = 1e-6;

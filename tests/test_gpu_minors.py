@@ -172,3 +172,50 @@ def test_mixed_ci_terms_whose_product_leaves_the_double_range():
     slater = ref - orc.jastrow(pos).detach().view(-1).log()
     assert float(slater.max()) < -745.0 and int(ok.sum()) >= 15  # below the smallest double
     assert ((la - ref).abs() <= bound)[ok].all() and torch.equal(sg[ok], ref_sg[ok])
+
+@pytest.mark.parametrize("n", [2, 5, 9, 13])
+def test_mixed_drift_beside_an_electron_beyond_the_fp32_range(n):
+    """An up electron so far out that its FP32 orbitals are zero: psi is zero, its
+    block has no part in the drift (the up electrons keep the Jastrow factor's),
+    the down electrons' is what it is."""
+    print("case minors zero row H%d" % n, flush=True)
+    mol = _chain(n)
+    wf, orc = helpers.make_pair(mol, w_ee=1.0, w_en=1.0)
+    pos = helpers.positions(mol, 67, seed=n).view(67, n, 3)
+    pos[:, 0, 0] += 60.0
+    pos = pos.reshape(67, -1)
+    drift, la, _ = (v.cpu() for v in wf.drift(pos.cuda(), "mixed"))
+    assert bool((la == -float("inf")).all())
+    x = pos.clone().requires_grad_()
+    mo = orc.mo(orc.ao(x))
+    dn = mo[:, mol.nup:, :mol.ndown]
+    log = torch.linalg.slogdet(dn)[1].sum() if mol.ndown else 0.0
+    ref = torch.autograd.grad(log + orc.jastrow(x).log().sum(), x)[0].view(67, n, 3)
+    # FP32 rows are good to about 10 roundings of 6e-8 of their terms' sum without
+    # signs, their gradients to 2 sqrt(13) = 7 times that (the tightest exponent);
+    # the inverse carries both into the drift
+    ao = orc.ao(pos).detach()
+    terms = ao.abs() @ orc.mo(torch.eye(ao.shape[-1]).to(ao)[None])[0].detach().abs()
+    inv = torch.linalg.matrix_norm(torch.linalg.inv(dn.detach()), 2)
+    bound = 4.2e-6 * (1.0 + inv * terms[..., :mol.ndown].amax((1, 2)))[:, None] * (1.0 + ref.norm(dim=-1))
+    assert ((drift - ref).norm(dim=-1) <= bound).all()
+    assert float((bound < 1e-2).double().mean()) > 0.5  # and mean something
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_drift_of_an_expansion_with_a_zero_determinant(precision):
+    """A virtual orbital that is zero everywhere: the configurations that hold it
+    have no determinant and no part in the drift."""
+    print("case minors zero configuration", precision, flush=True)
+    mol = _chain(6)
+    wf, _ = helpers.make_pair(mol, configs="cas(2,2)", w_ee=1.0, w_en=1.0)
+    one, _ = helpers.make_pair(mol, w_ee=1.0, w_en=1.0)
+    with torch.no_grad():
+        wf.mo.mo_modifier[:, mol.nup] = 0.0
+    x = helpers.positions(mol, 67, seed=4).cuda()
+    got, want = wf.drift(x, precision), one.drift(x, precision)
+    # two instances of the kernel: rows one rounding apart (1e-16, 6e-8), times the
+    # blocks' condition, below 1e4 for 67 walkers around their atoms
+    tol = 1e-10 if precision == "fp64" else 1e-3
+    assert float(((got[0] - want[0]).norm(dim=-1) / (1.0 + want[0].norm(dim=-1))).max()) < tol
+    assert torch.equal(got[2], want[2])
