@@ -72,7 +72,7 @@ typedef struct QmcSystemDesc {
     const int32_t* grp_prim_src; /* [sum nprim] index into bas_exp */
     const int32_t* grp_ao0;      /* [ngroup] offset into AO entries */
     const int32_t* grp_nao;      /* [ngroup] */
-    const int32_t* grp_tight;    /* [ngroup] 1: evaluated in FP64 by the mixed local energy, or NULL */
+    const int32_t* grp_tight;    /* not used: [ngroup] of 0 and 1, or NULL (every local energy is FP64) */
     int32_t nentry;              /* number of AO entries */
     const int32_t* gao_mu;       /* [nentry] */
     const int32_t* gao_k;        /* [nentry] */

@@ -77,7 +77,6 @@ uint64_t layout_signature(const QmcSystemDesc* d) {
     f.words(d->grp_prim0, d->ngroup);
     f.words(d->grp_ao0, d->ngroup);
     f.words(d->grp_nao, d->ngroup);
-    f.words(d->grp_tight, d->ngroup);
     f.word(d->nentry);
     f.words(d->gao_mu, d->nentry);
     f.words(d->gao_k, d->nentry);
@@ -383,7 +382,6 @@ int qmc_plan_create(const QmcSystemDesc* d, QmcPlan** out) {
         p->nexp_grp = nprim_tot;
         t.grp_ao0 = (decltype(t.grp_ao0))p->upload(d->grp_ao0, d->ngroup);
         t.grp_nao = (decltype(t.grp_nao))p->upload(d->grp_nao, d->ngroup);
-        t.grp_tight = (decltype(t.grp_tight))p->upload(d->grp_tight, d->grp_tight ? d->ngroup : 0);
         t.gao_mu = (decltype(t.gao_mu))p->upload(d->gao_mu, d->nentry);
         t.gao_k = (decltype(t.gao_k))p->upload(d->gao_k, d->nentry);
         t.gao_K = (decltype(t.gao_K))p->upload(d->gao_K, (size_t)d->nentry * QMC_MAXP);

@@ -41,7 +41,6 @@ struct Tables {
     const QMC_CONST int* grp_prim_src;
     const QMC_CONST int* grp_ao0;
     const QMC_CONST int* grp_nao;
-    const QMC_CONST int* grp_tight;
     const QMC_CONST int* gao_mu;
     const QMC_CONST int* gao_k;
     const QMC_CONST double* gao_K;

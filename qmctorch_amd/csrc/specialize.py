@@ -38,7 +38,7 @@ def layout_signature(tab) -> int:
     and 32-bit little-endian encoding as layout_signature in qmc_abi.hip)."""
     h = FNV_OFFSET
     h = _fnv(h, [tab.radial, tab.natom, len(tab.grp_atom)])
-    for arr in (tab.grp_atom, tab.grp_nprim, tab.grp_prim0, tab.grp_ao0, tab.grp_nao, tab.grp_tight):
+    for arr in (tab.grp_atom, tab.grp_nprim, tab.grp_prim0, tab.grp_ao0, tab.grp_nao):
         h = _fnv(h, arr)
     h = _fnv(h, [len(tab.gao_mu)])
     h = _fnv(h, tab.gao_mu)

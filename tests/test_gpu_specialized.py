@@ -7,6 +7,7 @@ within 1e-13 relative, the mixed-precision sweep walker for walker, and the
 mixed-precision drift of the HMC kernel within FP32 rounding (1e-4 relative
 to 1 + |drift|, median below 1e-6).
 """
+import ctypes
 import math
 import sys
 
@@ -133,3 +134,23 @@ def test_generated_sweep_of_an_expansion_in_the_ground_states_bucket():
     torch.cuda.synchronize()
     for a, b in zip(mix, alone):
         assert torch.equal(a.pos, b.pos) and torch.equal(a.logabs, b.logabs) and int(a.naccept.sum()) > 0
+
+
+def test_layout_does_not_depend_on_the_unused_table():
+    """grp_tight is in the description's struct and in nothing else: without it, with
+    zeros and with ones the plan has the layout's kernels."""
+    _say("case unused table")
+    mol, wf = _wf("h2o", "ground_state")
+    tables = wf.device_plan().tables
+    lib = N.load()
+    for flags in (None, 0, 1):
+        d = tables.desc()
+        keep = np.full(d.ngroup, flags or 0, dtype=np.int32)
+        if flags is not None:
+            d.grp_tight = keep.ctypes.data_as(N.c_i32p)
+        h = ctypes.c_void_p()
+        N.check(lib.qmc_plan_create(ctypes.byref(d), ctypes.byref(h)))
+        try:
+            assert lib.qmc_plan_specialization(h) == b"h2o", flags
+        finally:
+            lib.qmc_plan_destroy(h)
