@@ -96,3 +96,14 @@ def test_one_and_few_walkers_chain_is_walker_zero_of_a_batch(nw):
     a, b = chain(nw), chain(64)
     assert torch.isfinite(a).all()
     assert torch.equal(a, b[:nw])
+
+
+def test_current_stream_is_torchs(monkeypatch):
+    """By either call: the default stream, and a side stream inside its context."""
+    _say("case current stream")
+    for raw in (N._raw_stream, None):
+        monkeypatch.setattr(N, "_raw_stream", raw)
+        assert N.current_stream() == torch.cuda.current_stream().cuda_stream
+        side = torch.cuda.Stream()
+        with torch.cuda.stream(side):
+            assert N.current_stream() == side.cuda_stream

@@ -203,3 +203,12 @@ def test_plan_create_rejects_bad_counts_and_missing_tables():
     d.nentry = d.nentry - 1  # the last group's entries then run past nentry
     assert lib.qmc_plan_create(ctypes.byref(d), ctypes.byref(h)) == N.QMC_ERR_ARG
     assert not h.value
+
+
+def test_current_stream_without_the_private_call(monkeypatch):
+    """The raw-stream call is private to torch: without it the Stream object serves."""
+    import types
+
+    monkeypatch.setattr(N, "_raw_stream", None)
+    monkeypatch.setattr(N.torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=0x5EED))
+    assert N.current_stream() == 0x5EED
