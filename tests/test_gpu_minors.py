@@ -219,3 +219,187 @@ def test_drift_of_an_expansion_with_a_zero_determinant(precision):
     tol = 1e-10 if precision == "fp64" else 1e-3
     assert float(((got[0] - want[0]).norm(dim=-1) / (1.0 + want[0].norm(dim=-1))).max()) < tol
     assert torch.equal(got[2], want[2])
+
+
+def _fp32_amplification(orc, mol, pos):
+    """Largest sum of a row's terms without signs times the norm of the blocks'
+    inverses, per walker: what an FP32 rounding of the rows becomes in the
+    inverse's products with them."""
+    ao = orc.ao(pos).detach()
+    terms = ao.abs() @ orc.mo(torch.eye(ao.shape[-1]).to(ao)[None])[0].detach().abs()
+    mo = orc.mo(ao).detach()
+    out = torch.ones(len(pos), dtype=torch.float64)
+    for rows, n in ((slice(0, mol.nup), mol.nup), (slice(mol.nup, None), mol.ndown)):
+        if n:
+            inv = torch.linalg.matrix_norm(torch.linalg.inv(mo[:, rows, :n]), 2)
+            out = out + inv * terms[:, rows, :n].amax((1, 2))
+    return out
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 6, 7, 9, 11, 13, 14, 15])
+def test_every_block_size_in_mixed_precision(n):
+    """The FP32 instances (unscaled rows, no fallback) against the FP64 ones."""
+    print("case minors mixed H%d" % n, flush=True)
+    mol = _chain(n)
+    wf, orc = helpers.make_pair(mol, w_ee=None if n == 1 else 1.0, w_en=1.0)
+    pos = helpers.positions(mol, 67, seed=n, sigma=1.0)
+    d32, l32, s32 = (v.cpu() for v in wf.drift(pos.cuda(), "mixed"))
+    d64, l64, s64 = (v.cpu() for v in wf.drift(pos.cuda(), "fp64"))
+    lpsi, spsi = (v.cpu() for v in wf.log_psi(pos.cuda(), "mixed"))
+    amp = _fp32_amplification(orc, mol, pos)
+    # about 10 roundings of 6e-8 a row entry, n rows; gradients 2 sqrt(13) = 7 times
+    ok = 6e-7 * n * amp < 0.1
+    assert int(ok.sum()) >= 50
+    for l, s in ((l32, s32), (lpsi, spsi)):
+        assert ((l - l64).abs() <= 6e-7 * n * amp)[ok].all() and torch.equal(s[ok], s64[ok])
+    err = (d32 - d64).norm(dim=-1).amax(1) / (1.0 + d64.norm(dim=-1).amax(1))
+    assert (err <= 4.2e-6 * n * amp)[ok].all()
+
+
+def _close_pair(mol, nw, seed):
+    """Ordinary positions; in every second walker two up electrons 1e-6 to 1e-2 bohr apart."""
+    pos = helpers.positions(mol, nw, seed=seed).view(nw, mol.nelec, 3)
+    rng = np.random.default_rng(seed)
+    step = rng.standard_normal((nw, 3))
+    step *= (10.0 ** rng.uniform(-6, -2, nw) / np.linalg.norm(step, axis=1))[:, None]
+    pos[1::2, 1] = pos[1::2, 0] + torch.as_tensor(step[1::2])
+    return pos.reshape(nw, -1)
+
+
+@pytest.mark.parametrize("n,configs", [(6, "ground_state"), (7, "ground_state"), (13, "ground_state"),
+                                       (6, "cas(2,2)"), (10, "cas(2,2)"), (12, "cas(2,2)")])
+def test_weak_blocks_beside_strong_ones(n, configs):
+    """Blocks near a node are eliminated, the others of the wavefront expanded: psi,
+    the drift, the local energy and both adjoints, for one and for several
+    configurations up to seven columns."""
+    print("case minors weak H%d" % n, configs, flush=True)
+    mol = _chain(n)
+    wf, orc = helpers.make_pair(mol, configs=configs, w_ee=1.0, w_en=1.0)
+    ci = torch.linspace(1.0, 0.1, wf.nci, dtype=torch.float64)
+    with torch.no_grad():
+        wf.fc.weight.copy_(ci.view(1, -1))
+        orc.fc_weight.copy_(ci.view(1, -1))
+    orc.bas_exp.requires_grad_(False)
+    orc.atom_coords.requires_grad_(False)
+    wf.ao.bas_exp.requires_grad_(False)
+    pos = _close_pair(mol, 67, seed=n)
+    x = pos.cuda()
+    ao, dao, d2ao = orc.ao(pos, "all")
+    mo = orc.mo(ao).detach()
+    kin = orc.kinetic_operator(pos, ao, dao, d2ao, orc.mo(ao)).detach()
+    kin = kin.reshape(mo.shape)
+    rows = mo / 2.0 ** torch.frexp(mo.abs().amax(-1, keepdim=True))[1]
+    psi_o = orc(pos).detach().view(-1)
+    cond, amp = torch.ones(67, dtype=torch.float64), torch.ones(67, dtype=torch.float64)
+    det0, terms = None, []
+    for c, cu, cd in zip(ci, *wf.configs):
+        part, tr = c * torch.ones(67, dtype=torch.float64), 0.0
+        for sl, cf in ((slice(0, mol.nup), cu.long()), (slice(mol.nup, None), cd.long())):
+            A = mo[:, sl][..., cf]
+            cond = torch.maximum(cond, torch.linalg.cond(rows[:, sl][..., cf]))
+            tr = tr + (torch.linalg.inv(A).transpose(1, 2) * kin[:, sl][..., cf]).abs().sum((1, 2))
+            part = part * torch.linalg.det(A)
+        det0 = torch.linalg.det(rows[:, :mol.nup][..., cu.long()]) if det0 is None else det0
+        terms.append((part, tr))
+    total = sum(p for p, _ in terms).abs()
+    cancel = sum(p.abs() for p, _ in terms) / total  # of the CI sum
+    amp = amp + sum(p.abs() * t for p, t in terms) / total
+    weak = det0.abs() < 1e-6
+    assert int(weak.sum()) >= 5 and int((~weak).sum()) >= 30
+    eps = 1.1e-16 * n * n * cond * cancel  # relative error of an inverse or a determinant, either way
+    ok = 1e3 * eps < 0.1
+    assert int((ok & weak).sum()) >= 5
+    la, sg = (v.cpu() for v in wf.log_psi(x, "fp64"))
+    assert ((la - psi_o.abs().log()).abs() <= 10 * eps)[ok].all() and torch.equal(sg[ok], psi_o.sign()[ok])
+    dr = wf.drift(x, "fp64")[0].cpu()
+    ref = (orc.gradients_jacobi(pos.clone().requires_grad_()).detach() / psi_o[:, None]).view(67, n, 3)
+    assert ((dr - ref).norm(dim=-1).amax(1) <= 100 * eps * (1.0 + ref.norm(dim=-1).amax(1)))[ok].all()
+    e, e_o = wf.local_energy(x).cpu().view(-1), orc.local_energy(pos).detach().view(-1)
+    assert ((e - e_o).abs() <= 100 * eps * (amp + e_o.abs()))[ok].all()
+    # adjoints walker by walker, the best conditioned of either kind; the local
+    # energy's is a difference of products of two inverses with the rows, each
+    # rounded in its terms
+    Y = torch.stack([torch.linalg.matrix_norm(torch.linalg.inv(mo[:, sl][..., cf[0].long()]), 2)
+                     for sl, cf in ((slice(0, mol.nup), wf.configs[0]), (slice(mol.nup, None), wf.configs[1]))]).amax(0)
+    size = orc.mo_scf.abs().max() * ao.detach().norm(dim=(1, 2)) * Y * Y * kin.norm(dim=(1, 2))
+    order = torch.argsort(eps)
+    close = [0, 0]
+    for k in [int(i) for i in order if weak[i]][:4] + [int(i) for i in order if not weak[i]][:2]:
+        one = pos[k:k + 1]
+        for f, f_o, extra in ((lambda v: wf(v).abs().log(), lambda v: orc(v).abs().log(), 0.0),
+                              (wf.local_energy_autodiff, orc.local_energy, float(size[k]))):
+            wf.zero_grad()
+            f(one.cuda()).sum().backward()
+            g_o = torch.autograd.grad(f_o(one).sum(), [orc.mo_modifier, orc.fc_weight])
+            bound = 100 * float(eps[k]) * float(g_o[0].norm()) + 10 * n * n * 1.1e-16 * extra
+            err = float((wf.mo.mo_modifier.grad.cpu() - g_o[0]).norm())
+            assert err <= bound
+            close[extra != 0.0] += int(bool(weak[k]) and bound < 0.1 * float(g_o[0].norm()))
+            if wf.nci > 1:
+                err = float((wf.fc.weight.grad.cpu() - g_o[1]).norm())
+                assert err <= 100 * float(eps[k]) * (float(g_o[1].norm()) + float(amp[k]))
+    # weak walkers whose gradients the bounds pin to a tenth
+    assert close[0] == 4 and close[1] >= 1
+
+
+@pytest.mark.parametrize("n,configs", [(11, "ground_state"), (13, "ground_state"), (10, "cas(2,2)"),
+                                       (12, "cas(2,2)")])
+def test_hmc_of_six_and_seven_columns_replays_the_oracle(n, configs):
+    from oracle import vmc_oracle as O
+    from qmctorch_amd.sampler import Hamiltonian
+    from tests.test_gpu_hmc import _host_noise
+
+    print("case minors hmc H%d" % n, configs, flush=True)
+    mol = _chain(n)
+    wf, orc = helpers.make_pair(mol, configs=configs, w_ee=1.0, w_en=1.0)
+    nw, nstep, L, eps, seed = 7, 2, 3, 0.05, 0x1234_5678
+    q = helpers.positions(mol, nw, seed=n)
+    s = Hamiltonian(nwalkers=nw, nstep=nstep, step_size=eps, L=L, ntherm=0, ndecor=1, nelec=n,
+                    init=mol.domain("normal"), cuda=True, seed=seed)
+    kept = s(wf.pdf, pos=q.cuda().clone(), with_tqdm=False).detach().cpu().view(nstep, nw, -1)
+    for step in range(nstep):
+        p, u = _host_noise(seed, nw, n, step)
+        q, acc = O.hmc_step(orc.pdf, q, p, eps, L, u)
+        # as test_hmc_fp64_replays_oracle_step
+        torch.testing.assert_close(kept[step], q, rtol=0, atol=1e-8)
+
+
+def test_slater_functions_of_several_r_powers():
+    """Contractions over Slater primitives of different r powers: one record per
+    primitive, the entry's parts delivered one after the other."""
+    print("case several r powers", flush=True)
+    mol = systems.hydrogen_atom("sto", 1.0)
+    b = mol.basis
+    # an s of r^0, r^1 and r^2, and p functions x, y, z of r^0 and r^1
+    b.nao = b.nmo = 4
+    b.nshells, b.nao_per_atom = np.array([9]), np.array([4])
+    b.index_ctr = np.array([0, 0, 0, 1, 1, 2, 2, 3, 3])
+    b.nctr_per_ao = np.array([3, 2, 2, 2])
+    b.bas_exp = np.array([1.6, 0.9, 0.7] + 3 * [1.1, 0.6])
+    b.bas_coeffs = np.array([0.5, 0.4, 0.2] + 3 * [0.6, 0.5])
+    b.bas_kr = np.array([0, 1, 2] + 3 * [0, 1])
+    b.bas_kx = np.array([0, 0, 0, 1, 1, 0, 0, 0, 0])
+    b.bas_ky = np.array([0, 0, 0, 0, 0, 1, 1, 0, 0])
+    b.bas_kz = np.array([0, 0, 0, 0, 0, 0, 0, 1, 1])
+    b.bas_n = list(b.bas_kr)
+    b.mos = np.linalg.qr(np.random.default_rng(0).standard_normal((4, 4)))[0]
+    mol.nelec, mol.nup, mol.ndown, mol.spin = 3, 2, 1, 1
+    mol.atomic_number, mol.atomic_nelec = [3], [3]
+    wf, orc = helpers.make_pair(mol, w_ee=0.7, w_en=1.0)
+    pos = helpers.positions(mol, 67, seed=5)
+    x = pos.cuda()
+    psi, psi_o = wf(x).detach().cpu().view(-1), orc(pos).detach().view(-1)
+    assert float(((psi - psi_o).abs() / psi_o.abs()).max()) < 1e-10
+    e, e_o = wf.local_energy(x).cpu().view(-1), orc.local_energy(pos).detach().view(-1)
+    assert float(((e - e_o).abs() / e_o.abs().clamp(min=1.0)).max()) < 1e-9
+    g_o = torch.autograd.grad(orc(pos).abs().log().sum(), [orc.mo_modifier, orc.bas_exp])
+    wf.zero_grad()
+    wf(x).abs().log().sum().backward()
+    for a, o in zip((wf.mo.mo_modifier.grad, wf.ao.bas_exp.grad), g_o):
+        torch.testing.assert_close(a.cpu(), o, rtol=1e-9, atol=1e-9)
+    wf.zero_grad()
+    wf.ao.bas_exp.requires_grad_(False)
+    orc.bas_exp.requires_grad_(False)
+    wf.local_energy_autodiff(x).sum().backward()
+    g_o = torch.autograd.grad(orc.local_energy(pos).sum(), [orc.mo_modifier])[0]
+    torch.testing.assert_close(wf.mo.mo_modifier.grad.cpu(), g_o, rtol=1e-8, atol=1e-8)
