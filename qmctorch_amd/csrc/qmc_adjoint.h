@@ -281,7 +281,7 @@ __device__ __forceinline__ void logpsi_adjoint_reduce(const GRedArgs& a, const W
 #pragma unroll
     for (int m = 0; m < NM; ++m) mo[m] = 0.0;
     {
-        auto sink = [&](int i, int, double val, double, double, double, double) {
+        auto sink = [&](int i, double val, double, double, double, double) {
             const QMC_CONST double* wr = (const QMC_CONST double*)W + (size_t)t.gao_mu[i] * t.nmo;
 #pragma unroll
             for (int m = 0; m < NM; ++m)
@@ -349,7 +349,7 @@ __device__ __forceinline__ void logpsi_adjoint_reduce(const GRedArgs& a, const W
         RedStage<NM, false> st{stage, nullptr, slot, L.lane, t.nmo, 0, 0, G, nullptr};
         st.clear();
         wave_lds_sync();
-        auto sink = [&](int i, int, double val, double, double, double, double) { st.put(i, v ? val : 0.0, 0.0); };
+        auto sink = [&](int i, double val, double, double, double, double) { st.put(i, v ? val : 0.0, 0.0); };
         ao_shells<double, RAD, false>(t, a.p, x, y, z, sink);
         st.flush();
     }
@@ -489,7 +489,7 @@ __device__ __forceinline__ void eloc_adjoint_reduce(const ERedArgs& a, const Wal
 #pragma unroll
     for (int m = 0; m < NM; ++m) mo[m] = gx[m] = gy[m] = gz[m] = lp[m] = 0.0;
     {
-        auto sink = [&](int i, int, double ao, double ax, double ay, double az, double al) {
+        auto sink = [&](int i, double ao, double ax, double ay, double az, double al) {
             const QMC_CONST double* wr = (const QMC_CONST double*)W + (size_t)t.gao_mu[i] * t.nmo;
 #pragma unroll
             for (int m = 0; m < NM; ++m) {
@@ -670,7 +670,7 @@ __device__ __forceinline__ void eloc_adjoint_reduce(const ERedArgs& a, const Wal
         RedStage<NM, true> st{stage, stage + 64 * (kRedCols + 1), slot, L.lane, t.nmo, 0, 0, G, H};
         st.clear();
         wave_lds_sync();
-        auto sink = [&](int i, int, double ao, double ax, double ay, double az, double al) {
+        auto sink = [&](int i, double ao, double ax, double ay, double az, double al) {
             st.put(i, v ? ao : 0.0, v ? -0.5 * (al + 2.0 * (g[0] * ax + g[1] * ay + g[2] * az) + l2 * ao) : 0.0);
         };
         ao_shells<double, RAD, true>(t, a.p, x, y, z, sink);

@@ -54,10 +54,6 @@ struct Tables {
     const QMC_CONST int* ci_dn;
     const QMC_CONST int* exc_up;  // [nconf_up][6] {level, h1, h2, p1, p2, sign}, or null
     const QMC_CONST int* exc_dn;
-    // inverse maps of the adjoint slot sum (CSR): the AO entries of AO mu are
-    // ao_ent[ao_ptr[mu] .. ao_ptr[mu + 1]), the exponent-term columns
-    // (entry i, primitive q) -> i * QMC_MAXP + q of bas_exp index k are
-    // exp_col[exp_ptr[k] .. exp_ptr[k + 1]), both ascending
     // shell records of the table-driven AO row (ao_shells), kRecWords words each,
     // and their contraction coefficients
     int nrec;
@@ -65,6 +61,10 @@ struct Tables {
     const QMC_CONST double* rec_K;
     const QMC_CONST float* rec_Kf;
     int nrec_K;  // their number
+    // inverse maps of the adjoint slot sum (CSR): the AO entries of AO mu are
+    // ao_ent[ao_ptr[mu] .. ao_ptr[mu + 1]), the exponent-term columns
+    // (entry i, primitive q) -> i * QMC_MAXP + q of bas_exp index k are
+    // exp_col[exp_ptr[k] .. exp_ptr[k + 1]), both ascending
     const QMC_CONST int* ao_ptr;
     const QMC_CONST int* ao_ent;
     const QMC_CONST int* exp_ptr;
@@ -156,7 +156,7 @@ __device__ __forceinline__ void cart_poly(T x, T y, T z, int kx, int ky, int kz,
 //        A = R (n (n+1) m0 / r^2 - 2 (n+1) m1 / r + m2), B = 2 c
 // (L the total Cartesian power), shared by the shell's 1, 3 or 6 entries.
 //
-// sink(i, mu, ao, gx, gy, gz, lap) is called once per AO entry i; entries of one
+// sink(i, ao, gx, gy, gz, lap) is called once per AO entry i; entries of one
 // AO that were split across groups are delivered separately (all consumers
 // are linear in the AO).
 
@@ -275,26 +275,26 @@ __device__ __forceinline__ void shell_entries(int i, const ShellRadial<T>& s, T 
 #pragma clang fp contract(off)
     const T v = s.v, c = s.c;
     if (TYPE == kShellS) {
-        sink(i, 0, v, c * x, c * y, c * z, s.A);
+        sink(i, v, c * x, c * y, c * z, s.A);
     } else if (TYPE == kShellP) {
         const T l = s.A + s.B, cx = c * x, cy = c * y, cz = c * z;
-        sink(i + 0, 0, v * x, fma(cx, x, v), cx * y, cx * z, l * x);
-        sink(i + 1, 0, v * y, cy * x, fma(cy, y, v), cy * z, l * y);
-        sink(i + 2, 0, v * z, cz * x, cz * y, fma(cz, z, v), l * z);
+        sink(i + 0, v * x, fma(cx, x, v), cx * y, cx * z, l * x);
+        sink(i + 1, v * y, cy * x, fma(cy, y, v), cy * z, l * y);
+        sink(i + 2, v * z, cz * x, cz * y, fma(cz, z, v), l * z);
     } else if (TYPE == kShellD) {
         const T l = fma(T(2), s.B, s.A), vf = v * f, cf = c * f, lf = l * f, v2 = v + v;
         const T xx = x * x, xy = x * y, xz = x * z, yy = y * y, yz = y * z, zz = z * z;
-        sink(i + 0, 0, v * xx, x * fma(c, xx, v2), c * xx * y, c * xx * z, fma(l, xx, v2));
-        sink(i + 1, 0, vf * xy, y * fma(cf, xx, vf), x * fma(cf, yy, vf), cf * xy * z, lf * xy);
-        sink(i + 2, 0, vf * xz, z * fma(cf, xx, vf), cf * xz * y, x * fma(cf, zz, vf), lf * xz);
-        sink(i + 3, 0, v * yy, c * yy * x, y * fma(c, yy, v2), c * yy * z, fma(l, yy, v2));
-        sink(i + 4, 0, vf * yz, cf * yz * x, z * fma(cf, yy, vf), y * fma(cf, zz, vf), lf * yz);
-        sink(i + 5, 0, v * zz, c * zz * x, c * zz * y, z * fma(c, zz, v2), fma(l, zz, v2));
+        sink(i + 0, v * xx, x * fma(c, xx, v2), c * xx * y, c * xx * z, fma(l, xx, v2));
+        sink(i + 1, vf * xy, y * fma(cf, xx, vf), x * fma(cf, yy, vf), cf * xy * z, lf * xy);
+        sink(i + 2, vf * xz, z * fma(cf, xx, vf), cf * xz * y, x * fma(cf, zz, vf), lf * xz);
+        sink(i + 3, v * yy, c * yy * x, y * fma(c, yy, v2), c * yy * z, fma(l, yy, v2));
+        sink(i + 4, vf * yz, cf * yz * x, z * fma(cf, yy, vf), y * fma(cf, zz, vf), lf * yz);
+        sink(i + 5, v * zz, c * zz * x, c * zz * y, z * fma(c, zz, v2), fma(l, zz, v2));
     } else {
         T Y, Yx = 0, Yy = 0, Yz = 0, Yl = 0;
         cart_poly<T, DERIV>(x, y, z, kx, ky, kz, Y, Yx, Yy, Yz, Yl);
         const T cY = c * Y;
-        sink(i, 0, v * Y, fma(cY, x, v * Yx), fma(cY, y, v * Yy), fma(cY, z, v * Yz),
+        sink(i, v * Y, fma(cY, x, v * Yx), fma(cY, y, v * Yy), fma(cY, z, v * Yz),
              fma(v, Yl, Y * fma(T(kx + ky + kz), s.B, s.A)));
     }
 }
@@ -556,7 +556,8 @@ __device__ __forceinline__ void gauss3_f64(const u4 r, double& a, double& b, dou
 // issued, so loads of any lane of the wavefront issued after the call see the
 // stores issued before it.  No wait is needed for that: the fences have
 // wavefront scope (at workgroup scope each drained the LDS counter; on its own
-// worth 1 to 2 % of the benzene and two-water sweeps, nothing elsewhere).
+// worth 1 to 2 % of the benzene and two-water sweeps, nothing elsewhere).  It
+// orders nothing between wavefronts and no access to global memory.
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -582,8 +583,8 @@ constexpr int kBlockWaves = kBlock / 64;
 // instructions in order, so that clear follows the reads of column k - 1 and
 // precedes the maxima of column k + 1.  Lanes outside every walker (real =
 // false, whose group may share its first lane index with a real group) only
-// read.  seg_pivot_init clears set 0 before column 0.  The wait after the
-// maxima also completes the caller's LDS stores issued before the call.
+// read.  seg_pivot_init clears set 0 before column 0.  The read of the
+// maximum is issued after every maximum and after the caller's earlier LDS stores.
 __device__ __forceinline__ uint32_t* seg_pivot_slots() {
     __shared__ uint32_t slots[kBlockWaves * 128];
     return slots + (threadIdx.x >> 6) * 128;
@@ -598,13 +599,13 @@ __device__ __forceinline__ double* det_recips() {
 
 __device__ __forceinline__ void seg_pivot_init(int myrow, int gbase, bool real) {
     uint32_t* S = seg_pivot_slots();
-    wave_lds_sync();  // earlier eliminations' reads of the slots are done
+    wave_lds_sync();  // earlier eliminations' reads of the slots come first
     if (real && myrow == 0) S[gbase] = 0u;
 }
 
 // seg_pivot_post issues column k's maximum (and the next column's clear);
-// seg_pivot_get waits for it, and for every LDS store the caller issued in
-// between, and returns the pivot row.
+// seg_pivot_get reads it, after every LDS store the caller issued in between,
+// and returns the pivot row.
 template <int NM>
 __device__ __forceinline__ void seg_pivot_post(int k, bool cand, double v, int myrow, int gbase, bool real) {
     static_assert(NM <= 32, "five bits of row index");
@@ -668,7 +669,7 @@ __device__ __forceinline__ void lane_det_lds(double (&a)[NM], int n, int nmax, i
                 const uint64_t bal = __ballot(!done && myrow < br);
                 if (colk) inversions += __popcll(bal & gmask);
                 const bool is_piv = colk && (myrow == br);
-                wave_lds_sync();  // the previous column's reads are done
+                wave_lds_sync();  // the previous column's reads come first
                 if (is_piv && may_store) {
 #pragma unroll
                     for (int j = k; j < NM; ++j) rowbuf[j] = a[j];
@@ -715,7 +716,7 @@ __device__ __forceinline__ void lane_det_lds(double (&a)[NM], int n, int nmax, i
                 const uint64_t bal = __ballot(!done && myrow < br);
                 if (colk) inversions += __popcll(bal & gmask);
                 const bool is_piv = colk && (myrow == br);
-                wave_lds_sync();  // the candidates' stores are done
+                wave_lds_sync();  // the candidates' stores come first
                 const double* const prow = rowbuf + br * NM;
                 const double piv = prow[k];
                 const double ip = recip[br];

@@ -30,7 +30,7 @@ __device__ __forceinline__ V* wave_sumbuf() {
 template <typename V>
 __device__ __forceinline__ V seg_sum(V v, int base, int cnt, int cnt_max) {
     V* B = wave_sumbuf<V>();
-    wave_lds_sync();  // the previous sum's loads are done
+    wave_lds_sync();  // the previous sum's loads come first
     B[threadIdx.x & 63] = v;
     wave_lds_sync();
     V s = V(0);
@@ -106,19 +106,16 @@ __device__ __forceinline__ int find_job(const J* __restrict__ jobs, int njobs, i
 
 // MO row accumulation sink: mo[m] += ao * W[mu, m]  (molecular_orbitals.py:79-95), with W
 // read from the entry-ordered copy (row i = W row of the entry's AO).
-// WT is the storage type of W, AT the accumulator type; AO values may arrive in
-// either precision (FP64 for tight exponent groups in the mixed local energy).
+// DERIV: the rows of its gradient too (the local energy has KinSink).
 // WLDS: W is the block's copy in LDS (qmc_dyn_lds) instead of the plan's
 // constant-space table.
-template <typename WT, int NM, bool DERIV, typename AT = WT, bool LAP = DERIV, bool WLDS = false>
+template <typename T, int NM, bool DERIV, bool WLDS = false>
 struct MoSink {
-    const WT* __restrict__ W;
-    int nmo;
-    AT* mo;
-    AT* gx;
-    AT* gy;
-    AT* gz;
-    AT* lp;
+    const T* __restrict__ W;
+    T* mo;
+    T* gx;
+    T* gy;
+    T* gz;
     // Generated AO rows call fence() at every exponent group.  With W in LDS it
     // replaces W by an opaque copy that depends on the MO accumulators, so the
     // next group's W reads are issued when that group is reached (not all at the
@@ -126,9 +123,9 @@ struct MoSink {
     // before the step loop).  Without LDS it does nothing.
     __device__ __forceinline__ void fence() {
         if constexpr (WLDS) {
-            const QMC_LDS WT* w = (const QMC_LDS WT*)W;
+            const QMC_LDS T* w = (const QMC_LDS T*)W;
             asm volatile("" : "+s"(w) : "v"(mo[0]));
-            W = (const WT*)w;
+            W = (const T*)w;
         }
     }
     // table pointers of a generated row (exponents, atom centres), made opaque
@@ -141,19 +138,17 @@ struct MoSink {
     }
     // row i of the entry-ordered W holds NM columns (zeros past nmo), so the
     // accumulation needs no per-column test
-    template <typename V>
-    __device__ __forceinline__ void operator()(int i, int, V ao, V ax, V ay, V az, V al) const {
-        using WP = typename std::conditional<WLDS, const QMC_LDS WT*, const QMC_CONST WT*>::type;
+    __device__ __forceinline__ void operator()(int i, T ao, T ax, T ay, T az, T) const {
+        using WP = typename std::conditional<WLDS, const QMC_LDS T*, const QMC_CONST T*>::type;
         const WP wr = (WP)W + (size_t)i * NM;  // W row of AO entry i
 #pragma unroll
         for (int m = 0; m < NM; ++m) {
-            const AT w = (AT)wr[m];
-            mo[m] += (AT)ao * w;
+            const T w = wr[m];
+            mo[m] += ao * w;
             if (DERIV) {
-                gx[m] += (AT)ax * w;
-                gy[m] += (AT)ay * w;
-                gz[m] += (AT)az * w;
-                if (LAP) lp[m] += (AT)al * w;
+                gx[m] += ax * w;
+                gy[m] += ay * w;
+                gz[m] += az * w;
             }
         }
     }
@@ -176,7 +171,7 @@ struct KinSink {
     __device__ __forceinline__ const P* pace(const P* p) const {
         return p;
     }
-    __device__ __forceinline__ void operator()(int i, int, double ao, double ax, double ay, double az, double al) const {
+    __device__ __forceinline__ void operator()(int i, double ao, double ax, double ay, double az, double al) const {
         const QMC_CONST double* wr = (const QMC_CONST double*)W + (size_t)i * NM;
         const double b = fma(gx2, ax, fma(gy2, ay, fma(gz2, az, fma(l2, ao, al))));
 #pragma unroll
@@ -289,7 +284,7 @@ struct MfmaPairSink {
         acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(A1, b, acc1, 0, 0, 0);
     }
     template <typename V>
-    __device__ __forceinline__ void operator()(int i, int, V ao, V, V, V, V) {
+    __device__ __forceinline__ void operator()(int i, V ao, V, V, V, V) {
         if (!have) {
             pend = (float)ao;
             pend_i = i;
@@ -304,7 +299,7 @@ struct MfmaPairSink {
         have = false;
         constexpr int S = NM + 1;  // odd row stride: conflict-free column reads
         float* T = (float*)wave_rowbuf<NM>();
-        wave_lds_sync();  // the previous elimination's reads of the buffer are done
+        wave_lds_sync();  // the previous elimination's reads of the buffer come first
         const int col = lane & 31, rb = 4 * (lane >> 5);
         if (col < NM) {
 #pragma unroll
@@ -431,7 +426,7 @@ struct MfmaQuadSink {
         issue();
     }
     template <typename V>
-    __device__ __forceinline__ void operator()(int i, int, V ao, V, V, V, V) {
+    __device__ __forceinline__ void operator()(int i, V ao, V, V, V, V) {
         if (npend > 0 && i != pend_i + npend) flush();  // entries arrive in order; else start a new four
         if (npend == 0) pend_i = i;
         p0 = p1;
@@ -444,7 +439,7 @@ struct MfmaQuadSink {
         flush();
         constexpr int S = NM + 1;  // odd row stride: conflict-free column reads
         float* Tt = (float*)wave_rowbuf<NM>();
-        wave_lds_sync();  // the previous elimination's reads of the buffer are done
+        wave_lds_sync();  // the previous elimination's reads of the buffer come first
         const int col = lane & 15, rq = 4 * (lane >> 4);
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
@@ -490,7 +485,7 @@ __device__ __forceinline__ void jastrow_and_potential(const Tables& t, const Qmc
     // partner coordinates through the wavefront's LDS block: one store of this
     // lane's position, one vector load per partner
     double* P = wave_posbuf<double>();
-    wave_lds_sync();  // the previous evaluation's loads are done
+    wave_lds_sync();  // the previous evaluation's loads come first
     P[L.lane * 4 + 0] = x;
     P[L.lane * 4 + 1] = y;
     P[L.lane * 4 + 2] = z;
@@ -566,7 +561,7 @@ __device__ __forceinline__ T jastrow_value(const Tables& t, const QmcParams& prm
         // this lane's position, one vector load per partner (independent loads
         // instead of three shuffles each)
         T* P = wave_posbuf<T>();
-        wave_lds_sync();  // the previous evaluation's loads are done
+        wave_lds_sync();  // the previous evaluation's loads come first
         P[L.lane * 4 + 0] = xs;
         P[L.lane * 4 + 1] = ys;
         P[L.lane * 4 + 2] = zs;
@@ -804,12 +799,21 @@ __device__ __forceinline__ void minor_det(const Tables& t, const WalkerLane& L, 
     });
 }
 
+// log|c0 D_up D_dn| and its sign in every lane, from the groups' determinants
+// d 2^ex (one logarithm for the product).
+__device__ __forceinline__ void single_product(const Tables& t, const WalkerLane& L, double d, int ex, double logc0,
+                                               double c0, double& logabs, double& sgn) {
+    const int dn_lane = L.wbase + (t.ndown > 0 ? t.nup : 0);
+    const double du = __shfl(d, L.wbase), dd_ = __shfl(d, dn_lane);
+    const int eu = __shfl(ex, L.wbase), ed = __shfl(ex, dn_lane);
+    const double dd = t.ndown > 0 ? dd_ : 1.0;
+    logabs = log_abs_product(du, dd, eu + (t.ndown > 0 ? ed : 0)) + logc0;
+    sgn = (((du < 0.0) != (dd < 0.0)) != (c0 < 0.0)) ? -1.0 : 1.0;
+}
+
 // Single configuration, single CI term: log|D_up D_dn| and its sign in every
 // lane, and (INV) this lane's inverse column y; ksum: the sum of kj over the
 // walker's lanes, in lane order, exchanged together with the rows.
-__device__ __forceinline__ void single_product(const Tables& t, const WalkerLane& L, double d, int ex, double logc0,
-                                               double c0, double& logabs, double& sgn);
-
 template <int NM, bool INV, typename T, typename KT>
 __device__ __forceinline__ void slater_single_minors(const Tables& t, const QmcParams& prm, const WalkerLane& L,
                                                      const T (&mo)[NM], double logc0, KT kj, double& logabs,
@@ -865,18 +869,6 @@ __device__ __forceinline__ void slater_single_minors(const Tables& t, const QmcP
             single_product(t, L, weak ? dw : D, weak ? ex + ew : ex, logc0, c0, logabs, sgn);
         }
     }
-}
-
-// log|c0 D_up D_dn| and its sign in every lane, from the groups' determinants
-// d 2^ex (one logarithm for the product).
-__device__ __forceinline__ void single_product(const Tables& t, const WalkerLane& L, double d, int ex, double logc0,
-                                               double c0, double& logabs, double& sgn) {
-    const int dn_lane = L.wbase + (t.ndown > 0 ? t.nup : 0);
-    const double du = __shfl(d, L.wbase), dd_ = __shfl(d, dn_lane);
-    const int eu = __shfl(ex, L.wbase), ed = __shfl(ex, dn_lane);
-    const double dd = t.ndown > 0 ? dd_ : 1.0;
-    logabs = log_abs_product(du, dd, eu + (t.ndown > 0 ? ed : 0)) + logc0;
-    sgn = (((du < 0.0) != (dd < 0.0)) != (c0 < 0.0)) ? -1.0 : 1.0;
 }
 
 // Single configuration, single CI term: log|D_up D_dn| and its sign (ground state).
@@ -1121,7 +1113,7 @@ __device__ __forceinline__ void slater_exc(const Tables& t, const QmcParams& prm
     double lg, sg, tp;
     int col;
     lane_gauss_jordan<NM, true>(a, b, n, t.nsig_max, L.myrow, L.gbase, L.gmask, lg, sg, tp, col);
-    wave_lds_sync();  // the previous evaluation's reads are done
+    wave_lds_sync();  // the previous evaluation's reads come first
     if (L.lane_real && col >= 0) {
 #pragma unroll
         for (int j = 0; j < NM; ++j) Mb[col * NM + j] = b[j];  // row col of A^-1 [A | V]
@@ -1211,7 +1203,7 @@ __device__ __forceinline__ void exc_gamma(const Tables& t, const QmcParams& prm,
     double lg, sg, tp;
     int col;
     lane_gauss_jordan<NM, true>(a, b, n, t.nsig_max, L.myrow, L.gbase, L.gmask, lg, sg, tp, col);
-    wave_lds_sync();  // the previous walkers' reads are done
+    wave_lds_sync();  // the previous walkers' reads come first
     if (L.lane_real && col >= 0) {
 #pragma unroll
         for (int j = 0; j < NM; ++j) Mb[col * NM + j] = b[j];  // row col of [I | M]
@@ -1351,7 +1343,7 @@ __device__ __forceinline__ double exc_eloc_gamma(const Tables& t, const QmcParam
         b[j] = mo[j];
     }
     lane_gauss_jordan<NM, true>(a, b, n, t.nsig_max, L.myrow, L.gbase, L.gmask, lg, sg, tp, col);
-    wave_lds_sync();  // the previous walkers' reads are done
+    wave_lds_sync();  // the previous walkers' reads come first
     if (L.lane_real && col >= 0) {
 #pragma unroll
         for (int j = 0; j < NM; ++j) Mb[col * NM + j] = b[j];  // row col of [I | M]
@@ -1472,7 +1464,7 @@ __device__ __forceinline__ double exc_eloc_gamma(const Tables& t, const QmcParam
             }
         }
     }
-    wave_lds_sync();  // every read of the Mk rows is done
+    wave_lds_sync();  // every read of the Mk rows comes first
     if (L.lane_real && col >= 0) {
 #pragma unroll
         for (int p = 0; p < NM; ++p) Kb[col * NM + p] = gK[p];  // now the G_K rows
@@ -1604,7 +1596,7 @@ __device__ __forceinline__ void wf_walkers(const KArgs& a, const WalkerLane& L, 
             asm volatile("" : "+v"(bk[m]));
         }
     } else {
-        MoSink<AT, NM, false, AT> sink{(const AT*)a.p.entry_w, t.nmo, mo, nullptr, nullptr, nullptr, nullptr};
+        MoSink<T, NM, false> sink{(const T*)a.p.entry_w, mo, nullptr, nullptr, nullptr};
         AO::template row<T, RAD, false>(t, a.p, x, y, z, sink);
     }
     double logabs, sgn, kin = 0.0, logj, svee = 0.0, sven = 0.0;
@@ -1667,7 +1659,8 @@ __device__ __forceinline__ int combine_table(int from, int wave_bytes) {
 }
 
 // Waves per SIMD the evaluation kernels are held to: what their registers allow
-// without spilling (168 VGPRs up to 5 columns, 3 with table-driven rows).
+// (168 VGPRs for three up to 5 columns, 3 with table-driven rows; up to 14 spilled
+// in the 3-column Slater and the 24-column instances).
 template <int NM, typename AO>
 constexpr int wf_waves() {
     return NM <= (AO::kEntries > 0 ? 5 : 3) ? 3 : (NM <= 12 ? 2 : 1);
@@ -1749,7 +1742,7 @@ __device__ __forceinline__ double eval_logpsi(const Tables& t, const QmcParams& 
     } else {
 #pragma unroll
         for (int m = 0; m < NM; ++m) mo[m] = T(0);
-        MoSink<T, NM, false, T, false, WLDS> sink{w, t.nmo, mo, nullptr, nullptr, nullptr, nullptr};
+        MoSink<T, NM, false, WLDS> sink{w, mo, nullptr, nullptr, nullptr};
         AO::template row<T, RAD, false>(t, prm, x, y, z, sink);
     }
     const T kj = jastrow_value<T>(t, prm, L, x, y, z);
@@ -2072,10 +2065,10 @@ __device__ __forceinline__ T jastrow_value_grad(const Tables& t, const QmcParams
 // lane's electron (slater_jastrow.py:346-447 without the psi factor):
 //   grad_i ln|S| = sum_c omega_c sum_k (A_c^-1)[k, i] grad phi_{conf_c[k]}(r_i),
 //   omega_c = sum_{n using c for this spin} c_n D_n / S,
-// plus grad_i ln J.  A_c^-1 comes from the lane elimination of [A_c | I] (the
-// lane that pivoted column k holds row k); the rows are transposed through
-// the wavefront's LDS block lds[64][NM] so that lane i reads column i.  AO and
-// MO rows in T, elimination and combination in FP64.  MC bounds the unique
+// plus grad_i ln J.  Column i of A_c^-1 comes from the lane's cofactors
+// (slater_single_minors, minor_det) or, above their sizes, from the in-place
+// inversion (lane_inverse).  AO and MO rows in T, inverses and combination in
+// FP64.  MC bounds the unique
 // configurations per spin (1 for the ground-state determinant, QMC_MAXCONF for
 // every other plan): the per-configuration values live in registers.
 template <typename T, int NM, int RAD, int MC, typename AO = AoGeneric>
@@ -2085,7 +2078,7 @@ __device__ __forceinline__ double eval_drift(const Tables& t, const QmcParams& p
 #pragma unroll
     for (int m = 0; m < NM; ++m) mo[m] = gx[m] = gy[m] = gz[m] = T(0);
     // values and gradients only: the row's Laplacian terms are dead code here
-    MoSink<T, NM, true, T, false> sink{(const T*)prm.entry_w, t.nmo, mo, gx, gy, gz, nullptr};
+    MoSink<T, NM, true> sink{(const T*)prm.entry_w, mo, gx, gy, gz};
     AO::template row<T, RAD, true>(t, prm, x, y, z, sink);
     if constexpr (use_minors<NM>()) {
         // formed here, not sunk past the determinants (as the kinetic row of wf_walkers)
@@ -2249,7 +2242,7 @@ __device__ __forceinline__ double eval_drift_exc(const Tables& t, const QmcParam
     T mo[NM], gx[NM], gy[NM], gz[NM];
 #pragma unroll
     for (int m = 0; m < NM; ++m) mo[m] = gx[m] = gy[m] = gz[m] = T(0);
-    MoSink<T, NM, true, T, false> sink{(const T*)prm.entry_w, t.nmo, mo, gx, gy, gz, nullptr};
+    MoSink<T, NM, true> sink{(const T*)prm.entry_w, mo, gx, gy, gz};
     AoGeneric::template row<T, RAD, true>(t, prm, x, y, z, sink);
     T jg[3];
     const T kj = jastrow_value_grad<T>(t, prm, L, x, y, z, jg);
@@ -2418,7 +2411,7 @@ __global__ __launch_bounds__(kBlock) void ao_kernel(AArgs a) {
     double* ao = a.ao;
     double* dao = a.dao;
     double* d2ao = a.d2ao;
-    auto sink = [&](int i, int, double val, double ax, double ay, double az, double al) {
+    auto sink = [&](int i, double val, double ax, double ay, double az, double al) {
         if (!v) return;
         const int mu = t.gao_mu[i];
         ao[row + mu] += val;
@@ -2622,7 +2615,7 @@ __global__ __launch_bounds__(kBlock) void grad_kernel(GArgs a) {
     {
         double* aor = a.ao_rows + row * t.nao;
         const double* W = (const double*)a.p.mo_w;
-        auto sink = [&](int i, int, double val, double, double, double, double) {
+        auto sink = [&](int i, double val, double, double, double, double) {
             const int mu = t.gao_mu[i];
             if (v) aor[mu] += val;
             const QMC_CONST double* wr = (const QMC_CONST double*)W + (size_t)mu * t.nmo;
@@ -2823,7 +2816,7 @@ __global__ __launch_bounds__(kBlock) void eloc_grad_kernel(EArgs a) {
         const double* W = (const double*)a.p.mo_w;
         double* aor = a.ao_rows ? a.ao_rows + row * t.nao : nullptr;
         double* bor = a.b_rows ? a.b_rows + row * t.nao : nullptr;
-        auto sink = [&](int i, int, double ao, double ax, double ay, double az, double al) {
+        auto sink = [&](int i, double ao, double ax, double ay, double az, double al) {
             const int mu = t.gao_mu[i];
             if (v && aor) aor[mu] += ao;
             if (v && bor) bor[mu] += -0.5 * (al + 2.0 * (g[0] * ax + g[1] * ay + g[2] * az) + l2 * ao);

@@ -201,8 +201,9 @@ int spec_%(name)s_hmc(const HArgs& a, int prec, hipStream_t s) {
 # straight-line row of a larger one (benzene: 120 entries x 24 columns) is
 # executed once per wavefront and waits for its instructions, where the
 # table-driven row is a loop that stays in the instruction cache: E_L of 1021
-# walkers 309 us generated, 180 us table-driven; water (24 entries x 5 columns),
-# 65536 walkers, is fastest with its generated row.
+# walkers 309 us generated, 180 us table-driven; water (25 entries x 5 columns),
+# 65536 walkers, is fastest with its generated row.  Of the layouts the next
+# smaller one is N2 (30 x 7): where between 210 and 2880 the line lies is not known.
 ELOC_MAX_W = 512
 
 NO_ELOC = '''

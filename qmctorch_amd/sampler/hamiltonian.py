@@ -9,8 +9,8 @@ E = U + |p|^2 / 2 and u ~ U[0,1), ``ntherm=-1`` keeps only the last
 positions, ``ndecor`` thins.
 
 Differences forced by the device design: grad U = -2 grad ln|psi| comes from
-the drift evaluated inside ``qmc_hmc_sweep`` (the lane Gauss-Jordan inverse),
-not from autograd through ``-log(pdf)``; the trajectory runs on the device
+the drift evaluated inside ``qmc_hmc_sweep`` (inverse columns by minors or, from
+8 columns on, by elimination), not from autograd through ``-log(pdf)``; the trajectory runs on the device
 with the walker state in registers; momenta and uniforms come from
 Philox4x32-10 keyed by a seed drawn from torch's global generator (chains agree
 with the reference statistically, not sample by sample); a move whose energy

@@ -5,7 +5,8 @@ Chains of n hydrogen atoms with one unpaired electron: the up block is
 runs with a group completed by unit rows, and 8 is the first size of the
 eliminations.  psi, the local energy and the gradient against the float64
 oracle; log|psi| far from every nucleus, where products of orbital values
-leave the double range, against the sum of the single-electron decays.
+leave the double range, against the sum of the single-electron decays; blocks
+near a node, which are eliminated; the same sizes in mixed precision.
 """
 import numpy as np
 import pytest
